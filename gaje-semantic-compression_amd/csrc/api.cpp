@@ -246,6 +246,25 @@ extern "C" int gaje_hip_q4_0_gemm(const void *packed, const float *X, const floa
                                   int64_t m, int64_t n, int64_t k, void *stream) {
     GAJE_TRY(check_dims(n, k));
     if (m < 0 || (m > 0 && (!X || !Y))) return set_error(GAJE_ERR_INVALID_ARG, "bad gemm arguments");
+    if (m >= 2 && n > 0 && k % 32 == 0 && packed && gemv_lds_bytes(k, FMT_Q4_0, false) + 1024 <= max_lds_per_block() &&
+        !(((uintptr_t)packed | (uintptr_t)X) & 15)) {
+        BatchGemvParams p{};
+        p.w = (const uint8_t *)packed;
+        p.fmt = FMT_Q4_0;
+        p.nb = (int32_t)(k / 32);
+        p.N = n;
+        p.K = k;
+        p.x = X;
+        p.ldx = k;
+        p.nv = m;
+        p.bias = bias;
+        p.bias_len = bias ? bias_len : 0;
+        p.mode = MODE_STORE;
+        p.y = Y;
+        p.ldy = n;
+        p.st_a = p.st_b = ST_NONE;
+        return launch_q4_rows(p, as_stream(stream));
+    }
     for (int64_t r = 0; r < m; ++r)
         GAJE_TRY(launch_gemv(plain_gemv(FMT_Q4_0, packed, X + r * k, bias, bias_len, Y + r * n, n, k), as_stream(stream)));
     return GAJE_OK;

@@ -560,12 +560,13 @@ __global__ __launch_bounds__(WIDE) void attn_batch_wide(AttnParams p) {
     const int g = group % p.n_head_kv, z = group / p.n_head_kv, h = g * R + slot % R;
     const int pos = p.seq_pos[z];
     if (pos < 0) return;  // (uniform)
+    const int64_t kvz = p.row_seq ? p.row_seq[z] : z;
     const int ctx = pos + 1;
     const float *q = p.q + z * p.seq_q_stride + (size_t)h * HD;
     const float scale = 1.0f / sqrtf((float)HD);
     const int64_t cap = p.kv_cap;
-    const float *Kh = p.k_cache + z * p.seq_kv_stride + (size_t)g * p.kv_head_stride;
-    const float *Vh = p.v_cache + z * p.seq_kv_stride + (size_t)g * p.kv_head_stride;
+    const float *Kh = p.k_cache + kvz * p.seq_kv_stride + (size_t)g * p.kv_head_stride;
+    const float *Vh = p.v_cache + kvz * p.seq_kv_stride + (size_t)g * p.kv_head_stride;
     const uint32_t rowb = (uint32_t)cap * 4;
     const int m = lane / S::QW, quad = wave * S::QW + lane % S::QW;
     const int n = chain_len(ctx);
@@ -727,8 +728,8 @@ __global__ __launch_bounds__(WIDE) void attn_batch_wide(AttnParams p) {
         }
         const int rel = (lane - (P - 1)) & 63;
         if (rel % L == 0) {
-            const int64_t i = (int64_t)h * HD + wave * G + rel / L, rows = (int64_t)p.n_head * HD;
-            p.out[z * p.seq_q_stride + (p.out_chain_major ? (i & 7) * (rows / 8) + (i >> 3) : i)] = acc;
+            const int64_t i = (int64_t)h * HD + wave * G + rel / L;
+            p.out[z * p.seq_q_stride + i] = acc;
         }
         if (waited_out && lane == 0) wait_ran_out(p, z);
     }
@@ -749,6 +750,7 @@ __global__ __launch_bounds__(THREADS) void attn_decode_batch(AttnParams p) {
     const int h = blockIdx.x, z = blockIdx.z;
     const int pos = p.seq_pos[z];
     if (pos < 0) return;
+    const int64_t kvz = p.row_seq ? p.row_seq[z] : z;
     const int ctx = pos + 1;
     if (tid < 32) tab[tid] = kExp2Tab[tid];
     const int g = h / (p.n_head / p.n_head_kv);
@@ -757,8 +759,8 @@ __global__ __launch_bounds__(THREADS) void attn_decode_batch(AttnParams p) {
     const int n = chain_len(ctx);
     float *sc = smem;
     const float *qg = p.q + z * p.seq_q_stride + (size_t)h * HD;
-    const float *Kh = p.k_cache + z * p.seq_kv_stride + (size_t)g * p.kv_head_stride;
-    const float *Vh = p.v_cache + z * p.seq_kv_stride + (size_t)g * p.kv_head_stride;
+    const float *Kh = p.k_cache + kvz * p.seq_kv_stride + (size_t)g * p.kv_head_stride;
+    const float *Vh = p.v_cache + kvz * p.seq_kv_stride + (size_t)g * p.kv_head_stride;
     // q: uniform (scalar) loads for HD = 64; a 128-float q does not fit the
     // scalar registers (the compiler spills them), so it is read from LDS
     __shared__ float qs[HD > 64 ? HD : 1];
@@ -824,8 +826,8 @@ __global__ __launch_bounds__(THREADS) void attn_decode_batch(AttnParams p) {
         int t0 = 0;
         for (; t0 + 4 * AH <= ctx; t0 += 4 * AH) block(t0, std::true_type{});
         if (t0 < ctx) block(t0, std::false_type{});
-        const int64_t i = (int64_t)h * HD + tid, rows = (int64_t)p.n_head * HD;
-        p.out[z * p.seq_q_stride + (p.out_chain_major ? (i & 7) * (rows / 8) + (i >> 3) : i)] = acc;
+        const int64_t i = (int64_t)h * HD + tid;
+        p.out[z * p.seq_q_stride + i] = acc;
     }
 }
 
@@ -860,10 +862,11 @@ __global__ __launch_bounds__(THREADS) void attn_decode_generic(AttnParams p) {
         const int z = blockIdx.z;
         if (p.seq_pos[z] < 0) return;
         ctx = p.seq_pos[z] + 1;
+        const int64_t kvz = p.row_seq ? p.row_seq[z] : z;
         p.q += z * p.seq_q_stride;
         p.out += z * p.seq_q_stride;
-        p.k_cache += z * p.seq_kv_stride;
-        p.v_cache += z * p.seq_kv_stride;
+        p.k_cache += kvz * p.seq_kv_stride;
+        p.v_cache += kvz * p.seq_kv_stride;
     }
     const float scale = 1.0f / sqrtf((float)hd);
 
@@ -899,8 +902,8 @@ __global__ __launch_bounds__(THREADS) void attn_decode_generic(AttnParams p) {
             const float prod = sc[t] * v[t];
             acc = acc + prod;
         }
-        const int64_t o = (int64_t)h * hd + i, rows = (int64_t)p.n_head * hd;
-        p.out[p.out_chain_major ? (o & 7) * (rows / 8) + (o >> 3) : o] = acc;
+        const int64_t o = (int64_t)h * hd + i;
+        p.out[o] = acc;
     }
 }
 
@@ -930,8 +933,6 @@ int launch_attention(const AttnParams &p, hipStream_t s) {
                          (long long)p.kv_cap);
     if (p.seq_pos && (p.n_seq <= 0 || p.n_seq > 65535)) return set_error(GAJE_ERR_INVALID_ARG, "attention: bad batch");
     const unsigned nz = p.seq_pos ? (unsigned)p.n_seq : 1u;
-    if (p.out_chain_major && (!p.seq_pos || ((int64_t)p.n_head * p.head_dim) % 8))
-        return set_error(GAJE_ERR_INVALID_ARG, "attention: chain-major output needs a batch and n_head*head_dim %% 8 == 0");
     const bool batch_kernel = p.seq_pos && p.kv_cap % 4 == 0 && (p.head_dim == 64 || p.head_dim == 128) &&
                               (size_t)chain_row(p.kv_cap) * 4 + 1024 <= max_lds_per_block();
     if (batch_kernel && batch_wide_lds_bytes(p.head_dim, p.kv_cap) + 1024 <= max_lds_per_block()) {

@@ -13,176 +13,8 @@
 namespace gaje {
 namespace {
 
-constexpr int BQ_CHUNK = 512;              // activation elements per staged chunk (4 packed groups)
-constexpr int BQ_CROW = BQ_CHUNK / 8 + 4;  // LDS floats per (vector, chain) row of a chunk
-
 __device__ __forceinline__ void seq_flag(uint32_t *codes, int s, int layer, int stage) {
     if (codes && stage >= 0) atomicMin(&codes[s], (uint32_t)(layer * 8 + stage));
-}
-
-// dequantised values of one packed group for chain l (genomic.rs:298-316): d = fma(q, scale, min)
-__device__ __forceinline__ void group_dequant(float (&d)[16], vu2 n, vu4 s) {
-    const uint32_t c[4] = {opaque_and(n.x, 0x0F0F0F0Fu), opaque_and(n.x >> 4, 0x0F0F0F0Fu),
-                           opaque_and(n.y, 0x0F0F0F0Fu), opaque_and(n.y >> 4, 0x0F0F0F0Fu)};
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        const float scale = half_lo(s[b]), mn = half_hi(s[b]);
-        d[4 * b + 0] = fmaf(ubyte0(c[b]), scale, mn);
-        d[4 * b + 1] = fmaf(ubyte1(c[b]), scale, mn);
-        d[4 * b + 2] = fmaf(ubyte2(c[b]), scale, mn);
-        d[4 * b + 3] = fmaf(ubyte3(c[b]), scale, mn);
-    }
-}
-
-// Packed Q4_0 rows x NV activation vectors (genomic_dot_product_q4_0_avx2,
-// genomic.rs:263-336, per vector).  Lane = (row slot lane>>3, chain l =
-// lane&7); a slot holds R rows (rows slot + 8j of the workgroup's 8R), so
-// each activation value read from LDS feeds R rows' chains; wave w owns
-// vectors vz + w*VPW.. (their accumulators; vz = blockIdx.y * NV, the
-// workgroup's share of the batch); the waves share the rows and the staged
-// chunk of all NV vectors.  Activations arrive chain-major
-// ([vector][chain l][K/8]: element k at chain k%8, column k/8), so a chunk is
-// 8 contiguous runs per vector, copied to LDS through registers
-// (double-buffered, loads always issued, clamped at the end).  Groups past the
-// row's end read as zero codes/scales against zero activations, and
-// fma(0, 0, acc) = acc (acc is never -0), so every chunk runs branch-free.
-template <int NV, int VPW, int R>
-__global__ __launch_bounds__(NV / VPW * 64) void gemv_batch_q4_kernel(BatchGemvParams p) {
-    constexpr int NTH = NV / VPW * 64;
-    constexpr int RUN = BQ_CHUNK / 8;                 // floats of one chain per chunk
-    constexpr int BUF = NV * 8 * BQ_CROW;
-    constexpr int UPT = NV * 8 * (RUN / 4) / NTH;     // float4s staged per thread per chunk
-    extern __shared__ __align__(16) float xs[];       // [2][NV][8][BQ_CROW]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int l = lane & 7;
-    const int nb = p.nb, G = (nb + 3) >> 2;
-    const int64_t K8 = (int64_t)nb * 4;               // column count of a chain row
-    const int nch = (int)((K8 + RUN - 1) / RUN);
-    int64_t row[R];
-    const uint8_t *wr[R];
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-        row[j] = (int64_t)blockIdx.x * 8 * R + 8 * j + (lane >> 3);
-        wr[j] = p.w + (size_t)(row[j] < p.N ? row[j] : p.N - 1) * G * 80;
-    }
-    const int v0 = wave * VPW;
-    const int vz = blockIdx.y * NV;  // first vector of this workgroup's share of the batch
-
-    vf4 st[UPT];
-    auto load_chunk = [&](int c) {
-#pragma unroll
-        for (int i = 0; i < UPT; ++i) {
-            const int u = tid + i * NTH, vl = u / (RUN / 4), q = u % (RUN / 4);  // vl = v * 8 + l
-            const int64_t col = (int64_t)c * RUN + 4 * q;
-            const bool in = col < K8;
-            const float *src = p.x + (size_t)(vz + (vl >> 3)) * p.ldx + (size_t)(vl & 7) * K8 + (in ? col : 0);
-            const vf4 a = *(const vf4 *)src;
-            st[i] = in ? a : (vf4){0.f, 0.f, 0.f, 0.f};
-        }
-    };
-    auto store_chunk = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < UPT; ++i) {
-            const int u = tid + i * NTH, vl = u / (RUN / 4), q = u % (RUN / 4);
-            *(vf4 *)(xs + buf * BUF + vl * BQ_CROW + 4 * q) = st[i];
-        }
-    };
-    vu2 wn[2][R][4];
-    vu4 ws[2][R][4];
-    auto load_w = [&](int c, int slot) {
-#pragma unroll
-        for (int j = 0; j < R; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int g = 4 * c + i;
-                const bool in = g < G;
-                const uint8_t *gp = wr[j] + (size_t)(in ? g : G - 1) * 80;
-                const vu2 n = *(const vu2 *)(gp + 8 * l);
-                const vu4 s = *(const vu4 *)(gp + 64);
-                const uint32_t keep = in ? 0xFFFFFFFFu : 0u;
-                wn[slot][j][i] = n & keep;
-                ws[slot][j][i] = s & keep;
-            }
-    };
-
-    float acc[R][VPW];
-#pragma unroll
-    for (int j = 0; j < R; ++j)
-#pragma unroll
-        for (int v = 0; v < VPW; ++v) acc[j][v] = 0.0f;
-
-    load_chunk(0);
-    load_w(0, 0);
-    store_chunk(0);
-    lds_barrier();
-    // one chunk from buffer `cur` (a constant at each call: the rings are
-    // indexed statically); the next chunk's loads are in flight meanwhile.
-    // The activations are issued before the weights: loads complete in order,
-    // so staging them waits for them alone, and the barriers order LDS only,
-    // leaving the next chunk's weights in flight across them.
-    auto chunk = [&](int c, int cur) {
-        const int cn = c + 1 < nch ? c + 1 : c;
-        load_chunk(cn);
-        load_w(cn, cur ^ 1);
-        const float *xb = xs + cur * BUF + (v0 * 8 + l) * BQ_CROW;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float d[R][16];
-#pragma unroll
-            for (int j = 0; j < R; ++j) group_dequant(d[j], wn[cur][j][i], ws[cur][j][i]);
-#pragma unroll
-            for (int v = 0; v < VPW; ++v) {
-                const float *xv = xb + v * 8 * BQ_CROW + 16 * i;
-                const float4 x0 = *(const float4 *)xv, x1 = *(const float4 *)(xv + 4);
-                const float4 x2 = *(const float4 *)(xv + 8), x3 = *(const float4 *)(xv + 12);
-                const float xx[16] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w,
-                                      x2.x, x2.y, x2.z, x2.w, x3.x, x3.y, x3.z, x3.w};
-#pragma unroll
-                for (int j = 0; j < R; ++j) {
-                    float a = acc[j][v];
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) a = fmaf(d[j][e], xx[e], a);
-                    acc[j][v] = a;
-                }
-            }
-        }
-        store_chunk(cur ^ 1);
-        lds_barrier();
-    };
-    for (int c = 0; c < nch; c += 2) {
-        chunk(c, 0);
-        if (c + 1 < nch) chunk(c + 1, 1);
-    }
-
-    // per (row, vector): ((a0+a4)+(a2+a6)) + ((a1+a5)+(a3+a7)) in lane l = 0, then the row epilogue
-#pragma unroll
-    for (int j = 0; j < R; ++j)
-#pragma unroll
-        for (int v = 0; v < VPW; ++v) {
-            const float a = acc[j][v];
-            const float t = red8_dpp(a);  // valid in lane 8r
-            const int s = vz + v0 + v;
-            const int64_t r = row[j];
-            if (l != 0 || r >= p.N || s >= p.nv) continue;
-            float y = flush_small(t);
-            if (p.a_ptr) {  // sparse anchors, then the bias (forward.rs:103-115)
-                for (int64_t k = p.a_ptr[r]; k < p.a_ptr[r + 1]; ++k) {
-                    const uint32_t col = p.a_col[k];
-                    const float prod = p.x[(size_t)s * p.ldx + (col & 7) * K8 + (col >> 3)] * half_bits(p.a_val[k]);
-                    y = y + prod;
-                }
-            }
-            if (r < p.bias_len) y = y + p.bias[r];
-            float *dst = p.y + (size_t)s * p.ldy + r;
-            if (p.mode == MODE_RESIDUAL) {
-                if (isnan(y)) seq_flag(p.nan_codes, s, p.layer, p.st_a);
-                const float h = *dst + y;
-                *dst = h;
-                if (isnan(h)) seq_flag(p.nan_codes, s, p.layer, p.st_b);
-            } else {
-                *dst = y;
-            }
-        }
 }
 
 // F32 rows in the tiled layout x NV vectors (dot_product, dot.rs:23-94, per
@@ -359,7 +191,6 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(BatchRowParams p) {
         inv = inv_slot;
     }
     bad = 0;
-    const int64_t K8 = p.K / 8;
     for (int64_t k = tid; k < p.K; k += 256) {
         float o = xs[k];  // no weight: the plain rows (an empty norm tensor is skipped, block/forward.rs:18-28)
         if (p.w) {
@@ -367,7 +198,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(BatchRowParams p) {
             o = t * p.w[k];
         }
         bad |= isnan(o);
-        p.y[(size_t)s * p.ldy + (p.chain_major ? (k & 7) * K8 + (k >> 3) : k)] = o;
+        p.y[(size_t)s * p.ldy + k] = o;
     }
     if (__syncthreads_or(bad) && tid == 0) seq_flag(p.nan_codes, s, p.layer, p.st_b);
 }
@@ -429,22 +260,24 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_cm_kernel(BatchRowParams p) 
     }
     bad = 0;
     float *y = p.y + (size_t)s * p.ldy;
+    const bool wide = !((uintptr_t)y & 15);
 #pragma unroll
     for (int u = 0; u < RN_XB4; ++u) {
         const int64_t m = u * 256 + tid;
         if (m >= K4) continue;
         const float v[4] = {xr[u].x, xr[u].y, xr[u].z, xr[u].w}, w[4] = {wr[u].x, wr[u].y, wr[u].z, wr[u].w};
+        float o[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int64_t k = 4 * m + j;
-            float o = v[j];  // no weight: the plain rows
+            o[j] = v[j];  // no weight: the plain rows
             if (p.w) {
-                const float t = o * inv;
-                o = t * w[j];
+                const float t = v[j] * inv;
+                o[j] = t * w[j];
             }
-            bad |= isnan(o);
-            y[p.chain_major ? (k & 7) * K8 + (k >> 3) : k] = o;
+            bad |= isnan(o[j]);
+            if (!wide) y[4 * m + j] = o[j];
         }
+        if (wide) *(float4 *)(y + 4 * m) = make_float4(o[0], o[1], o[2], o[3]);
     }
     if (__syncthreads_or(bad) && tid == 0) seq_flag(p.nan_codes, s, p.layer, p.st_b);
 }
@@ -461,7 +294,7 @@ __global__ __launch_bounds__(256) void swiglu_elems_kernel(BatchRowParams p) {
         bad_u = isnan(uv);
         const float o = swiglu1(g[k], uv);
         bad_o = isnan(o);
-        p.y[(size_t)s * p.ldy + (p.chain_major ? (k & 7) * (p.K / 8) + (k >> 3) : k)] = o;
+        p.y[(size_t)s * p.ldy + k] = o;
     }
     if (__any(bad_u) && (threadIdx.x & 63) == 0) seq_flag(p.nan_codes, s, p.layer, p.st_a);
     if (__any(bad_o) && (threadIdx.x & 63) == 0) seq_flag(p.nan_codes, s, p.layer, p.st_b);
@@ -504,7 +337,7 @@ __global__ __launch_bounds__(256) void swiglu_rows_kernel(BatchRowParams p) {
         if (rms > p.h_scale) sc = p.h_scale / rms;
     }
     for (int64_t k = tid; k < p.K; k += 256)
-        p.y[(size_t)s * p.ldy + (p.chain_major ? (k & 7) * (p.K / 8) + (k >> 3) : k)] = p.gnorm ? xs[k] * sc : xs[k];
+        p.y[(size_t)s * p.ldy + k] = p.gnorm ? xs[k] * sc : xs[k];
 }
 
 // Greedy argmax per sequence (llm/forward.rs:262-271: strict '>', so the first
@@ -564,28 +397,6 @@ __global__ void batch_end_kernel(BatchState b, uint32_t *out, int64_t n, int64_t
     if (out) out[(size_t)s * n + i] = nx;
 }
 
-template <int NV, int VPW>
-int launch_q4(const BatchGemvParams &p, hipStream_t s) {
-    // two rows per lane halve the LDS reads per FMA (long matrices); one row
-    // per lane when that leaves too few workgroups, and then the batch is
-    // split over the grid's second dimension, four vectors per workgroup (two
-    // waves of two): with fewer rows than lanes to fill the chip, more and
-    // smaller workgroups keep more SIMDs busy (Qwen2.5-1.5B shapes, batch 16:
-    // 5.45 -> 4.96 ms per step)
-    if (p.N >= 16 * 1024) {
-        const size_t lds = (size_t)2 * NV * 8 * BQ_CROW * 4;
-        hipLaunchKernelGGL((gemv_batch_q4_kernel<NV, VPW, 2>), dim3((unsigned)((p.N + 15) / 16)), dim3(NV / VPW * 64), lds, s, p);
-    } else {
-        constexpr int SNV = 4, SVPW = 2;
-        static_assert(NV % SNV == 0, "the batch splits into groups of four vectors");
-        const size_t lds = (size_t)2 * SNV * 8 * BQ_CROW * 4;
-        hipLaunchKernelGGL((gemv_batch_q4_kernel<SNV, SVPW, 1>), dim3((unsigned)((p.N + 7) / 8), NV / SNV),
-                           dim3(SNV / SVPW * 64), lds, s, p);
-    }
-    GAJE_HIP_CHECK(hipGetLastError());
-    return GAJE_OK;
-}
-
 template <int NV>
 int launch_f32(const BatchGemvParams &p, hipStream_t s) {
     const size_t lds = (size_t)NV * p.K * 4;
@@ -601,15 +412,10 @@ int launch_f32(const BatchGemvParams &p, hipStream_t s) {
 int batch_lanes(int64_t n) { return n <= 4 ? 4 : n <= 8 ? 8 : 16; }
 
 int launch_gemv_batch(const BatchGemvParams &p, hipStream_t s) {
+    if (p.fmt == FMT_Q4_0) return launch_q4_rows(p, s);
     if (!p.w || !p.x || !p.y || p.N <= 0 || p.nv <= 0 || p.nv > 16 || p.ldx < p.K || p.ldy < p.N)
         return set_error(GAJE_ERR_INVALID_ARG, "batched matvec: bad arguments");
     const int nv = batch_lanes(p.nv);
-    if (p.fmt == FMT_Q4_0) {
-        if (p.nb <= 0 || (int64_t)p.nb * 32 != p.K) return set_error(GAJE_ERR_INVALID_ARG, "batched matvec: bad K");
-        if (nv == 4) return launch_q4<4, 4>(p, s);
-        if (nv == 8) return launch_q4<8, 4>(p, s);
-        return launch_q4<16, 4>(p, s);
-    }
     if (p.fmt == FMT_F32) {
         if (!p.f32_tiled || p.K % 8) return set_error(GAJE_ERR_UNSUPPORTED, "batched matvec: f32 rows must be tiled");
         if (p.mode != MODE_STORE) return set_error(GAJE_ERR_UNSUPPORTED, "batched matvec: f32 rows store only");
@@ -640,7 +446,7 @@ int launch_gemv_batch(const BatchGemvParams &p, hipStream_t s) {
 }
 
 int launch_rmsnorm_rows(const BatchRowParams &p, hipStream_t s) {
-    if (!p.x || !p.y || p.K <= 0 || p.nv <= 0 || (p.chain_major && p.K % 8))
+    if (!p.x || !p.y || p.K <= 0 || p.nv <= 0 || p.nv > INT32_MAX)
         return set_error(GAJE_ERR_INVALID_ARG, "rmsnorm rows: bad arguments");
     if (p.K % 32 == 0 && p.K <= RN_XB4 * 4 * 256 && p.ldx % 4 == 0 && !(((uintptr_t)p.x | (uintptr_t)p.w) & 15)) {
         hipLaunchKernelGGL(rmsnorm_rows_cm_kernel, dim3((unsigned)p.nv), dim3(256), (size_t)8 * rn_chain_row(p.K) * 4, s, p);
@@ -654,7 +460,7 @@ int launch_rmsnorm_rows(const BatchRowParams &p, hipStream_t s) {
 }
 
 int launch_swiglu_rows(const BatchRowParams &p, hipStream_t s) {
-    if (!p.x || !p.y || p.K <= 0 || p.nv <= 0) return set_error(GAJE_ERR_INVALID_ARG, "swiglu rows: bad arguments");
+    if (!p.x || !p.y || p.K <= 0 || p.nv <= 0 || p.nv > 65535) return set_error(GAJE_ERR_INVALID_ARG, "swiglu rows: bad arguments");
     if (!p.gnorm) {
         hipLaunchKernelGGL(swiglu_elems_kernel, dim3((unsigned)((p.K + 255) / 256), (unsigned)p.nv), dim3(256), 0, s, p);
         GAJE_HIP_CHECK(hipGetLastError());

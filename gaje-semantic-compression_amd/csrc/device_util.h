@@ -166,6 +166,50 @@ __device__ __forceinline__ float4 ld_f4(const float *p) {
     return make_float4(v.x, v.y, v.z, v.w);
 }
 
+// Q4_0 dequantisation of packed groups (launch_pack_q4_0's layout).
+// The codes are never converted to float on their own.  A 4-bit code q masked
+// into bits 0..3 of a 16-bit half is the f16 subnormal q * 2^-24, and masked
+// into bits 4..7 it is q * 2^-20; v_fma_mix_f32 reads such a half exactly, so
+// fma(q * 2^-k, scale * 2^k, min) with the f32 scale * 2^k (exact: a power-of-
+// two shift of an f16) has the exact product q * scale and rounds once, the
+// same value as fma(q, scale, min) for every scale and min.  A chain dword h
+// holds block 2h's codes in the low nibbles (element c in byte c) and block
+// 2h+1's in the high ones, so one AND gives two of block 2h's codes at 2^-24
+// (elements 0 and 2 in the halves) and one two of block 2h+1's at 2^-20; the
+// dword shifted right by 8 gives elements 1 and 3 the same way.  Per group
+// that is 2 shifts, 8 ANDs and 4 scale products instead of 16 byte-to-float
+// conversions (half-rate instructions) and 6 masks.
+__device__ __forceinline__ float f16_lo(uint32_t v) {
+    union { uint16_t u; _Float16 h; } c;
+    c.u = (uint16_t)v;
+    return (float)c.h;
+}
+__device__ __forceinline__ float f16_hi(uint32_t v) {
+    union { uint16_t u; _Float16 h; } c;
+    c.u = (uint16_t)(v >> 16);
+    return (float)c.h;
+}
+
+// The four values of block 2h (dq = 0) or 2h+1 (dq = 1) of chain dword n,
+// with sm its scale | min << 16 word.
+template <int DQ>
+__device__ __forceinline__ void q4_dequant_dw(float (&d)[4], uint32_t n, uint32_t sm) {
+    constexpr uint32_t M = DQ ? 0x00F000F0u : 0x000F000Fu;
+    // S = scale * 2^20 or 2^24 in one v_fma_mix_f32 reading the f16 scale from
+    // the low half (exact: a power-of-two shift of an f16; + -0 keeps the
+    // product's sign, zeros included), in place of a conversion and a multiply
+    float S;
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]"
+        : "=v"(S)
+        : "v"(sm), "v"(DQ ? 1048576.0f : 16777216.0f), "v"(-0.0f));
+    const float mn = half_hi(sm);
+    const uint32_t e02 = opaque_and(n, M), e13 = opaque_and(n >> 8, M);
+    d[0] = fmaf(f16_lo(e02), S, mn);
+    d[1] = fmaf(f16_lo(e13), S, mn);
+    d[2] = fmaf(f16_hi(e02), S, mn);
+    d[3] = fmaf(f16_hi(e13), S, mn);
+}
+
 // Orderable encoding of a float: a > b  <=>  key(a) > key(b) (NaN excluded).
 __device__ __forceinline__ uint32_t order_key(float f) {
     uint32_t u = __float_as_uint(f);

@@ -173,14 +173,13 @@ struct AttnParams {
     float *out;              // [n_head * head_dim]
     DevState *st;            // positions 0..st->pos are attended; if null, 0..ctx-1
     int64_t ctx;
-    // batched decode (seq_pos non-null): blockIdx.z = sequence z attends to
-    // positions 0..seq_pos[z] of its own cache (k/v_cache + z * seq_kv_stride);
-    // its q and out rows are z * seq_q_stride floats on; seq_pos[z] < 0 skips
-    // it; out_chain_major writes each out row chain-major over n_head*head_dim
-    const int32_t *seq_pos;
+    // rows of several tokens (seq_pos non-null): row z attends to positions
+    // 0..seq_pos[z] of the cache of sequence row_seq[z] (row_seq null: z), at
+    // k/v_cache + sequence * seq_kv_stride; its q and out rows are
+    // z * seq_q_stride floats on; seq_pos[z] < 0 skips it
+    const int32_t *seq_pos, *row_seq;
     int64_t seq_kv_stride, seq_q_stride;
-    int32_t n_seq;
-    int32_t out_chain_major;
+    int32_t n_seq;           // rows
     // where a kernel whose LDS producers and consumers wait on each other
     // reports a wait that ran out of its spin bound (layer * 8 + ST_WAIT):
     // st->nan_code for one sequence, seq_nan[z] for batched sequence z
@@ -379,9 +378,10 @@ struct PrefillRopeParams {
     int64_t cap, pos0, P;
     int32_t n_head, n_kv, head_dim, rope_split;
     const float *rope_cos, *rope_sin;  // [cap][head_dim / 2]
-    // batched decode: row t is sequence t at position seq_pos[t] (< 0: skipped)
-    // of its own cache (k/v_cache + t * seq_kv_stride); pos0 unused
-    const int32_t *seq_pos;
+    // rows of several sequences: row t is a token of sequence row_seq[t]
+    // (row_seq null: t) at position seq_pos[t] (< 0: skipped) of its cache
+    // (k/v_cache + sequence * seq_kv_stride); pos0 unused
+    const int32_t *seq_pos, *row_seq;
     int64_t seq_kv_stride;
     // prefill: the qkv rows from a split-K product's partials, [nsplit][P][ldq]
     // (its deferred reduce: flush_small(sum) + bias), or null
@@ -419,17 +419,17 @@ constexpr int PREFILL_ATTN_REC_PAD = 4;
 int64_t prefill_kv16_halves(int64_t keys, int64_t n_kv, int64_t head_dim);
 int launch_prefill_attention(const PrefillAttnParams &p, hipStream_t s);
 
-// Batched decode: NV (<= 16) activation vectors per matvec, each product in
-// the batch-1 order (bit-identical per vector).
+// nv activation vectors per matvec (FMT_F32: at most 16), each product in the
+// batch-1 order (bit-identical per vector).
 struct BatchGemvParams {
     const uint8_t *w;        // FMT_Q4_0 packed rows, or FMT_F32 tiled rows
     int32_t fmt;
     int32_t f32_tiled;
     int32_t nb;              // K / 32 (Q4_0)
     int64_t N, K;
-    const float *x;          // [nv][ldx]; FMT_Q4_0: each row chain-major (element k at (k%8)*K/8 + k/8)
+    const float *x;          // [nv][ldx]
     int64_t ldx;
-    int32_t nv;              // vectors (sequences)
+    int64_t nv;              // vectors (sequences)
     const float *bias;
     int64_t bias_len;
     const int64_t *a_ptr;    // sparse anchors (Q4_0 only) or null
@@ -442,6 +442,8 @@ struct BatchGemvParams {
     int32_t layer, st_a, st_b;
 };
 int launch_gemv_batch(const BatchGemvParams &p, hipStream_t s);
+// Its Q4_0 products (any nv).
+int launch_q4_rows(const BatchGemvParams &p, hipStream_t s);
 // Activation lanes a batch of n sequences is padded to (4, 8 or 16).
 int batch_lanes(int64_t n);
 // Per-sequence row passes of the batched step.
@@ -452,10 +454,9 @@ struct BatchRowParams {
     int64_t ldy;
     const float *w;          // rms_norm weight [K]
     int64_t K;
-    int32_t nv;
+    int64_t nv;
     float eps, h_scale;
     int32_t gnorm;
-    int32_t chain_major;     // write y rows chain-major (input of a batched Q4_0 matvec)
     uint32_t *nan_codes;
     int32_t layer, st_a, st_b;
 };
@@ -500,6 +501,8 @@ int launch_moe_combine_split(const MoeParams &p, const float *part, int nsplit, 
 
 int launch_finalize(DevState *st, uint32_t *out_tokens, hipStream_t s);
 int launch_kwta(float *x, int64_t n, int64_t k, DevState *st, hipStream_t s);
+// The same for `rows` rows x + r * ld.
+int launch_kwta_rows(float *x, int64_t n, int64_t ld, int64_t rows, int64_t k, hipStream_t s);
 // Greedy generate step on the device: gen_select replaces st->token with the
 // argmax of the penalised logits (penalty > 1) into gs->key; gen_control takes
 // that choice (select) or st->token, appends it to the generated tokens and

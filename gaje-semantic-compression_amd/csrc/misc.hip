@@ -80,7 +80,8 @@ __device__ __forceinline__ void kw_count(uint32_t *h, uint32_t key, bool in, int
 }
 
 template <int T>
-__global__ __launch_bounds__(T) void kwta_kernel(float *x, int64_t n, int64_t k, DevState *st) {
+__global__ __launch_bounds__(T) void kwta_kernel(float *x, int64_t n, int64_t k, DevState *st, int64_t ld) {
+    x += (size_t)blockIdx.x * ld;
     constexpr int W = T / 64, HW = W < 8 ? W : 8;  // waves, histogram copies (waves w and w + 8 share one)
     if (st && st->halted) return;
     if (n <= k || k <= 0) return;
@@ -183,7 +184,8 @@ __global__ __launch_bounds__(T) void kwta_kernel(float *x, int64_t n, int64_t k,
 // (the blocks' hidden states): one wave, the row copied into LDS, wave_kwta
 // (the fused form the QKV matvec runs), the row written back.
 constexpr int KWW_MAX = WAVE * 4 * KW_WQ;
-__global__ __launch_bounds__(WAVE) void kwta_wave_kernel(float *x, int n, int64_t k, DevState *st) {
+__global__ __launch_bounds__(WAVE) void kwta_wave_kernel(float *x, int n, int64_t k, DevState *st, int64_t ld) {
+    x += (size_t)blockIdx.x * ld;
     __shared__ __align__(16) float xs[KWW_MAX];
     __shared__ __align__(16) uint32_t hist[4 * 320];
     if (st && st->halted) return;
@@ -388,15 +390,23 @@ int launch_state_set(DevState *st, int32_t pos, uint32_t token, int32_t out_cap,
     return GAJE_OK;
 }
 
-int launch_kwta(float *x, int64_t n, int64_t k, DevState *st, hipStream_t s) {
-    if (!x || n < 0) return set_error(GAJE_ERR_INVALID_ARG, "kwta: bad arguments");
+namespace {
+int kwta_grid(float *x, int64_t n, int64_t ld, int64_t rows, int64_t k, DevState *st, hipStream_t s) {
+    if (!x || n < 0 || rows < 1 || rows > INT32_MAX || (rows > 1 && ld < n)) return set_error(GAJE_ERR_INVALID_ARG, "kwta: bad arguments");
     if (n <= k || k <= 0) return GAJE_OK;
     if (n % 4 == 0 && n <= KWW_MAX)
-        hipLaunchKernelGGL(kwta_wave_kernel, dim3(1), dim3(WAVE), 0, s, x, (int)n, k, st);
+        hipLaunchKernelGGL(kwta_wave_kernel, dim3((unsigned)rows), dim3(WAVE), 0, s, x, (int)n, k, st, ld);
     else
-        hipLaunchKernelGGL(kwta_kernel<1024>, dim3(1), dim3(1024), 0, s, x, n, k, st);
+        hipLaunchKernelGGL(kwta_kernel<1024>, dim3((unsigned)rows), dim3(1024), 0, s, x, n, k, st, ld);
     GAJE_HIP_CHECK(hipGetLastError());
     return GAJE_OK;
+}
+}  // namespace
+
+int launch_kwta(float *x, int64_t n, int64_t k, DevState *st, hipStream_t s) { return kwta_grid(x, n, n, 1, k, st, s); }
+
+int launch_kwta_rows(float *x, int64_t n, int64_t ld, int64_t rows, int64_t k, hipStream_t s) {
+    return kwta_grid(x, n, ld, rows, k, nullptr, s);
 }
 
 int launch_argmax(const float *x, int64_t n, uint32_t *idx, hipStream_t s) {

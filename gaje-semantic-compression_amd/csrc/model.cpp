@@ -261,6 +261,15 @@ int fuse_linears(std::vector<HostLinear> parts, const std::string &name, HostLin
     return GAJE_OK;
 }
 
+// Activations of several token rows passing through the blocks together
+// (rows_blocks): rows of one prompt, or of the sequences of a batch.
+struct RowBufs {
+    int64_t rows = 0;        // rows they hold
+    float *H = nullptr, *XN = nullptr, *QKV = nullptr, *Q = nullptr, *ATT = nullptr, *GU = nullptr, *ACT = nullptr;
+    uint32_t *ids = nullptr;  // [3][rows]: embedding rows, then each row's position and sequence
+    uint32_t *nan_codes = nullptr;  // [rows] guards
+};
+
 }  // namespace
 }  // namespace gaje
 
@@ -323,6 +332,7 @@ struct gaje_hip_model {
         uint16_t *kv16 = nullptr;  // attention's f16 keys and values, prefill_kv16_halves(kv16_keys, ..)
         int64_t kv16_keys = 0;
     } pf;
+    RowBufs rb;  // the bit-exact prompt's rows
 
     std::vector<void *> allocs;
     std::vector<gaje_hip_batch *> batches;  // open batches over these weights
@@ -567,9 +577,7 @@ int enqueue_head(gaje_hip_model *m) {
     return launch_finalize(m->st, m->out_tokens, m->stream);
 }
 
-// Enqueue one decode step (embedding -> blocks -> output norm -> lm_head ->
-// argmax/advance) on the model stream.
-int enqueue_token(gaje_hip_model *m, hipEvent_t ev_blocks_done) {
+EmbedParams embed_params(const gaje_hip_model *m, float *h) {
     EmbedParams ep;
     memset(&ep, 0, sizeof ep);
     ep.w = m->embd.w;
@@ -581,7 +589,14 @@ int enqueue_token(gaje_hip_model *m, hipEvent_t ev_blocks_done) {
     ep.vocab = m->vocab_embd;
     ep.rows_valid = m->embd.rows_valid;
     ep.K = m->n_embd;
-    ep.h = m->h;
+    ep.h = h;
+    return ep;
+}
+
+// Enqueue one decode step (embedding -> blocks -> output norm -> lm_head ->
+// argmax/advance) on the model stream.
+int enqueue_token(gaje_hip_model *m, hipEvent_t ev_blocks_done) {
+    EmbedParams ep = embed_params(m, m->h);
     ep.st = m->st;
     GAJE_TRY(launch_embed(ep, m->stream));
 
@@ -993,12 +1008,184 @@ extern "C" int gaje_hip_reserve(gaje_hip_model *m, int64_t positions) {
     return m->n_layers > 0 ? reserve_ctx(m, positions) : GAJE_OK;
 }
 
-extern "C" int gaje_hip_prefill(gaje_hip_model *m, const uint32_t *ids, int64_t n, float *last_logits_host) {
-    clear_error();
-    GAJE_TRY(check_model(m));
-    if (n < 0 || (n > 0 && !ids)) return set_error(GAJE_ERR_INVALID_ARG, "bad prefill arguments");
-    if (n == 0) return GAJE_OK;
-    GAJE_TRY(reserve_ctx(m, m->pos + n));
+namespace {
+
+// Rows of one bit-exact pass: enough that the products' tiles fill the chip
+// several times, few enough that the buffers stay small (the gate/up rows of a
+// 1.5B-parameter model: 73 MB).
+constexpr int64_t ROWS_CHUNK = 1024;
+
+// Token rows whose blocks run together (rows_blocks): row r is a token of
+// sequence seq[r] at position pos[r] of its cache (pos[r] < 0: computed and
+// discarded), or, with pos null, row r is position pos0 + r of the one cache.
+struct RowPass {
+    const RowBufs *b = nullptr;
+    int64_t R = 0;
+    const int32_t *pos = nullptr, *seq = nullptr;
+    int64_t pos0 = 0;
+    float *k_cache = nullptr, *v_cache = nullptr;  // layer 0
+    int64_t layer_kv = 0, seq_kv = 0, cap = 0;     // floats per layer and per sequence, positions
+    const float *rope_cos = nullptr, *rope_sin = nullptr;
+};
+
+// Whether every block runs on rows: complete Q4_0 body tensors of sizes that
+// the token step takes.
+bool rows_supported(const gaje_hip_model *m) {
+    for (const Layer &Ly : m->layers)
+        for (const DevLinear *D : {&Ly.qkv, &Ly.o, &Ly.gate_up, &Ly.down})
+            if (D->fmt != FMT_Q4_0 || D->rows_valid != D->N || D->K % 32 || D->N <= 0 ||
+                gemv_lds_bytes(D->K, FMT_Q4_0, D == &Ly.qkv || D == &Ly.gate_up) + 1024 > max_lds_per_block())
+                return false;
+    return m->n_layers > 0;
+}
+
+// Owner: gaje_hip_model or gaje_hip_batch (alloc and release).
+template <class Owner>
+int rows_reserve(Owner *o, const gaje_hip_model *m, RowBufs &b, int64_t rows) {
+    if (rows <= b.rows) return GAJE_OK;
+    GAJE_HIP_CHECK(hipStreamSynchronize(m->stream));
+    for (void *p : {(void *)b.H, (void *)b.XN, (void *)b.QKV, (void *)b.Q, (void *)b.ATT, (void *)b.GU, (void *)b.ACT,
+                    (void *)b.ids, (void *)b.nan_codes})
+        if (p) o->release(p);
+    b = RowBufs();
+    const Layer &L0 = m->layers[0];
+    GAJE_TRY(o->alloc(&b.H, (size_t)(rows * m->n_embd)));
+    GAJE_TRY(o->alloc(&b.XN, (size_t)(rows * m->n_embd)));
+    GAJE_TRY(o->alloc(&b.QKV, (size_t)(rows * L0.qkv.N)));
+    GAJE_TRY(o->alloc(&b.Q, (size_t)(rows * m->q_rows)));
+    GAJE_TRY(o->alloc(&b.ATT, (size_t)(rows * m->q_rows)));
+    GAJE_TRY(o->alloc(&b.GU, (size_t)(rows * L0.gate_up.N)));
+    GAJE_TRY(o->alloc(&b.ACT, (size_t)(rows * m->ffn)));
+    GAJE_TRY(o->alloc(&b.ids, (size_t)(3 * rows)));
+    GAJE_TRY(o->alloc(&b.nan_codes, (size_t)rows));
+    b.rows = rows;
+    return GAJE_OK;
+}
+
+BatchGemvParams rows_gemv(const DevLinear &D, const float *x, int64_t ldx, float *y, int64_t ldy, int64_t rows,
+                          uint32_t *nan_codes) {
+    BatchGemvParams p{};
+    p.w = D.w;
+    p.fmt = D.fmt;
+    p.f32_tiled = D.f32_tiled;
+    p.nb = (int32_t)(D.K / 32);
+    p.N = D.N;
+    p.K = D.K;
+    p.x = x;
+    p.ldx = ldx;
+    p.nv = rows;
+    p.bias = D.bias;
+    p.bias_len = D.bias_len;
+    p.a_ptr = D.a_ptr;
+    p.a_col = D.a_col;
+    p.a_val = D.a_val;
+    p.mode = MODE_STORE;
+    p.y = y;
+    p.ldy = ldy;
+    p.nan_codes = nan_codes;
+    p.st_a = p.st_b = ST_NONE;
+    return p;
+}
+
+BatchRowParams rows_pass(const gaje_hip_model *m, const float *x, int64_t ldx, float *y, int64_t ldy, int64_t K,
+                         int64_t rows, uint32_t *nan_codes) {
+    BatchRowParams r{};
+    r.x = x;
+    r.ldx = ldx;
+    r.y = y;
+    r.ldy = ldy;
+    r.K = K;
+    r.nv = rows;
+    r.eps = m->eps;
+    r.h_scale = 1.0f;
+    r.nan_codes = nan_codes;
+    r.st_a = r.st_b = ST_NONE;
+    return r;
+}
+
+// Every block (RustGenomicBlock::forward_core, block/forward.rs:10-157) for the
+// rows of a pass, in place on b->H.  Each row's values and guards are those of
+// its own token step (enqueue_token), bit for bit: the same chains and
+// reductions, several rows at a time.
+int rows_blocks(gaje_hip_model *m, const RowPass &c) {
+    hipStream_t s = m->stream;
+    const RowBufs &b = *c.b;
+    const int64_t R = c.R, E = m->n_embd;
+    for (int64_t l = 0; l < m->n_layers; ++l) {
+        Layer &Ly = m->layers[l];
+        const int32_t li = (int32_t)l;
+        const int64_t qkvN = Ly.qkv.N, guN = Ly.gate_up.N;
+        float *kc = c.k_cache + l * c.layer_kv, *vc = c.v_cache + l * c.layer_kv;
+        BatchRowParams r = rows_pass(m, b.H, E, b.XN, E, E, R, b.nan_codes);
+        r.w = Ly.attn_norm;  // null: the rows as they are
+        r.layer = li;
+        r.st_a = ST_INPUT;
+        r.st_b = Ly.attn_norm ? ST_ATTN_NORM : ST_NONE;
+        GAJE_TRY(launch_rmsnorm_rows(r, s));
+        GAJE_TRY(launch_gemv_batch(rows_gemv(Ly.qkv, b.XN, E, b.QKV, qkvN, R, b.nan_codes), s));
+        PrefillRopeParams rp{};
+        rp.qkv = b.QKV;
+        rp.ldq = qkvN;
+        rp.q_out = b.Q;
+        rp.k_cache = kc;
+        rp.v_cache = vc;
+        rp.cap = c.cap;
+        rp.pos0 = c.pos0;
+        rp.P = R;
+        rp.n_head = (int32_t)m->n_head;
+        rp.n_kv = (int32_t)m->n_kv;
+        rp.head_dim = (int32_t)m->hd;
+        rp.rope_split = m->rope_split;
+        rp.rope_cos = c.rope_cos;
+        rp.rope_sin = c.rope_sin;
+        rp.seq_pos = c.pos0 >= 0 ? nullptr : c.pos;
+        rp.row_seq = c.seq;
+        rp.seq_kv_stride = c.seq_kv;
+        GAJE_TRY(launch_rope_kv(rp, s));
+        AttnParams ap{};
+        ap.q = b.Q;
+        ap.k_cache = kc;
+        ap.v_cache = vc;
+        ap.kv_head_stride = c.cap * m->hd;
+        ap.n_head = (int32_t)m->n_head;
+        ap.n_head_kv = (int32_t)m->n_kv;
+        ap.head_dim = (int32_t)m->hd;
+        ap.kv_cap = c.cap;
+        ap.out = b.ATT;
+        ap.seq_pos = c.pos;
+        ap.row_seq = c.seq;
+        ap.seq_kv_stride = c.seq_kv;
+        ap.seq_q_stride = m->q_rows;
+        ap.n_seq = (int32_t)R;
+        ap.seq_nan = b.nan_codes;
+        ap.layer = li;
+        GAJE_TRY(launch_attention(ap, s));
+        BatchGemvParams g = rows_gemv(Ly.o, b.ATT, m->q_rows, b.H, E, R, b.nan_codes);
+        g.mode = MODE_RESIDUAL;
+        GAJE_TRY(launch_gemv_batch(g, s));
+        r = rows_pass(m, b.H, E, b.XN, E, E, R, b.nan_codes);
+        r.w = Ly.ffn_norm;
+        GAJE_TRY(launch_rmsnorm_rows(r, s));
+        GAJE_TRY(launch_gemv_batch(rows_gemv(Ly.gate_up, b.XN, E, b.GU, guN, R, b.nan_codes), s));
+        r = rows_pass(m, b.GU, guN, b.ACT, m->ffn, m->ffn, R, b.nan_codes);
+        r.gnorm = m->use_genomic_norm;
+        r.layer = li;
+        r.st_a = ST_UP;
+        r.st_b = ST_FFN_OUT;
+        GAJE_TRY(launch_swiglu_rows(r, s));
+        g = rows_gemv(Ly.down, b.ACT, m->ffn, b.H, E, R, b.nan_codes);
+        g.mode = MODE_RESIDUAL;
+        g.layer = li;
+        g.st_a = ST_PROJ_FFN;
+        g.st_b = ST_FINAL;
+        GAJE_TRY(launch_gemv_batch(g, s));
+        if (const int64_t k = block_kwta_k(m)) GAJE_TRY(launch_kwta_rows(b.H, E, E, R, k, s));
+    }
+    return GAJE_OK;
+}
+
+// n tokens one step at a time from m->pos (the captured token graph).
+int prefill_steps(gaje_hip_model *m, const uint32_t *ids, int64_t n, DevState &s) {
     if (!m->profile) GAJE_TRY(ensure_graph(m));
     GAJE_TRY(launch_state_set(m->st, (int32_t)m->pos, ids[0], -1, -1, 1, m->stream));
     for (int64_t i = 0; i < n; ++i) {
@@ -1006,18 +1193,82 @@ extern "C" int gaje_hip_prefill(gaje_hip_model *m, const uint32_t *ids, int64_t 
         if (i > 0) GAJE_TRY(launch_state_set(m->st, -1, ids[i], -1, -1, 0, m->stream));
         GAJE_TRY(run_token(m));
     }
-    if (last_logits_host && m->kwta_ratio > 0.0f && m->kwta_ratio < 1.0f)
-        GAJE_TRY(launch_kwta(m->logits, m->vocab_out, kwta_k(m->vocab_out, m->kwta_ratio), m->st, m->stream));
-    DevState s;
     GAJE_TRY(read_state(m, s));
-    const int64_t done = (int64_t)s.pos - m->pos;
     m->pos = s.pos;
-    if (s.halted || s.nan_code != NAN_NONE) {
-        (void)done;
-        return nan_error(s);
+    return s.halted || s.nan_code != NAN_NONE ? nan_error(s) : GAJE_OK;
+}
+
+// n tokens (at most ROWS_CHUNK) as rows of one pass at positions m->pos..: the
+// keys and values appended, the rows' hidden states in m->rb.H.  `clean` tells
+// whether every guard held; if one fired nothing is committed (the cache length
+// stays), and the caller runs the tokens one by one, which stops at the token
+// that the reference stops at.
+int prefill_rows(gaje_hip_model *m, const uint32_t *ids, int64_t n, bool &clean) {
+    RowBufs &b = m->rb;
+    hipStream_t s = m->stream;
+    GAJE_TRY(rows_reserve(m, m, b, n));
+    std::vector<uint32_t> up((size_t)(2 * n));
+    for (int64_t i = 0; i < n; ++i) {
+        up[i] = ids[i];
+        up[n + i] = (uint32_t)(m->pos + i);
     }
-    if (last_logits_host)
-        GAJE_HIP_CHECK(hipMemcpy(last_logits_host, m->logits, (size_t)m->vocab_out * 4, hipMemcpyDeviceToHost));
+    GAJE_HIP_CHECK(hipMemcpyAsync(b.ids, up.data(), up.size() * 4, hipMemcpyHostToDevice, s));
+    GAJE_TRY(launch_fill_u32(b.nan_codes, NAN_NONE, n, s));
+    GAJE_TRY(launch_embed_rows(embed_params(m, b.H), b.ids, n, s));
+    RowPass c;
+    c.b = &b;
+    c.R = n;
+    c.pos = (const int32_t *)(b.ids + n);
+    c.pos0 = m->pos;
+    c.k_cache = m->k_cache;
+    c.v_cache = m->v_cache;
+    c.layer_kv = m->n_kv * m->cap * m->hd;
+    c.cap = m->cap;
+    c.rope_cos = m->rope_cos;
+    c.rope_sin = m->rope_sin;
+    GAJE_TRY(rows_blocks(m, c));
+    GAJE_HIP_CHECK(hipMemcpyAsync(up.data(), b.nan_codes, (size_t)n * 4, hipMemcpyDeviceToHost, s));
+    GAJE_HIP_CHECK(hipStreamSynchronize(s));
+    clean = true;
+    for (int64_t i = 0; i < n; ++i) clean = clean && up[i] == NAN_NONE;
+    return GAJE_OK;
+}
+
+}  // namespace
+
+extern "C" int gaje_hip_prefill(gaje_hip_model *m, const uint32_t *ids, int64_t n, float *last_logits_host) {
+    clear_error();
+    GAJE_TRY(check_model(m));
+    if (n < 0 || (n > 0 && !ids)) return set_error(GAJE_ERR_INVALID_ARG, "bad prefill arguments");
+    if (n == 0) return GAJE_OK;
+    GAJE_TRY(reserve_ctx(m, m->pos + n));
+    DevState s;
+    const bool rows = n > 1 && !m->profile && rows_supported(m);
+    for (int64_t c0 = 0; c0 < n;) {
+        const int64_t P = rows ? std::min(ROWS_CHUNK, n - c0) : n;
+        bool clean = false;
+        if (rows) GAJE_TRY(prefill_rows(m, ids + c0, P, clean));
+        if (!clean) {
+            GAJE_TRY(prefill_steps(m, ids + c0, P, s));
+        } else if (c0 + P < n) {
+            m->pos += P;
+        } else {
+            // the last token's head, as its step ends: logits, argmax, position
+            GAJE_HIP_CHECK(hipMemcpyAsync(m->h, m->rb.H + (P - 1) * m->n_embd, (size_t)m->n_embd * 4,
+                                          hipMemcpyDeviceToDevice, m->stream));
+            GAJE_TRY(launch_state_set(m->st, (int32_t)(m->pos + P - 1), ids[n - 1], -1, -1, 1, m->stream));
+            GAJE_TRY(enqueue_head(m));
+            GAJE_TRY(read_state(m, s));
+            m->pos = s.pos;
+            if (s.halted || s.nan_code != NAN_NONE) return nan_error(s);
+        }
+        c0 += P;
+    }
+    if (!last_logits_host) return GAJE_OK;
+    if (m->kwta_ratio > 0.0f && m->kwta_ratio < 1.0f)
+        GAJE_TRY(launch_kwta(m->logits, m->vocab_out, kwta_k(m->vocab_out, m->kwta_ratio), m->st, m->stream));
+    GAJE_HIP_CHECK(hipMemcpyAsync(last_logits_host, m->logits, (size_t)m->vocab_out * 4, hipMemcpyDeviceToHost, m->stream));
+    GAJE_HIP_CHECK(hipStreamSynchronize(m->stream));
     return GAJE_OK;
 }
 
@@ -1315,19 +1566,7 @@ extern "C" int gaje_hip_prefill_mfma(gaje_hip_model *m, const uint32_t *ids, int
         }
         auto &f = m->pf;
         GAJE_HIP_CHECK(hipMemcpyAsync(f.ids, ids + c0, (size_t)P * 4, hipMemcpyHostToDevice, s));
-        EmbedParams ep;
-        memset(&ep, 0, sizeof ep);
-        ep.w = m->embd.w;
-        ep.fmt = m->embd.fmt;
-        ep.lut = m->embd.lut;
-        ep.lut_rows_own = m->embd.lut_rows_own;
-        ep.lut_block_stride = m->embd.lut_block_stride;
-        ep.lut_len = m->embd.lut_len;
-        ep.vocab = m->vocab_embd;
-        ep.rows_valid = m->embd.rows_valid;
-        ep.K = m->n_embd;
-        ep.h = f.H;
-        GAJE_TRY(launch_embed_rows(ep, f.ids, P, s));
+        GAJE_TRY(launch_embed_rows(embed_params(m, f.H), f.ids, P, s));
         PendingReduce pending;
         for (int64_t l = 0; l < m->n_layers; ++l) GAJE_TRY(prefill_layer(m, l, pos0 + c0, P, pending));
         last_rows = P;
@@ -1360,12 +1599,12 @@ struct gaje_hip_batch {
     int64_t nseq = 0, lanes = 0, cap = 0;
     float *k_cache = nullptr, *v_cache = nullptr;  // [layer][seq][n_kv][head_dim][cap]
     float *rope_cos = nullptr, *rope_sin = nullptr;
-    float *H = nullptr, *XN = nullptr, *QKV = nullptr, *Q = nullptr, *ATT = nullptr, *GU = nullptr, *ACT = nullptr,
-          *LOG = nullptr;
+    RowBufs sb, rb;  // a step's rows (one per sequence), and fed prompts' rows (grown on demand)
+    float *LOG = nullptr;
     uint32_t *ids = nullptr, *out = nullptr;  // fed tokens / greedy outputs [seq][n]
     int64_t ids_cap = 0, out_cap = 0;
     BatchState st{};
-    std::vector<int32_t> pos;  // host mirror of st.pos
+    std::vector<int32_t> pos, halted;  // host mirrors of st.pos and st.halted
     std::vector<void *> allocs;
 
     ~gaje_hip_batch() {
@@ -1404,144 +1643,38 @@ int batch_supported(const gaje_hip_model *m) {
     return GAJE_OK;
 }
 
-BatchGemvParams batch_gemv(const gaje_hip_batch *b, const DevLinear &D, const float *x, int64_t ldx, float *y,
-                           int64_t ldy) {
-    BatchGemvParams p{};
-    p.w = D.w;
-    p.fmt = D.fmt;
-    p.f32_tiled = D.f32_tiled;
-    p.nb = (int32_t)(D.K / 32);
-    p.N = D.N;
-    p.K = D.K;
-    p.x = x;
-    p.ldx = ldx;
-    p.nv = (int32_t)b->lanes;
-    p.bias = D.bias;
-    p.bias_len = D.bias_len;
-    p.a_ptr = D.a_ptr;
-    p.a_col = D.a_col;
-    p.a_val = D.a_val;
-    p.mode = MODE_STORE;
-    p.y = y;
-    p.ldy = ldy;
-    p.nan_codes = b->st.nan_codes;
-    p.st_a = p.st_b = ST_NONE;
-    return p;
-}
-
-BatchRowParams batch_rows(const gaje_hip_batch *b, const float *x, int64_t ldx, float *y, int64_t ldy, int64_t K) {
-    BatchRowParams r{};
-    r.x = x;
-    r.ldx = ldx;
-    r.y = y;
-    r.ldy = ldy;
-    r.K = K;
-    r.nv = (int32_t)b->lanes;
-    r.eps = b->m->eps;
-    r.h_scale = 1.0f;
-    r.nan_codes = b->st.nan_codes;
-    r.st_a = r.st_b = ST_NONE;
-    return r;
+// The rows of a pass over the batch's caches.
+RowPass batch_rows(const gaje_hip_batch *b, const RowBufs &rows, int64_t R, const int32_t *pos, const int32_t *seq) {
+    const gaje_hip_model *m = b->m;
+    RowPass c;
+    c.b = &rows;
+    c.R = R;
+    c.pos = pos;
+    c.seq = seq;
+    c.pos0 = -1;
+    c.k_cache = b->k_cache;
+    c.v_cache = b->v_cache;
+    c.seq_kv = m->n_kv * m->hd * b->cap;
+    c.layer_kv = b->nseq * c.seq_kv;
+    c.cap = b->cap;
+    c.rope_cos = b->rope_cos;
+    c.rope_sin = b->rope_sin;
+    return c;
 }
 
 // One step of every running sequence (the batched counterpart of enqueue_token).
 int batch_enqueue_step(gaje_hip_batch *b, const uint32_t *ids, int64_t n, int64_t i, uint32_t *out, bool greedy) {
     gaje_hip_model *m = b->m;
     hipStream_t s = m->stream;
-    const int64_t L = b->lanes, E = m->n_embd;
+    const int64_t E = m->n_embd;
     GAJE_TRY(launch_batch_begin(b->st, ids, n, i, s));
-    EmbedParams ep;
-    memset(&ep, 0, sizeof ep);
-    ep.w = m->embd.w;
-    ep.fmt = m->embd.fmt;
-    ep.lut = m->embd.lut;
-    ep.lut_rows_own = m->embd.lut_rows_own;
-    ep.lut_block_stride = m->embd.lut_block_stride;
-    ep.lut_len = m->embd.lut_len;
-    ep.vocab = m->vocab_embd;
-    ep.rows_valid = m->embd.rows_valid;
-    ep.K = E;
-    ep.h = b->H;
-    GAJE_TRY(launch_embed_rows(ep, b->st.embed_ids, L, s));
-    const int64_t seq_kv = m->n_kv * m->hd * b->cap;
-    const int64_t qkvN = m->layers.empty() ? 0 : m->layers[0].qkv.N, guN = m->layers.empty() ? 0 : m->layers[0].gate_up.N;
-    for (int64_t l = 0; l < m->n_layers; ++l) {
-        Layer &Ly = m->layers[l];
-        const int32_t li = (int32_t)l;
-        float *kc = b->k_cache + l * b->nseq * seq_kv, *vc = b->v_cache + l * b->nseq * seq_kv;
-        BatchRowParams r = batch_rows(b, b->H, E, b->XN, E, E);
-        r.w = Ly.attn_norm;  // null: the rows as they are
-        r.chain_major = 1;
-        r.layer = li;
-        r.st_a = ST_INPUT;
-        r.st_b = Ly.attn_norm ? ST_ATTN_NORM : ST_NONE;
-        GAJE_TRY(launch_rmsnorm_rows(r, s));
-        GAJE_TRY(launch_gemv_batch(batch_gemv(b, Ly.qkv, b->XN, E, b->QKV, qkvN), s));
-        PrefillRopeParams rp{};
-        rp.qkv = b->QKV;
-        rp.ldq = qkvN;
-        rp.q_out = b->Q;
-        rp.k_cache = kc;
-        rp.v_cache = vc;
-        rp.cap = b->cap;
-        rp.P = L;
-        rp.n_head = (int32_t)m->n_head;
-        rp.n_kv = (int32_t)m->n_kv;
-        rp.head_dim = (int32_t)m->hd;
-        rp.rope_split = m->rope_split;
-        rp.rope_cos = b->rope_cos;
-        rp.rope_sin = b->rope_sin;
-        rp.seq_pos = b->st.cur_pos;
-        rp.seq_kv_stride = seq_kv;
-        GAJE_TRY(launch_rope_kv(rp, s));
-        AttnParams ap{};
-        ap.q = b->Q;
-        ap.k_cache = kc;
-        ap.v_cache = vc;
-        ap.kv_head_stride = b->cap * m->hd;
-        ap.n_head = (int32_t)m->n_head;
-        ap.n_head_kv = (int32_t)m->n_kv;
-        ap.head_dim = (int32_t)m->hd;
-        ap.kv_cap = b->cap;
-        ap.out = b->ATT;
-        ap.seq_pos = b->st.cur_pos;
-        ap.seq_kv_stride = seq_kv;
-        ap.seq_q_stride = m->q_rows;
-        ap.n_seq = (int32_t)b->nseq;
-        ap.out_chain_major = 1;
-        ap.seq_nan = b->st.nan_codes;
-        ap.layer = (int32_t)li;
-        GAJE_TRY(launch_attention(ap, s));
-        BatchGemvParams g = batch_gemv(b, Ly.o, b->ATT, m->q_rows, b->H, E);
-        g.mode = MODE_RESIDUAL;
-        GAJE_TRY(launch_gemv_batch(g, s));
-        r = batch_rows(b, b->H, E, b->XN, E, E);
-        r.w = Ly.ffn_norm;
-        r.chain_major = 1;
-        GAJE_TRY(launch_rmsnorm_rows(r, s));
-        GAJE_TRY(launch_gemv_batch(batch_gemv(b, Ly.gate_up, b->XN, E, b->GU, guN), s));
-        r = batch_rows(b, b->GU, guN, b->ACT, m->ffn, m->ffn);
-        r.gnorm = m->use_genomic_norm;
-        r.chain_major = 1;
-        r.layer = li;
-        r.st_a = ST_UP;
-        r.st_b = ST_FFN_OUT;
-        GAJE_TRY(launch_swiglu_rows(r, s));
-        g = batch_gemv(b, Ly.down, b->ACT, m->ffn, b->H, E);
-        g.mode = MODE_RESIDUAL;
-        g.layer = li;
-        g.st_a = ST_PROJ_FFN;
-        g.st_b = ST_FINAL;
-        GAJE_TRY(launch_gemv_batch(g, s));
-        if (m->block_kwta_ratio > 0.0f && m->block_kwta_ratio < 1.0f) {
-            const int64_t k = kwta_k(E, m->block_kwta_ratio);
-            for (int64_t q = 0; q < b->nseq; ++q) GAJE_TRY(launch_kwta(b->H + q * E, E, k, nullptr, s));
-        }
-    }
-    BatchRowParams r = batch_rows(b, b->H, E, b->XN, E, E);
+    GAJE_TRY(launch_embed_rows(embed_params(m, b->sb.H), b->st.embed_ids, b->nseq, s));
+    GAJE_TRY(rows_blocks(m, batch_rows(b, b->sb, b->nseq, b->st.cur_pos, nullptr)));
+    BatchRowParams r = rows_pass(m, b->sb.H, E, b->sb.XN, E, E, b->nseq, b->st.nan_codes);
     r.w = m->output_norm;
     GAJE_TRY(launch_rmsnorm_rows(r, s));
-    GAJE_TRY(launch_gemv_batch(batch_gemv(b, m->lm_head, b->XN, E, b->LOG, m->vocab_out), s));
+    // the f32 head reads whole lanes; idle lanes' rows are zeros
+    GAJE_TRY(launch_gemv_batch(rows_gemv(m->lm_head, b->sb.XN, E, b->LOG, m->vocab_out, b->lanes, nullptr), s));
     GAJE_TRY(launch_argmax_rows(b->LOG, m->vocab_out, m->vocab_out, b->nseq, b->st.next, s));
     return launch_batch_end(b->st, out, n, i, greedy ? 1 : 0, s);
 }
@@ -1549,7 +1682,7 @@ int batch_enqueue_step(gaje_hip_batch *b, const uint32_t *ids, int64_t n, int64_
 // Reads the device state back; a sequence halted by a guard reports the
 // reference's message (the first such sequence's).
 int batch_sync(gaje_hip_batch *b, int32_t *status) {
-    std::vector<int32_t> halted((size_t)b->lanes);
+    std::vector<int32_t> &halted = b->halted;
     std::vector<uint32_t> err((size_t)b->lanes);
     hipStream_t s = b->m->stream;
     GAJE_HIP_CHECK(hipMemcpyAsync(b->pos.data(), b->st.pos, (size_t)b->lanes * 4, hipMemcpyDeviceToHost, s));
@@ -1564,6 +1697,55 @@ int batch_sync(gaje_hip_batch *b, int32_t *status) {
     if (first >= 0)
         return set_error((int)(err[first] % 8) == ST_WAIT ? GAJE_ERR_HIP : GAJE_ERR_NAN, "%s",
                          nan_message((int)(err[first] % 8)));
+    return GAJE_OK;
+}
+
+// Steps i0 .. i1 - 1 of a feed (ids on the host and in b->ids, [seq][n]) as
+// rows of shared passes: every running sequence's tokens at once, up to
+// ROWS_CHUNK rows a pass.  Nothing of a pass in which a guard fired is
+// committed: its steps run one at a time instead, where the sequence halts at
+// its own token and the others go on.
+int batch_feed_rows(gaje_hip_batch *b, const uint32_t *ids, int64_t n, int64_t i0, int64_t i1) {
+    gaje_hip_model *m = b->m;
+    hipStream_t s = m->stream;
+    const int64_t per = std::max<int64_t>(1, ROWS_CHUNK / b->nseq);
+    std::vector<uint32_t> up;
+    for (int64_t c0 = i0; c0 < i1; c0 += per) {
+        const int64_t c1 = std::min(i1, c0 + per);
+        std::vector<uint32_t> tok, pos, seq;
+        std::vector<int32_t> end(b->pos);
+        for (int64_t q = 0; q < b->nseq; ++q)
+            for (int64_t i = c0; i < c1 && !b->halted[q]; ++i)
+                if (ids[q * n + i] != BATCH_INACTIVE) {
+                    tok.push_back(ids[q * n + i]);
+                    pos.push_back((uint32_t)end[q]++);
+                    seq.push_back((uint32_t)q);
+                }
+        const int64_t R = (int64_t)tok.size();
+        if (R == 0) continue;
+        GAJE_TRY(rows_reserve(b, m, b->rb, R));
+        up.assign(tok.begin(), tok.end());
+        up.insert(up.end(), pos.begin(), pos.end());
+        up.insert(up.end(), seq.begin(), seq.end());
+        GAJE_HIP_CHECK(hipMemcpyAsync(b->rb.ids, up.data(), up.size() * 4, hipMemcpyHostToDevice, s));
+        GAJE_TRY(launch_fill_u32(b->rb.nan_codes, NAN_NONE, R, s));
+        GAJE_TRY(launch_embed_rows(embed_params(m, b->rb.H), b->rb.ids, R, s));
+        const int32_t *dpos = (const int32_t *)(b->rb.ids + R);
+        GAJE_TRY(rows_blocks(m, batch_rows(b, b->rb, R, dpos, dpos + R)));
+        GAJE_HIP_CHECK(hipMemcpyAsync(up.data(), b->rb.nan_codes, (size_t)R * 4, hipMemcpyDeviceToHost, s));
+        GAJE_HIP_CHECK(hipStreamSynchronize(s));
+        bool clean = true;
+        for (int64_t r = 0; r < R; ++r) clean = clean && up[r] == NAN_NONE;
+        if (clean) {
+            b->pos = end;
+            GAJE_HIP_CHECK(hipMemcpyAsync(b->st.pos, b->pos.data(), (size_t)b->lanes * 4, hipMemcpyHostToDevice, s));
+            GAJE_HIP_CHECK(hipStreamSynchronize(s));
+            continue;
+        }
+        for (int64_t i = c0; i < c1; ++i) GAJE_TRY(batch_enqueue_step(b, b->ids, n, i, nullptr, false));
+        const int rc = batch_sync(b, nullptr);
+        if (rc != GAJE_OK && rc != GAJE_ERR_NAN) return rc;  // (a halted sequence is reported at the feed's end)
+    }
     return GAJE_OK;
 }
 
@@ -1619,22 +1801,23 @@ extern "C" int gaje_hip_batch_open(gaje_hip_model *m, int64_t n_seq, int64_t cap
     }
     const int64_t qkvN = m->layers.empty() ? 1 : m->layers[0].qkv.N, guN = m->layers.empty() ? 2 : m->layers[0].gate_up.N;
     const int64_t qn = std::max<int64_t>(m->q_rows, 1), ffn = std::max<int64_t>(m->ffn, 1);
-    GAJE_TRY(b->alloc(&b->H, (size_t)(L * E)));
-    GAJE_TRY(b->alloc(&b->XN, (size_t)(L * E)));
-    GAJE_TRY(b->alloc(&b->QKV, (size_t)(L * qkvN)));
-    GAJE_TRY(b->alloc(&b->Q, (size_t)(L * qn)));
-    GAJE_TRY(b->alloc(&b->ATT, (size_t)(L * qn)));
-    GAJE_TRY(b->alloc(&b->GU, (size_t)(L * guN)));
-    GAJE_TRY(b->alloc(&b->ACT, (size_t)(L * ffn)));
+    RowBufs &sb = b->sb;
+    GAJE_TRY(b->alloc(&sb.H, (size_t)(L * E)));
+    GAJE_TRY(b->alloc(&sb.XN, (size_t)(L * E)));
+    GAJE_TRY(b->alloc(&sb.QKV, (size_t)(L * qkvN)));
+    GAJE_TRY(b->alloc(&sb.Q, (size_t)(L * qn)));
+    GAJE_TRY(b->alloc(&sb.ATT, (size_t)(L * qn)));
+    GAJE_TRY(b->alloc(&sb.GU, (size_t)(L * guN)));
+    GAJE_TRY(b->alloc(&sb.ACT, (size_t)(L * ffn)));
     GAJE_TRY(b->alloc(&b->LOG, (size_t)(L * m->vocab_out)));
     // rows of idle lanes are computed and discarded; zeroed, they stay finite
-    GAJE_HIP_CHECK(hipMemset(b->H, 0, (size_t)(L * E) * 4));
-    GAJE_HIP_CHECK(hipMemset(b->XN, 0, (size_t)(L * E) * 4));
-    GAJE_HIP_CHECK(hipMemset(b->QKV, 0, (size_t)(L * qkvN) * 4));
-    GAJE_HIP_CHECK(hipMemset(b->Q, 0, (size_t)(L * qn) * 4));
-    GAJE_HIP_CHECK(hipMemset(b->ATT, 0, (size_t)(L * qn) * 4));
-    GAJE_HIP_CHECK(hipMemset(b->GU, 0, (size_t)(L * guN) * 4));
-    GAJE_HIP_CHECK(hipMemset(b->ACT, 0, (size_t)(L * ffn) * 4));
+    GAJE_HIP_CHECK(hipMemset(sb.H, 0, (size_t)(L * E) * 4));
+    GAJE_HIP_CHECK(hipMemset(sb.XN, 0, (size_t)(L * E) * 4));
+    GAJE_HIP_CHECK(hipMemset(sb.QKV, 0, (size_t)(L * qkvN) * 4));
+    GAJE_HIP_CHECK(hipMemset(sb.Q, 0, (size_t)(L * qn) * 4));
+    GAJE_HIP_CHECK(hipMemset(sb.ATT, 0, (size_t)(L * qn) * 4));
+    GAJE_HIP_CHECK(hipMemset(sb.GU, 0, (size_t)(L * guN) * 4));
+    GAJE_HIP_CHECK(hipMemset(sb.ACT, 0, (size_t)(L * ffn) * 4));
     BatchState &st = b->st;
     st.nseq = (int32_t)n_seq;
     st.lanes = (int32_t)L;
@@ -1649,7 +1832,10 @@ extern "C" int gaje_hip_batch_open(gaje_hip_model *m, int64_t n_seq, int64_t cap
     for (void *p : {(void *)st.pos, (void *)st.cur_pos, (void *)st.halted, (void *)st.err, (void *)st.tok,
                     (void *)st.embed_ids, (void *)st.next})
         GAJE_HIP_CHECK(hipMemset(p, 0, (size_t)L * 4));
+    sb.rows = L;
+    sb.nan_codes = st.nan_codes;
     b->pos.assign((size_t)L, 0);
+    b->halted.assign((size_t)L, 0);
     m->batches.push_back(b.get());
     *out = b.release();
     return GAJE_OK;
@@ -1682,7 +1868,7 @@ extern "C" int gaje_hip_batch_reset(gaje_hip_batch *b, int64_t seq) {
             GAJE_HIP_CHECK(hipMemcpyAsync(b->st.pos + q, &zero, 4, hipMemcpyHostToDevice, b->m->stream));
             GAJE_HIP_CHECK(hipMemcpyAsync(b->st.halted + q, &zero, 4, hipMemcpyHostToDevice, b->m->stream));
             GAJE_HIP_CHECK(hipStreamSynchronize(b->m->stream));
-            b->pos[q] = 0;
+            b->pos[q] = b->halted[q] = 0;
         }
     return GAJE_OK;
 }
@@ -1708,7 +1894,13 @@ extern "C" int gaje_hip_batch_feed(gaje_hip_batch *b, const uint32_t *ids, int64
         b->ids_cap = (int64_t)need;
     }
     GAJE_HIP_CHECK(hipMemcpyAsync(b->ids, ids, need * 4, hipMemcpyHostToDevice, s));
-    for (int64_t i = 0; i < n; ++i) GAJE_TRY(batch_enqueue_step(b, b->ids, n, i, nullptr, false));
+    // the last step gives the logits; the steps before it run as rows
+    if (n > 1 && rows_supported(m)) {
+        GAJE_TRY(batch_feed_rows(b, ids, n, 0, n - 1));
+        GAJE_TRY(batch_enqueue_step(b, b->ids, n, n - 1, nullptr, false));
+    } else {
+        for (int64_t i = 0; i < n; ++i) GAJE_TRY(batch_enqueue_step(b, b->ids, n, i, nullptr, false));
+    }
     if (last_logits_host && m->kwta_ratio > 0.0f && m->kwta_ratio < 1.0f)
         for (int64_t q = 0; q < b->nseq; ++q)
             GAJE_TRY(launch_kwta(b->LOG + q * m->vocab_out, m->vocab_out, kwta_k(m->vocab_out, m->kwta_ratio), nullptr, s));

@@ -29,8 +29,9 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(PrefillRopeParams p) {
     if (p.seq_pos) {
         pos = p.seq_pos[t];
         if (pos < 0) return;
-        p.k_cache += t * p.seq_kv_stride;
-        p.v_cache += t * p.seq_kv_stride;
+        const int64_t q = p.row_seq ? p.row_seq[t] : t;
+        p.k_cache += q * p.seq_kv_stride;
+        p.v_cache += q * p.seq_kv_stride;
     }
     const float *row = p.qkv + t * p.ldq;
     const int hd = p.head_dim, half = hd >> 1;

@@ -1,0 +1,302 @@
+// Q4_0 weight rows x several activation rows, bit for bit
+// genomic_dot_product_q4_0_avx2 (genomic.rs:263-336) per (weight row,
+// activation row), on the f32 matrix cores.
+//
+// The reference's dot is eight independent FMA chains (chain l takes element
+// 8c + l of each block's chunk c, in order) and one fixed reduction.  A matrix
+// instruction with a single k step, v_mfma_f32_{16x16x1_4b,32x32x1_2b}, is one
+// fma per output, rounded once: checked against fmaf over normal, subnormal,
+// infinite, NaN and zero operands, no difference.  So one MFMA block runs one
+// chain: block b of the instruction holds chain l(b) of a 16 x 16 or 32 x 32
+// tile of (weight row, activation row) pairs, each step feeds it one
+// dequantised weight and one activation per row, and the accumulators of the
+// eight chains are reduced in the reference's order at the end.  Against one
+// chain per VALU lane this shares each dequantised weight between 16 or 32
+// activation rows (about 1.9 VALU instructions per weight, once per tile) and
+// runs the FMAs at the f32 matrix rate (122-130 TFLOP/s measured for
+// independent MFMAs, against 67 for v_fma_f32).
+#include <hip/hip_runtime.h>
+
+#include "common.h"
+#include "device_util.h"
+#include "kernels.h"
+
+namespace gaje {
+namespace {
+
+typedef float vf16 __attribute__((ext_vector_type(16)));
+typedef float vf32 __attribute__((ext_vector_type(32)));
+
+// Bytes of a stage (TM activation rows and TN packed weight rows of one group)
+// and of the workgroup's LDS: the ring, reused for the reduction.
+constexpr int rq_stage(int TM, int TN) { return TM * 512 + TN * 80; }
+constexpr int rq_lds(int TM, int TN, int S) {
+    const int ring = S * rq_stage(TM, TN), red = TM == 32 ? TN / 32 * 16384 : TN / 16 * 4096;
+    return ring > red ? ring : red;
+}
+
+__device__ __forceinline__ void row_flag(uint32_t *codes, int64_t row, int layer, int stage) {
+    if (codes && stage >= 0) atomicMin(&codes[row], (uint32_t)(layer * 8 + stage));
+}
+
+// The row epilogue for outputs n .. n+3 of activation row m, from the reduced
+// dots t: flush, sparse anchors, bias (linear/forward.rs:84-115), residual.
+__device__ __forceinline__ void rows_finish(const BatchGemvParams &p, int64_t m, int64_t n, const float (&t)[4]) {
+    if (m >= p.nv || n >= p.N) return;
+    const int cnt = (int)min((int64_t)4, p.N - n);
+    float v[4];
+    float *dst = p.y + (size_t)m * p.ldy + n;
+    const bool wide = cnt == 4 && !((uintptr_t)dst & 15);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        v[r] = flush_small(t[r]);
+        if (r >= cnt) continue;
+        if (p.a_ptr)
+            for (int64_t k = p.a_ptr[n + r]; k < p.a_ptr[n + r + 1]; ++k) {
+                const float prod = p.x[(size_t)m * p.ldx + p.a_col[k]] * half_bits(p.a_val[k]);
+                v[r] = v[r] + prod;
+            }
+        if (n + r < p.bias_len) v[r] = v[r] + p.bias[n + r];
+    }
+    if (p.mode == MODE_RESIDUAL) {
+        bool bad_a = false, bad_b = false;
+        float old[4] = {0.f, 0.f, 0.f, 0.f};
+        if (wide) {
+            const float4 o = *(const float4 *)dst;
+            old[0] = o.x, old[1] = o.y, old[2] = o.z, old[3] = o.w;
+        } else {
+            for (int r = 0; r < cnt; ++r) old[r] = dst[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (r >= cnt) continue;
+            bad_a |= isnan(v[r]);
+            v[r] = old[r] + v[r];
+            bad_b |= isnan(v[r]);
+        }
+        if (bad_a) row_flag(p.nan_codes, m, p.layer, p.st_a);
+        if (bad_b) row_flag(p.nan_codes, m, p.layer, p.st_b);
+    }
+    if (wide) {
+        *(float4 *)dst = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+        for (int r = 0; r < cnt; ++r) dst[r] = v[r];
+    }
+}
+
+// One workgroup of TN / 8 waves: TN weight rows x TM activation rows.
+//
+// TM = 32: wave 4t + j runs chains 2j and 2j + 1 of weight rows 32t .. 32t + 31
+// (32x32x1_2b, two blocks).  TM = 16: waves 2t and 2t + 1 run chains 0..3 and
+// 4..7 of weight rows 16t .. 16t + 15 (16x16x1_4b, four blocks).  Splitting a tile by chain
+// keeps a wave's serial length at K / 8 MFMAs, so that a few hundred tiles fill
+// the chip.  Lane i of a wave feeds row i % TMF of chain i / TMF as both
+// operands (weight row for A, activation row for B).
+//
+// Per packed group (128 elements) a ring of S stages in LDS holds the TM
+// activation rows (512 bytes each, 16-byte pieces XORed by row & 7 so that a
+// chain's strided reads spread over the banks) and the 32 rows' packed groups
+// as they are; all of it is copied by LDS-direct loads S - 1 groups ahead, one
+// barrier per group.  The copies are the loop's only vector memory accesses,
+// and every wave issues the same number, so the waits are exact counts.
+template <int TM, int TN, int S>
+__global__ __launch_bounds__(TN * 8) void rows_q4_kernel(BatchGemvParams p, int64_t ntiles, int64_t mtiles) {
+    constexpr int XR = TM / (TN / 8);       // activation rows a wave copies per stage
+    constexpr int XI = XR / 2;              // copies they take (two rows each)
+    constexpr int CP = XI + 1;              // + one of eight packed rows
+    static_assert(XI >= 1, "every wave copies activations");
+    constexpr int STAGE = rq_stage(TM, TN);
+    extern __shared__ __align__(16) uint8_t lds[];
+    // An XCD takes every activation tile of the weight tiles congruent to it
+    // (workgroups go to the eight XCDs in turn), so each weight row is read
+    // into one L2 once.
+    const int64_t j = blockIdx.x >> 3;
+    const int64_t nt = (j / mtiles) * 8 + (blockIdx.x & 7);
+    if (nt >= ntiles) return;  // whole workgroup
+    const int64_t n0 = nt * TN, m0 = (j % mtiles) * TM;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nb = p.nb, G = (nb + 3) >> 2;
+
+    // ---- copies: sources of this lane ----
+    const float *xb = p.x + (size_t)m0 * p.ldx;
+    const uint8_t *wb = p.w + (size_t)n0 * G * 80;
+    const int mlast = (int)min((int64_t)TM, p.nv - m0) - 1, nlast = (int)min((int64_t)TN, p.N - n0) - 1;
+    uint32_t xrow[XI];
+    int xpiece[XI];
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int r = wave * XR + 2 * i + (lane >> 5);
+        xrow[i] = (uint32_t)min(r, mlast) * (uint32_t)p.ldx * 4;
+        xpiece[i] = 4 * ((lane & 31) ^ (r & 7));
+    }
+    const int wl = min(lane, 39), wr = wave * 8 + wl / 5;
+    const uint32_t woff = (uint32_t)min(wr, nlast) * (uint32_t)G * 80 + (uint32_t)(wl % 5) * 16;
+    const uint32_t lds0 = lds_addr(lds);
+    const int K = nb * 32;
+    auto issue = [&](int g, int slot) {
+        const uint32_t base = lds0 + (uint32_t)slot * STAGE;
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            // pieces past the row's end (its last group may be partial) read the row's start; unused
+            const int k = g * 128 + xpiece[i];
+            lds_dma16_so(xb, xrow[i] + (uint32_t)(k < K ? k : 0) * 4, base + (wave * XR + 2 * i) * 512);
+        }
+        if (lane < 40) lds_dma16_so(wb, woff + (uint32_t)g * 80, base + TM * 512 + wave * 640);
+    };
+
+    // ---- operands of this lane ----
+    const int m = lane & (TM - 1);
+    const int row = (TM == 32 ? 32 * (wave >> 2) : 16 * (wave >> 1)) + m;
+    const int l = TM == 32 ? 2 * (wave & 3) + (lane >> 5) : 4 * (wave & 1) + (lane >> 4);  // chain
+    uint32_t xo[4];  // of step 4b + c in block b: + 128 b
+#pragma unroll
+    for (int c = 0; c < 4; ++c) xo[c] = m * 512 + (((2 * c + (l >> 2)) ^ (m & 7)) << 4) + 4 * (l & 3);
+    const uint32_t wo = TM * 512 + row * 80;
+
+    typename std::conditional<TM == 32, vf32, vf16>::type acc = {};
+    auto step = [&](float w, float x) {
+        if constexpr (TM == 32) acc = __builtin_amdgcn_mfma_f32_32x32x1f32(w, x, acc, 0, 0, 0);
+        else acc = __builtin_amdgcn_mfma_f32_16x16x1f32(w, x, acc, 0, 0, 0);
+    };
+
+    // operands of a group: read from its stage a group ahead of its MFMAs, so
+    // that the LDS reads and the dequantisation run under the previous group's
+    // (two operand sets, used in turn)
+    vu2 n;
+    vu4 sc;
+    float x[2][16], d[4][4];
+    auto read = [&](float (&xr)[16], int slot) {
+        const uint8_t *st = lds + slot * STAGE;
+        n = *(const vu2 *)(st + wo + 8 * l);
+        sc = *(const vu4 *)(st + wo + 64);
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) xr[4 * b + c] = *(const float *)(st + xo[c] + 128 * b);
+    };
+    auto dequant = [&]() {
+        q4_dequant_dw<0>(d[0], n.x, sc.x);
+        q4_dequant_dw<1>(d[1], n.x, sc.y);
+        q4_dequant_dw<0>(d[2], n.y, sc.z);
+        q4_dequant_dw<1>(d[3], n.y, sc.w);
+    };
+
+#pragma unroll
+    for (int s = 0; s < S; ++s) issue(min(s, G - 1), s);
+    wait_vmcnt<(S - 1) * CP>();
+    lds_barrier();
+    read(x[0], 0);
+    dequant();
+    int slot = 0;
+    // group g (whole: not the last) from set cur
+    auto group = [&](int g, float (&xc)[16], float (&xr)[16]) {
+        const int next = slot + 1 == S ? 0 : slot + 1;
+        wait_vmcnt<(S - 2) * CP>();
+        lds_barrier();  // stage g + 1 has landed for every wave, and stage g has been read
+        issue(min(g + S, G - 1), slot);
+        read(xr, next);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) step(d[i >> 2][i & 3], xc[i]);
+        dequant();
+        slot = next;
+    };
+    auto last = [&](float (&xc)[16]) {
+        const int left = nb - 4 * (G - 1);  // blocks of the last group (uniform)
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+            if (b == 0 || b < left) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) step(d[b][c], xc[4 * b + c]);
+            }
+    };
+    int g = 0;
+    for (; g + 2 < G; g += 2) {
+        group(g, x[0], x[1]);
+        group(g + 1, x[1], x[0]);
+    }
+    if (g + 1 < G) {
+        group(g, x[0], x[1]);
+        last(x[1]);
+    } else {
+        last(x[0]);
+    }
+    wait_vmcnt<0>();
+    lds_barrier();
+
+    // ---- ((a0+a4)+(a2+a6)) + ((a1+a5)+(a3+a7)), then the row epilogue ----
+    float t[4];
+    if constexpr (TM == 32) {
+        // registers 16 bk + 4 q + r: chain 2 (wave & 3) + bk, weight row 8 q + 4 (lane >> 5) + r;
+        // wave j of the four sums q = j, two q in LDS at a time
+        uint8_t *red = lds + (wave >> 2) * 16384;
+        const int jw = wave & 3;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int bk = 0; bk < 2; ++bk)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int i = 16 * bk + 8 * h + 4 * q;
+                    *(float4 *)(red + (((2 * jw + bk) * 2 + q) * 64 + lane) * 16) = make_float4(acc[i], acc[i + 1], acc[i + 2], acc[i + 3]);
+                }
+            lds_barrier();
+            if ((jw >> 1) == h) {
+                vf4 a[8];
+#pragma unroll
+                for (int c = 0; c < 8; ++c) a[c] = *(const vf4 *)(red + ((c * 2 + (jw & 1)) * 64 + lane) * 16);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    t[r] = ((a[0][r] + a[4][r]) + (a[2][r] + a[6][r])) + ((a[1][r] + a[5][r]) + (a[3][r] + a[7][r]));
+            }
+            if (h == 0) lds_barrier();
+        }
+        rows_finish(p, m0 + m, n0 + 32 * (wave >> 2) + 8 * jw + 4 * (lane >> 5), t);
+    } else {
+        // registers 4 b + r: chain 4 (wave & 1) + b, weight row 4 (lane >> 4) + r
+        uint8_t *red = lds + (wave >> 1) * 4096;
+        if (wave & 1) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                *(float4 *)(red + (b * 64 + lane) * 16) = make_float4(acc[4 * b], acc[4 * b + 1], acc[4 * b + 2], acc[4 * b + 3]);
+        }
+        lds_barrier();
+        if (wave & 1) return;
+        vf4 a[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) a[b] = *(const vf4 *)(red + (b * 64 + lane) * 16);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            t[r] = ((acc[r] + a[0][r]) + (acc[8 + r] + a[2][r])) + ((acc[4 + r] + a[1][r]) + (acc[12 + r] + a[3][r]));
+        rows_finish(p, m0 + m, n0 + 16 * (wave >> 1) + 4 * (lane >> 4), t);
+    }
+}
+
+template <int TM, int TN, int S>
+int launch_rows(const BatchGemvParams &p, hipStream_t s) {
+    const int64_t ntiles = (p.N + TN - 1) / TN, mtiles = (p.nv + TM - 1) / TM;
+    const int64_t grid = (ntiles + 7) / 8 * 8 * mtiles;
+    if (grid > INT32_MAX) return set_error(GAJE_ERR_UNSUPPORTED, "q4_0 rows: %lld tiles", (long long)grid);
+    hipLaunchKernelGGL((rows_q4_kernel<TM, TN, S>), dim3((unsigned)grid), dim3(TN * 8), rq_lds(TM, TN, S), s, p, ntiles, mtiles);
+    GAJE_HIP_CHECK(hipGetLastError());
+    return GAJE_OK;
+}
+
+}  // namespace
+
+int launch_q4_rows(const BatchGemvParams &p, hipStream_t s) {
+    if (!p.w || !p.x || !p.y || p.N <= 0 || p.nv <= 0 || p.ldx < p.K || p.ldx % 4 || p.ldy < p.N || p.nb <= 0 ||
+        (int64_t)p.nb * 32 != p.K || p.K > (1 << 20) || (((uintptr_t)p.x | (uintptr_t)p.w) & 15) ||
+        (p.mode != MODE_STORE && p.mode != MODE_RESIDUAL))
+        return set_error(GAJE_ERR_INVALID_ARG, "q4_0 rows: bad arguments");
+    // 32 x 64 tiles read an activation row's group once for 64 weight rows and
+    // a weight row's once for 32 activations (1536 x 17920 x 1536: 834 us
+    // against 999 with 16 x 32 tiles; 1536 x 1536 x 8960: 405 against 476), but
+    // need enough tiles to fill the chip: at 1064 of them (201 x 9728 x 896)
+    // 53 us against 48, at 560 (64 x 17920 x 1536) 51 against 47, and a few
+    // rows leave most of it idle (16 x 1536 x 8960: 89 against 35).
+    if (((p.nv + 31) / 32) * ((p.N + 63) / 64) >= 9 * (int64_t)device_cu_count() / 2) return launch_rows<32, 64, 2>(p, s);
+    return launch_rows<16, 32, 2>(p, s);
+}
+
+}  // namespace gaje

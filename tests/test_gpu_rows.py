@@ -1,0 +1,164 @@
+"""Bit parity of the row-parallel products and prompts with the CPU oracle.
+
+Several activation rows share one pass over the weights (q4_0_gemm, a bit-exact
+prompt, a batch's steps and prompts).  Every row must be the oracle's
+forward_core for that row alone, bit for bit: the row products run the same FMA
+chains on the f32 matrix cores, and the rest of a block is the same arithmetic.
+"""
+import struct
+
+import numpy as np
+import pytest
+
+from conftest import GNORM_MODEL, write_genomic_norm_model
+
+pytestmark = pytest.mark.gpu
+
+TINY = dict(n_embd=128, n_head=4, n_head_kv=2, n_blocks=2, ffn=256, vocab_size=1000, eps=1e-6,
+            rope_base=1e4, arch_family=1, qkv_bias=1, tied_embeddings=0)
+HD64 = dict(TINY, n_embd=256, ffn=544)
+HD128 = dict(TINY, n_embd=384, n_head=3, n_head_kv=1, ffn=512, n_blocks=1)
+NAN_TOKEN = 42
+
+
+@pytest.fixture(scope="module")
+def hip():
+    import gaje_hip
+    if gaje_hip.ops.device_count() < 1:
+        pytest.fail("no HIP device visible")
+    return gaje_hip
+
+
+@pytest.fixture(scope="module")
+def O():
+    from oracle import oracle
+    return oracle
+
+
+def _same(a, b):
+    """Equal bits, any NaN equal to any NaN."""
+    a, b = np.ascontiguousarray(a, np.float32), np.ascontiguousarray(b, np.float32)
+    nan = np.isnan(a) & np.isnan(b)
+    return a.shape == b.shape and bool(np.all((a.view(np.uint32) == b.view(np.uint32)) | nan))
+
+
+def _blocks(rng, n, k):
+    nb = k // 32
+    w = np.zeros((n, nb, 20), np.uint8)
+    s = (0.01 + 0.04 * rng.random((n, nb))).astype(np.float16)
+    w[..., 0:2] = s.view(np.uint8).reshape(n, nb, 2)
+    w[..., 2:4] = (-7.5 * s).astype(np.float16).view(np.uint8).reshape(n, nb, 2)
+    w[..., 4:] = rng.integers(0, 256, (n, nb, 16), np.uint8)
+    return w.reshape(-1)
+
+
+# rows below, at and past the 4-, 8-, 16- and 32-row tiles; last groups of 1, 2, 3 and 4
+# blocks; one weight row; a long sum; and a product large enough for the 32 x 64 tiles
+@pytest.mark.parametrize("m,n,k", [(2, 1, 32), (3, 37, 96), (4, 8, 128), (5, 200, 160), (8, 33, 576), (9, 64, 896),
+                                   (16, 65, 1536), (17, 31, 64), (31, 40, 224), (33, 129, 1152), (4, 24, 8960),
+                                   (7, 40, 5888), (64, 16, 4864), (70, 24608, 96)])
+def test_row_products_match_the_oracle(hip, O, m, n, k):
+    rng = np.random.default_rng(m * 1000003 + n * 1009 + k)
+    blocks, X = _blocks(rng, n, k), rng.standard_normal((m, k)).astype(np.float32)
+    X[m - 1, :k // 2] *= np.float32(1e-38)     # subnormal products and sums
+    if m > 2:
+        X[1, k - 1], X[2, 0] = np.inf, np.nan  # stay in their own rows
+    bias = rng.standard_normal(max(n - 3, 1)).astype(np.float32)
+    ops = hip.ops
+    Y = ops.DeviceBuffer(m * n * 4)
+    ops.q4_0_gemm(ops.q4_0_upload(blocks, n, k), ops.DeviceBuffer.from_array(X), Y, m, n, k,
+                  ops.DeviceBuffer.from_array(bias), bias.size)
+    ops.synchronize()
+    got = Y.read(np.float32, m * n).reshape(m, n)
+    L = O.GenomicLinear(blocks, b"", None, n, k, bias, 4)
+    for r in range(m):
+        assert _same(got[r], L.forward_core(X[r])), f"row {r}"
+
+
+def _write(hip, tmp_models, name, cfg):
+    if cfg is GNORM_MODEL:
+        return write_genomic_norm_model(str(tmp_models), seed=17)
+    p = tmp_models / f"rows_{name}.flat"
+    if not p.exists():
+        hip.synth.write_flat(str(p), seed=61, **cfg)
+    return str(p)
+
+
+def _with_nan_token(path, out, n_embd):
+    from oracle.flat import FlatFile
+    ff, data = FlatFile(path), bytearray(open(path, "rb").read())
+    off = ff.weights_offset + ff.tensors["token_embd"]["dna_off"] + NAN_TOKEN * n_embd * 4
+    data[off:off + 4] = struct.pack("<f", float("nan"))
+    open(out, "wb").write(bytes(data))
+    return str(out)
+
+
+def _oracle(O, path, kwta):
+    r = O.load_genomic(path)
+    r.set_k_wta_ratio(kwta)
+    r.clear_cache_core()
+    return r
+
+
+# prompts of two tokens, of a few tiles, and of more rows than one pass takes, on an
+# empty cache and after it
+@pytest.mark.parametrize("name,cfg,kwta,lengths", [("tiny", TINY, 0.0, [2, 33, 1]), ("tiny", TINY, 0.5, [19]),
+                                                   ("hd64", HD64, 0.0, [65, 3]), ("hd128", HD128, 0.0, [130]),
+                                                   ("gnorm", GNORM_MODEL, 0.0, [17]), ("tiny", TINY, 0.0, [1040])])
+def test_prompt_rows_match_the_oracle(hip, O, tmp_models, name, cfg, kwta, lengths):
+    p = _write(hip, tmp_models, name, cfg)
+    g, r = hip.load_genomic_auto(p), _oracle(O, p, kwta)
+    g.set_k_wta_ratio(kwta)
+    rng = np.random.default_rng(sum(lengths))
+    for n in lengths:
+        ids = rng.integers(0, cfg["vocab_size"], n).astype(np.uint32)
+        got = g.prefill(ids, want_logits=True)
+        for t in ids:
+            want = r.forward_core(int(t))
+        assert _same(got, want), f"prompt of {n}"
+    assert g.cache_len() == sum(lengths)
+    assert _same(g.forward(7), r.forward_core(7))
+    g.close()
+
+
+def test_prompt_rows_stop_at_a_guard(hip, O, tmp_models):
+    p = _with_nan_token(_write(hip, tmp_models, "tiny", TINY), tmp_models / "rows_nan.flat", TINY["n_embd"])
+    g, r = hip.load_genomic_auto(p), _oracle(O, p, 0.0)
+    g.set_k_wta_ratio(0.0)
+    ids = [5, 6, 7, 8, NAN_TOKEN, 9, 10]
+    with pytest.raises(ValueError, match="Input x is NaN"):
+        g.prefill(ids)
+    assert g.cache_len() == 4
+    for t in ids[:4]:
+        r.forward_core(t)
+    assert _same(g.forward(11), r.forward_core(11))
+    g.close()
+
+
+def test_batch_rows_with_gaps_and_a_guard(hip, O, tmp_models):
+    """Skipped steps inside a prompt, a sequence that never runs, and one that a
+    guard halts in the middle of its prompt while the others go on."""
+    p = _with_nan_token(_write(hip, tmp_models, "tiny", TINY), tmp_models / "rows_nan.flat", TINY["n_embd"])
+    g = hip.load_genomic_auto(p)
+    g.set_k_wta_ratio(0.0)
+    X = hip.BATCH_INACTIVE
+    for nan_at in (None, 2):
+        ids = np.array([[1, 2, X, 3, 4, 5], [9, 8, 7, 6, 5, 4], [X] * 6, [X, 11, 12, X, 13, 14]], np.uint32)
+        if nan_at is not None:
+            ids[1, nan_at] = NAN_TOKEN
+        b = hip.GenomicBatch(g, 4, 64)
+        logits, status, rc = b.feed(ids, want_logits=True, status=True)
+        assert (rc == 0) == (nan_at is None)
+        for s in (0, 1, 3):
+            r = _oracle(O, p, 0.0)
+            toks = [int(t) for t in ids[s] if t != X]
+            if s == 1 and nan_at is not None:
+                assert status[1] == 1 and b.cache_len(1) == nan_at
+                continue
+            assert status[s] == 0 and b.cache_len(s) == len(toks)
+            for t in toks:
+                want = r.forward_core(t)
+            assert _same(logits[s], want), f"sequence {s}"
+        assert b.cache_len(2) == 0
+        b.close()
+    g.close()

@@ -282,6 +282,167 @@ int launch_rows(const BatchGemvParams &p, hipStream_t s) {
     return GAJE_OK;
 }
 
+// Few tiles: v_mfma_f32_4x4x1_16b, whose step is 8 weight rows x 4 activation
+// rows x 8 chains in a wave (8 cycles, 13 when it waits for the step before it): a
+// product of few rows spreads over four times as many waves as with the
+// 16x16 form, and its serial length of K / 8 steps costs less.
+//
+// One workgroup of four waves: 32 weight rows (an octet each) x 4 activation
+// rows.  Lane i is (row quad i >> 5, chain (i >> 2) & 7, i & 3): A is weight row
+// 4 (i >> 5) + (i & 3) of the octet and B activation row i & 3, both of that chain;
+// register r is weight row r of the quad against activation row i & 3.
+//
+// A wave pays for everything beside its MFMAs in issue slots between them (an f32
+// MFMA and its own wave's VALU do not overlap): about two VALU instructions of
+// dequantisation a step, the loads, and the activations' way into LDS.  Measured
+// on 16 x 1536 x 8960 by leaving parts out: 21.0 us in all, 11.8 without
+// dequantisation, loads and staging; the rest splits evenly between the three.
+// So the weights go straight into a register ring of R4_D groups, loads are a
+// uniform offset that advances and a lane's constant one, and the activations are
+// transposed into one row of steps per (chain, activation row), so that a lane
+// reads four steps with one conflict-free 16-byte read.  Their ring holds three
+// chunks of R4_CG groups: written two chunks ahead of their use, loaded two before
+// that, and read a group ahead of the MFMAs across the chunk's barrier.
+// (Operands dequantised and transposed into LDS by other waves: 22.9 us, bound by
+// the LDS port.)
+constexpr int R4_CG = 4, R4_D = 2 * R4_CG;
+constexpr int R4_ROW = 16 * R4_CG + 4;   // floats of a (chain, row): rows 4 banks apart
+constexpr int R4_CHAIN = 4 * R4_ROW, R4_BUF = 8 * R4_CHAIN;
+constexpr int R4_XT = R4_CG / 2;         // activation quads of a thread and chunk
+
+__device__ __forceinline__ auto tile_buffer(const void *p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, 0x7FFFFFFF, 0x00027000);
+}
+
+__global__ __launch_bounds__(256) void rows4_q4_kernel(BatchGemvParams p, int64_t ntiles, int64_t mtiles) {
+    __shared__ __align__(16) float lds[3 * R4_BUF];
+    const int64_t j = blockIdx.x >> 3;  // (XCD order as above)
+    const int64_t nt = (j / mtiles) * 8 + (blockIdx.x & 7);
+    if (nt >= ntiles) return;  // whole workgroup
+    const int64_t n0 = nt * 32, m0 = (j % mtiles) * 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nb = p.nb, G = (nb + 3) >> 2, K = nb * 32;
+    const int m = lane & 3, l = (lane >> 2) & 7, row = 8 * wave + 4 * (lane >> 5) + m;
+
+    // ---- weights: 8 code bytes of this lane's chain and the 16 scale bytes, per group ----
+    const auto wbuf = tile_buffer(p.w + (size_t)n0 * G * 80);
+    const uint32_t wscale = (uint32_t)min((int64_t)row, p.N - 1 - n0) * (uint32_t)G * 80 + 64, wcode = wscale - 64 + 8 * l;
+    vu2 wn[R4_D];
+    vu4 ws[R4_D];
+    auto load_w = [&](int i, int g) {  // past the row's end its last group is read again
+        const int at = min(g, G - 1) * 80;
+        wn[i] = __builtin_bit_cast(vu2, __builtin_amdgcn_raw_buffer_load_b64(wbuf, wcode, at, 0));
+        ws[i] = __builtin_bit_cast(vu4, __builtin_amdgcn_raw_buffer_load_b128(wbuf, wscale, at, 0));
+    };
+    // ---- activations ----
+    const auto xbuf = tile_buffer(p.x + (size_t)m0 * p.ldx);
+    uint32_t xsrc[R4_XT];
+    float *xdst[R4_XT];
+#pragma unroll
+    for (int i = 0; i < R4_XT; ++i) {
+        // elements k .. k+3 of a row's chunk: chains 4 (k / 4 % 2) .. + 3, step k / 8
+        const int u = tid + 256 * i, r = u / (32 * R4_CG), q = u % (32 * R4_CG);
+        xsrc[i] = ((uint32_t)min((int64_t)r, p.nv - 1 - m0) * (uint32_t)p.ldx + 4 * q) * 4;
+        xdst[i] = lds + 4 * (q & 1) * R4_CHAIN + r * R4_ROW + (q >> 1);
+    }
+    auto xk = [&](int i, int c) { return c * 128 * R4_CG + 4 * ((tid + 256 * i) % (32 * R4_CG)); };
+    const int whole = K / (128 * R4_CG);  // chunks that lie inside the row
+    vf4 xq[2][R4_XT];
+    auto load_x = [&](vf4 (&x)[R4_XT], int c) {  // past the row's end its start is read, and stored as zeros
+        const int at = c * 512 * R4_CG;
+#pragma unroll
+        for (int i = 0; i < R4_XT; ++i)
+            x[i] = c < whole ? __builtin_bit_cast(vf4, __builtin_amdgcn_raw_buffer_load_b128(xbuf, xsrc[i], at, 0))
+                             : __builtin_bit_cast(vf4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                           xbuf, xk(i, c) < K ? xsrc[i] + at : xsrc[i] - xk(i, 0) * 4, 0, 0));
+    };
+    auto store_x = [&](const vf4 (&x)[R4_XT], int c, int buf) {
+        if (c < whole) {
+#pragma unroll
+            for (int i = 0; i < R4_XT; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) xdst[i][buf * R4_BUF + e * R4_CHAIN] = x[i][e];
+        } else {
+#pragma unroll
+            for (int i = 0; i < R4_XT; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) xdst[i][buf * R4_BUF + e * R4_CHAIN] = xk(i, c) < K ? x[i][e] : 0.0f;
+        }
+    };
+    const float *xl = lds + l * R4_CHAIN + m * R4_ROW;
+    vf4 x[2][4];
+    auto read_x = [&](vf4 (&xr)[4], int buf, int g) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) xr[b] = *(const vf4 *)(xl + buf * R4_BUF + 16 * g + 4 * b);
+    };
+
+    load_x(xq[0], 0);
+    load_x(xq[1], 1);
+#pragma unroll
+    for (int i = 0; i < R4_D; ++i) load_w(i, i);
+    store_x(xq[0], 0, 0);
+    store_x(xq[1], 1, 1);
+    load_x(xq[0], 2);
+    load_x(xq[1], 3);
+    lds_barrier();
+    read_x(x[0], 0, 0);
+    vf4 acc = {0.f, 0.f, 0.f, 0.f};
+    int buf = 0;
+    // R4_D groups (`all`: every one exists, else the row ends among them).  The
+    // blocks that the row's last group lacks are zero weights against zero
+    // activations, and fma(0, 0, acc) = acc (never -0).
+    auto round = [&](int g0, auto all) {
+#pragma unroll
+        for (int u = 0; u < R4_D; ++u) {
+            if (!decltype(all)::value && g0 + u >= G) continue;  // (uniform)
+            const int next = buf == 2 ? 0 : buf + 1;
+            if (u % R4_CG == 0) {
+                const int c = (g0 + u) / R4_CG, nn = next == 2 ? 0 : next + 1;
+                store_x(xq[u / R4_CG], c + 2, nn);
+                load_x(xq[u / R4_CG], c + 4);
+            }
+            vf4(&xc)[4] = x[u & 1];
+            if (u % R4_CG != R4_CG - 1) read_x(x[(u + 1) & 1], buf, u % R4_CG + 1);
+            else read_x(x[(u + 1) & 1], next, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            float d[4][4];
+            q4_dequant_dw<0>(d[0], wn[u].x, ws[u].x);
+            q4_dequant_dw<1>(d[1], wn[u].x, ws[u].y);
+            q4_dequant_dw<0>(d[2], wn[u].y, ws[u].z);
+            q4_dequant_dw<1>(d[3], wn[u].y, ws[u].w);
+            if (decltype(all)::value) load_w(u, g0 + u + R4_D);
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                acc = __builtin_amdgcn_mfma_f32_4x4x1f32(d[e >> 2][e & 3], xc[e >> 2][e & 3], acc, 0, 0, 0);
+            if (u % R4_CG == R4_CG - 1) {
+                buf = next;
+                lds_barrier();
+            }
+        }
+    };
+    int g0 = 0;
+    for (; g0 + R4_D <= G; g0 += R4_D) round(g0, std::true_type{});
+    if (g0 < G) round(g0, std::false_type{});
+
+    // ((a0+a4)+(a2+a6)) + ((a1+a5)+(a3+a7)): the chains are lane bits 2..4
+    float t[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        float v = acc[r];
+        v = v + __shfl_xor(v, 16, WAVE);
+        v = v + __shfl_xor(v, 8, WAVE);
+        t[r] = v + __shfl_xor(v, 4, WAVE);
+    }
+    if (l == 0) rows_finish(p, m0 + m, n0 + 8 * wave + 4 * (lane >> 5), t);
+}
+
+int launch_rows4(const BatchGemvParams &p, hipStream_t s) {
+    const int64_t ntiles = (p.N + 31) / 32, mtiles = (p.nv + 3) / 4;
+    hipLaunchKernelGGL(rows4_q4_kernel, dim3((unsigned)((ntiles + 7) / 8 * 8 * mtiles)), dim3(256), 0, s, p, ntiles, mtiles);
+    GAJE_HIP_CHECK(hipGetLastError());
+    return GAJE_OK;
+}
+
 }  // namespace
 
 int launch_q4_rows(const BatchGemvParams &p, hipStream_t s) {
@@ -289,12 +450,17 @@ int launch_q4_rows(const BatchGemvParams &p, hipStream_t s) {
         (int64_t)p.nb * 32 != p.K || p.K > (1 << 20) || (((uintptr_t)p.x | (uintptr_t)p.w) & 15) ||
         (p.mode != MODE_STORE && p.mode != MODE_RESIDUAL))
         return set_error(GAJE_ERR_INVALID_ARG, "q4_0 rows: bad arguments");
+    // 4-row tiles while they are few enough to run at once, about two and a half
+    // workgroups per CU: 8.6 -> 6.9 us for 16 x 2048 x 1536, 35.4 -> 21.0 for 16 x 1536
+    // x 8960, 17.7 -> 12.8 for 4 x 17920 x 1536 (560 workgroups); past that the
+    // larger tiles' reuse wins (768 workgroups, 64 x 1536 x 8960: 47 against 37 us;
+    // 1216, 16 x 9728 x 896: 12.8 against 8.9).
+    if (((p.nv + 3) / 4) * ((p.N + 31) / 32) <= 5 * (int64_t)device_cu_count() / 2) return launch_rows4(p, s);
     // 32 x 64 tiles read an activation row's group once for 64 weight rows and
     // a weight row's once for 32 activations (1536 x 17920 x 1536: 834 us
     // against 999 with 16 x 32 tiles; 1536 x 1536 x 8960: 405 against 476), but
     // need enough tiles to fill the chip: at 1064 of them (201 x 9728 x 896)
-    // 53 us against 48, at 560 (64 x 17920 x 1536) 51 against 47, and a few
-    // rows leave most of it idle (16 x 1536 x 8960: 89 against 35).
+    // 53 us against 48, at 560 (64 x 17920 x 1536) 51 against 47.
     if (((p.nv + 31) / 32) * ((p.N + 63) / 64) >= 9 * (int64_t)device_cu_count() / 2) return launch_rows<32, 64, 2>(p, s);
     return launch_rows<16, 32, 2>(p, s);
 }

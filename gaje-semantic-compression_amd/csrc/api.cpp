@@ -345,8 +345,7 @@ extern "C" int gaje_hip_q4_0_gemm_mfma(const void *packed, const float *X, const
     sp.sl = w.sl;
     sp.ldsum = w.ldsum;
     GAJE_TRY(launch_split_rows(sp, s));
-    GAJE_TRY(launch_q4_mins((const uint8_t *)packed, n, k, w.mins, w.ldsum, s));
-    GAJE_TRY(launch_q4_frags((const uint8_t *)packed, n, k, w.wf, w.wsc, s));
+    GAJE_TRY(launch_q4_operands((const uint8_t *)packed, n, k, w.wf, w.wsc, w.mins, w.ldsum, s));
     GemmBsParams p{};
     p.wf = w.wf;
     p.wsc = w.wsc;
@@ -673,8 +672,8 @@ extern "C" int gaje_hip_moe_prepare(const void *const *gate_up, const void *cons
     for (int i = 0; i < 2; ++i)
         for (int64_t e = 0; e < n_expert; ++e) {
             const uint8_t *pk = (const uint8_t *)(i == 0 ? gate_up[e] : down[e]);
-            GAJE_TRY(launch_q4_frags(pk, NN[i], KK[i], w.wf[i] + e * w.wf_stride[i], w.wsc[i] + e * w.wsc_stride[i], s));
-            GAJE_TRY(launch_q4_mins(pk, NN[i], KK[i], w.mins[i] + e * w.mins_stride[i], w.ldm[i], s));
+            GAJE_TRY(launch_q4_operands(pk, NN[i], KK[i], w.wf[i] + e * w.wf_stride[i], w.wsc[i] + e * w.wsc_stride[i],
+                                        w.mins[i] + e * w.mins_stride[i], w.ldm[i], s));
         }
     return GAJE_OK;
 }

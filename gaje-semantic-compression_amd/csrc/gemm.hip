@@ -40,7 +40,7 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-enum SplitPrologue { SPLIT_PLAIN = 0, SPLIT_NORM = 1, SPLIT_SWIGLU = 2 };
+enum SplitPrologue { SPLIT_PLAIN = 0, SPLIT_NORM = 1, SPLIT_SWIGLU = 2, SPLIT_ATTN = 3 };
 
 // swiglu_balanced (activation.rs:40-49: the gate clamped to [-64, 64], the
 // sigmoid from exp(-|g|), silu(g) * u) for the MFMA paths, which are held to
@@ -105,8 +105,10 @@ __global__ __launch_bounds__(256) void q4_row_exp_kernel(const uint8_t *w, int64
 // trees (the lanes' partials, then the waves') rather than in the chain order.
 // Latency-bound: every input load of a thread is issued at once, the row's
 // values stay in registers (NTH threads x IT float4s), and the pass has three
-// barriers.
-template <int PRO, int NTH, int IT>
+// barriers.  The prologues are template arguments because their registers add up:
+// with the attention merge (8 chunk records per float4) and the split-K reduce
+// (PART) compiled into the plain pass it spilled (K = 8960, 77 rows: 53.5 us).
+template <int PRO, bool PART, int NTH, int IT>
 __global__ __launch_bounds__(NTH) void split_rows_kernel(SplitParams p) {
     constexpr int NWV = NTH / 64;
     extern __shared__ __align__(16) float xs[];
@@ -124,31 +126,29 @@ __global__ __launch_bounds__(NTH) void split_rows_kernel(SplitParams p) {
     // attention-merge prologue: the row's float4 i lies in head 4 i / hd; the
     // records of its key chunks c < nc (clamped reads)
     constexpr int NCH = PREFILL_ATTN_CHUNKS;
-    float am[PRO == SPLIT_PLAIN ? IT : 1][NCH], al[PRO == SPLIT_PLAIN ? IT : 1][NCH];
-    float4 ao[PRO == SPLIT_PLAIN ? IT : 1][NCH];
-    const int anc = p.attn_ws ? (int)((p.attn_pos0 + m) / p.attn_kch) + 1 : 0;
+    float am[PRO == SPLIT_ATTN ? IT : 1][NCH], al[PRO == SPLIT_ATTN ? IT : 1][NCH];
+    float4 ao[PRO == SPLIT_ATTN ? IT : 1][NCH];
+    const int anc = PRO == SPLIT_ATTN ? (int)((p.attn_pos0 + m) / p.attn_kch) + 1 : 0;
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
         const int64_t i = tid + (int64_t)NTH * it;
         if (i < K4) {
-            if constexpr (PRO == SPLIT_PLAIN) {
-                if (p.attn_ws) {
-                    const int64_t h = 4 * i / p.attn_hd, d = 4 * i - h * p.attn_hd;
-                    const int64_t rs = (int64_t)p.attn_hd + PREFILL_ATTN_REC_PAD;
+            if constexpr (PRO == SPLIT_ATTN) {
+                const int64_t h = 4 * i / p.attn_hd, d = 4 * i - h * p.attn_hd;
+                const int64_t rs = (int64_t)p.attn_hd + PREFILL_ATTN_REC_PAD;
 #pragma unroll
-                    for (int c = 0; c < NCH; ++c) {
-                        const float *rc = p.attn_ws + (((int64_t)min(c, anc - 1) * p.M + m) * p.attn_heads + h) * rs;
-                        am[it][c] = rc[0];
-                        al[it][c] = rc[1];
-                        ao[it][c] = *(const float4 *)(rc + PREFILL_ATTN_REC_PAD + d);
-                    }
-                    continue;
+                for (int c = 0; c < NCH; ++c) {
+                    const float *rc = p.attn_ws + (((int64_t)min(c, anc - 1) * p.M + m) * p.attn_heads + h) * rs;
+                    am[it][c] = rc[0];
+                    al[it][c] = rc[1];
+                    ao[it][c] = *(const float4 *)(rc + PREFILL_ATTN_REC_PAD + d);
                 }
+                continue;
             }
             if constexpr (PRO == SPLIT_SWIGLU) {
                 g4[it] = *(const float4 *)(xr + 4 * i);
                 u4[it] = *(const float4 *)(p.up + src_row * p.ldx + 4 * i);
-            } else if (p.part) {
+            } else if constexpr (PART) {
                 pv[it] = *(const float4 *)(p.part + m * p.K + 4 * i);
                 if (4 * i + 4 <= p.bias_len) {
                     b4[it] = *(const float4 *)(p.bias + 4 * i);
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(NTH) void split_rows_kernel(SplitParams p) {
             o.w = swiglu_fast(g.w, u.w);
             bad |= (isnan(o.x) | isnan(o.y) | isnan(o.z) | isnan(o.w)) << 1;
             v[it] = o;
-        } else if (p.part) {
+        } else if constexpr (PART) {
             // the deferred split-K reduce, in gemm_reduce_kernel's order: the
             // partials in split order (eight in flight, clamped reads), flush,
             // bias, residual
@@ -213,30 +213,28 @@ __global__ __launch_bounds__(NTH) void split_rows_kernel(SplitParams p) {
             v[it] = make_float4(a[0], a[1], a[2], a[3]);
             *(float4 *)(const_cast<float *>(p.x) + m * p.ldx + 4 * i) = v[it];  // x is the product's output here
             bad |= isnan(a[0]) | isnan(a[1]) | isnan(a[2]) | isnan(a[3]);
-        } else if (PRO == SPLIT_PLAIN && p.attn_ws) {
+        } else if constexpr (PRO == SPLIT_ATTN) {
             // out = (sum_c O_c 2^(m_c - m)) / (sum_c l_c 2^(m_c - m) + 1e-12), m =
             // max_c m_c, as prefill_attn_merge_kernel (the maxima in log2 units)
-            if constexpr (PRO == SPLIT_PLAIN) {
-                float mx = -INFINITY;
+            float mx = -INFINITY;
 #pragma unroll
-                for (int c = 0; c < NCH; ++c)
-                    if (c < anc) mx = fmaxf(mx, am[it][c]);
-                float l = 0.0f;
-                float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int c = 0; c < NCH; ++c)
+                if (c < anc) mx = fmaxf(mx, am[it][c]);
+            float l = 0.0f;
+            float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-                for (int c = 0; c < NCH; ++c)
-                    if (c < anc) {
-                        const float e = exp2f(am[it][c] - mx);
-                        l = l + al[it][c] * e;
-                        o.x = o.x + ao[it][c].x * e;
-                        o.y = o.y + ao[it][c].y * e;
-                        o.z = o.z + ao[it][c].z * e;
-                        o.w = o.w + ao[it][c].w * e;
-                    }
-                const float r = 1.0f / (l + 1e-12f);
-                v[it] = make_float4(o.x * r, o.y * r, o.z * r, o.w * r);
-                bad |= isnan(v[it].x) | isnan(v[it].y) | isnan(v[it].z) | isnan(v[it].w);
-            }
+            for (int c = 0; c < NCH; ++c)
+                if (c < anc) {
+                    const float e = exp2f(am[it][c] - mx);
+                    l = l + al[it][c] * e;
+                    o.x = o.x + ao[it][c].x * e;
+                    o.y = o.y + ao[it][c].y * e;
+                    o.z = o.z + ao[it][c].z * e;
+                    o.w = o.w + ao[it][c].w * e;
+                }
+            const float r = 1.0f / (l + 1e-12f);
+            v[it] = make_float4(o.x * r, o.y * r, o.z * r, o.w * r);
+            bad |= isnan(v[it].x) | isnan(v[it].y) | isnan(v[it].z) | isnan(v[it].w);
         } else {
             v[it] = g4[it];
             bad |= isnan(v[it].x) | isnan(v[it].y) | isnan(v[it].z) | isnan(v[it].w);
@@ -305,12 +303,12 @@ __global__ __launch_bounds__(NTH) void split_rows_kernel(SplitParams p) {
         int b = 0;
 #pragma unroll
         for (int w = 0; w < NWV; ++w) b |= badw[w];
-        if (p.part) {
+        if constexpr (PART) {
             if (b & 4) nan_flag(p.st, p.y_layer, p.st_ya);
             if (b & 8) nan_flag(p.st, p.y_layer, p.st_yb);
         }
         if (b & 1) nan_flag(p.st, p.layer, p.st_a);
-        if ((b & 2) && PRO != SPLIT_PLAIN) nan_flag(p.st, p.layer, p.st_b);
+        if (b & 2) nan_flag(p.st, p.layer, p.st_b);
     }
     if (p.sh) {
         // block-scaled layout: one plane, block b at halves 64 b.. holding its
@@ -653,7 +651,7 @@ size_t gemm_lds() { return (size_t)((GA ? 0 : 4 * MT * GM_ROW) + 4 * GM_NT * GM_
 // 2 kg + 8 (t & 3) + (t >> 2), so the 8 halves of MFMA lane group kg are the
 // 8 codes of that word pair.  A code byte becomes f16 1024 + q by v_perm
 // against 0x64 bytes, then q by a packed f16 subtraction.  This expansion runs
-// once per weight matrix (q4_frag_kernel): the products read the codes as f16
+// once per weight matrix (q4_operands_kernel): the products read the codes as f16
 // fragments, [16-row tile][block][64 lanes][8 halves] (1 KiB per tile and
 // block, in the MFMA's lane order), and the scales as fp32 [tile][block][16],
 // both zero past the last row and block: four times the packed bytes, traded
@@ -1059,51 +1057,49 @@ __global__ __launch_bounds__(64 * W, (BsShape<W, BPI, R, NB>::WG_PER_CU)) void g
     }
 }
 
-// mins[n][b] = the f16 min of block b of row n (the high half of word b % 4
-// of the group's scale words, at byte 64 of its 80), 0 for b >= nb.
-__global__ __launch_bounds__(256) void q4_mins_kernel(const uint8_t *w, int64_t N, int nb, uint16_t *mins, int64_t ldm) {
-    const int64_t G = (nb + 3) / 4, total = N * ldm;
-    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {
-        const int64_t n = e / ldm;
-        const int b = (int)(e - n * ldm);
-        uint16_t v = 0;
-        if (b < nb) v = (uint16_t)(*(const uint32_t *)(w + (n * G + (b >> 2)) * 80 + 64 + 4 * (b & 3)) >> 16);
-        mins[e] = v;
-    }
-}
-
 // The product's weight operands from packed Q4_0 rows: per 16-row tile and
 // block, the MFMA fragment of its codes as f16 (lane (fr, kg) holds the codes
 // of row 16 tile + fr, block b, elements 2 kg + 8 (t & 3) + (t >> 2), t =
-// 0..7, the activation plane's order), and the 16 rows' scales as fp32; zero
-// past row N and block nb.  One wave per (tile, block).
-__global__ __launch_bounds__(256) void q4_frag_kernel(const uint8_t *w, int64_t N, int nb, int64_t nbp4, uint16_t *wf,
-                                                      float *wsc) {
+// 0..7, the activation plane's order), and the 16 rows' scales as fp32, both
+// zero past row N and block nb (blocks padded to a multiple of 4, nbp4); and
+// mins[n][b], the blocks' f16 mins, zero up to column ldm.  One wave per (tile,
+// group of four blocks): it reads the group once for its four fragments, scales
+// and mins.  Bound by writing the fragments, two bytes per weight (17920 x 1536:
+// 16.9 us with one wave per block, each reading the whole group, plus 5.3 for the
+// mins in a launch of their own).
+__global__ __launch_bounds__(256) void q4_operands_kernel(const uint8_t *w, int64_t N, int nb, int64_t nbp4, uint16_t *wf,
+                                                          float *wsc, uint16_t *mins, int64_t ldm) {
     const int lane = threadIdx.x & 63, fr = lane & 15, kg = lane >> 4;
-    const int64_t T = (N + 15) / 16, G = (nb + 3) / 4;
+    const int64_t T = (N + 15) / 16, G = (nb + 3) / 4, GM = ldm / 4;  // GM >= G groups of mins
     const int64_t chunk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (chunk >= T * nbp4) return;
-    const int64_t tile = chunk / nbp4;
-    const int b = (int)(chunk - tile * nbp4);
+    if (chunk >= T * GM) return;
+    const int64_t tile = chunk / GM, g = chunk - tile * GM;
     const int64_t n = 16 * tile + fr;
-    vu4 f = {0u, 0u, 0u, 0u};
-    float scale = 0.0f;
-    if (n < N && b < nb) {
-        const uint8_t *grp = w + (n * G + (b >> 2)) * 80;
-        const vu4 q = *(const vu4 *)(grp + 16 * kg);
-        const int u = b & 3;
+    vu4 q = {0u, 0u, 0u, 0u}, sm = {0u, 0u, 0u, 0u};
+    if (n < N && g < G) {
+        const uint8_t *grp = w + (n * G + g) * 80;
+        q = *(const vu4 *)(grp + 16 * kg);
+        sm = *(const vu4 *)(grp + 64);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (4 * g + u >= nb) sm[u] = 0u;
+    }
+    if (kg == 0 && n < N)
+        *(vu2 *)(mins + n * ldm + 4 * g) = (vu2){(sm[0] >> 16) | (sm[1] & 0xFFFF0000u), (sm[2] >> 16) | (sm[3] & 0xFFFF0000u)};
+    if (g >= G) return;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
         uint32_t wa = u & 2 ? q[1] : q[0], wb = u & 2 ? q[3] : q[2];
         if (u & 1) {
             wa >>= 4;
             wb >>= 4;
         }
-        wa &= 0x0F0F0F0Fu;
-        wb &= 0x0F0F0F0Fu;
-        f = (vu4){code_pair<0>(wa), code_pair<1>(wa), code_pair<0>(wb), code_pair<1>(wb)};
-        scale = half_lo(*(const uint32_t *)(grp + 64 + 4 * u));
+        wa = 4 * g + u < nb ? wa & 0x0F0F0F0Fu : 0u;
+        wb = 4 * g + u < nb ? wb & 0x0F0F0F0Fu : 0u;
+        const int64_t c = tile * nbp4 + 4 * g + u;
+        *(vu4 *)(wf + c * 512 + lane * 8) = (vu4){code_pair<0>(wa), code_pair<1>(wa), code_pair<0>(wb), code_pair<1>(wb)};
+        if (kg == 0) wsc[c * 16 + fr] = half_lo(sm[u]);
     }
-    *(vu4 *)(wf + chunk * 512 + lane * 8) = f;
-    if (kg == 0) wsc[chunk * 16 + fr] = scale;
 }
 
 }  // namespace
@@ -1112,13 +1108,14 @@ int64_t q4_frag_nbp4(int64_t K) { return (K / 32 + 3) / 4 * 4; }
 int64_t q4_frag_halves(int64_t N, int64_t K) { return (N + 15) / 16 * q4_frag_nbp4(K) * 512; }
 int64_t q4_frag_scale_floats(int64_t N, int64_t K) { return (N + 15) / 16 * q4_frag_nbp4(K) * 16; }
 
-int launch_q4_frags(const uint8_t *packed, int64_t N, int64_t K, uint16_t *wf, float *wsc, hipStream_t s) {
-    if (!packed || !wf || !wsc || N <= 0 || K <= 0 || K % 32)
-        return set_error(GAJE_ERR_INVALID_ARG, "q4 fragments: bad arguments");
-    const int64_t chunks = (N + 15) / 16 * q4_frag_nbp4(K);
-    if ((chunks + 3) / 4 > 0x7fffffff) return set_error(GAJE_ERR_UNSUPPORTED, "q4 fragments: too many");
-    hipLaunchKernelGGL(q4_frag_kernel, dim3((unsigned)((chunks + 3) / 4)), dim3(256), 0, s, packed, N, (int)(K / 32),
-                       q4_frag_nbp4(K), wf, wsc);
+int launch_q4_operands(const uint8_t *packed, int64_t N, int64_t K, uint16_t *wf, float *wsc, uint16_t *mins, int64_t ldm,
+                       hipStream_t s) {
+    if (!packed || !wf || !wsc || !mins || N <= 0 || K <= 0 || K % 32 || ldm < gemm_bs_sum_cols(K) || ldm % 4)
+        return set_error(GAJE_ERR_INVALID_ARG, "q4 operands: bad arguments");
+    const int64_t chunks = (N + 15) / 16 * (ldm / 4);
+    if ((chunks + 3) / 4 > 0x7fffffff) return set_error(GAJE_ERR_UNSUPPORTED, "q4 operands: too many");
+    hipLaunchKernelGGL(q4_operands_kernel, dim3((unsigned)((chunks + 3) / 4)), dim3(256), 0, s, packed, N, (int)(K / 32),
+                       q4_frag_nbp4(K), wf, wsc, mins, ldm);
     GAJE_HIP_CHECK(hipGetLastError());
     return GAJE_OK;
 }
@@ -1167,16 +1164,24 @@ int launch_split_rows(const SplitParams &p, hipStream_t s) {
     // threads x float4s per thread covering the row: 256 x 2, 256 x 4, 1024 x 4, 1024 x 10
     const int64_t K4 = p.K / 4;
     const dim3 grid((unsigned)p.M);
-    auto go = [&](auto pro) {
+    auto go = [&](auto pro, auto part) {
         constexpr int PRO = decltype(pro)::value;
-        if (K4 <= 512) split_rows_kernel<PRO, 256, 2><<<grid, dim3(256), lds, s>>>(p);
-        else if (K4 <= 1024) split_rows_kernel<PRO, 256, 4><<<grid, dim3(256), lds, s>>>(p);
-        else if (K4 <= 4096) split_rows_kernel<PRO, 1024, 4><<<grid, dim3(1024), lds, s>>>(p);
-        else split_rows_kernel<PRO, 1024, 10><<<grid, dim3(1024), lds, s>>>(p);
+        constexpr bool PART = decltype(part)::value;
+        if (K4 <= 512) split_rows_kernel<PRO, PART, 256, 2><<<grid, dim3(256), lds, s>>>(p);
+        else if (K4 <= 1024) split_rows_kernel<PRO, PART, 256, 4><<<grid, dim3(256), lds, s>>>(p);
+        else if (K4 <= 4096) split_rows_kernel<PRO, PART, 1024, 4><<<grid, dim3(1024), lds, s>>>(p);
+        else split_rows_kernel<PRO, PART, 1024, 10><<<grid, dim3(1024), lds, s>>>(p);
     };
-    if (p.up) go(std::integral_constant<int, SPLIT_SWIGLU>{});
-    else if (p.norm_w) go(std::integral_constant<int, SPLIT_NORM>{});
-    else go(std::integral_constant<int, SPLIT_PLAIN>{});
+    const std::true_type yes{};
+    const std::false_type no{};
+    const std::integral_constant<int, SPLIT_PLAIN> plain{};
+    const std::integral_constant<int, SPLIT_NORM> norm{};
+    if (p.up) go(std::integral_constant<int, SPLIT_SWIGLU>{}, no);
+    else if (p.attn_ws) go(std::integral_constant<int, SPLIT_ATTN>{}, no);
+    else if (p.norm_w && p.part) go(norm, yes);
+    else if (p.norm_w) go(norm, no);
+    else if (p.part) go(plain, yes);
+    else go(plain, no);
     GAJE_HIP_CHECK(hipGetLastError());
     return GAJE_OK;
 }
@@ -1226,16 +1231,6 @@ GemmPlan plan_gemm_q4_grouped(int64_t R, int64_t E, int64_t N, int64_t K) {
 
 int64_t gemm_bs_sum_cols(int64_t K) { return (K / 32 + 31) / 32 * 32; }
 
-int launch_q4_mins(const uint8_t *packed, int64_t N, int64_t K, uint16_t *mins, int64_t ldm, hipStream_t s) {
-    if (!packed || !mins || N <= 0 || K <= 0 || K % 32 || ldm < gemm_bs_sum_cols(K) || N * ldm >= ((int64_t)1 << 40))
-        return set_error(GAJE_ERR_INVALID_ARG, "q4 block mins: bad arguments");
-    const int64_t total = N * ldm;
-    int64_t g = (total + 255) / 256;
-    if (g > 65536) g = 65536;
-    hipLaunchKernelGGL(q4_mins_kernel, dim3((unsigned)g), dim3(256), 0, s, packed, N, (int)(K / 32), mins, ldm);
-    GAJE_HIP_CHECK(hipGetLastError());
-    return GAJE_OK;
-}
 int64_t gemm_bs_plane_rows(int64_t M) { return (M + 255) / 256 * 256; }
 
 GemmBsPlan plan_gemm_q4_bs(int64_t M, int64_t N, int64_t K) {

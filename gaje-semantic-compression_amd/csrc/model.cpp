@@ -61,7 +61,7 @@ struct DevLinear {
     int64_t bytes = 0;
     uint16_t *mins = nullptr;  // FMT_Q4_0: the block mins [N][ldm] the MFMA prefill's products read
     int64_t ldm = 0;
-    uint16_t *wf = nullptr;    // and their code fragments and scales (launch_q4_frags)
+    uint16_t *wf = nullptr;    // and their code fragments and scales (launch_q4_operands)
     float *wsc = nullptr;
 };
 
@@ -1533,10 +1533,9 @@ extern "C" int gaje_hip_prefill_mfma(gaje_hip_model *m, const uint32_t *ids, int
             for (DevLinear *D : {&Ly.qkv, &Ly.o, &Ly.gate_up, &Ly.down}) {
                 D->ldm = gemm_bs_sum_cols(D->K);
                 GAJE_TRY(m->alloc(&D->mins, (size_t)(D->N * D->ldm)));
-                GAJE_TRY(launch_q4_mins(D->w, D->N, D->K, D->mins, D->ldm, s));
                 GAJE_TRY(m->alloc(&D->wf, (size_t)q4_frag_halves(D->N, D->K)));
                 GAJE_TRY(m->alloc(&D->wsc, (size_t)q4_frag_scale_floats(D->N, D->K)));
-                GAJE_TRY(launch_q4_frags(D->w, D->N, D->K, D->wf, D->wsc, s));
+                GAJE_TRY(launch_q4_operands(D->w, D->N, D->K, D->wf, D->wsc, D->mins, D->ldm, s));
             }
     }
     if (m->n_layers > 0 && m->pf.kv16_keys < pos0 + n) {

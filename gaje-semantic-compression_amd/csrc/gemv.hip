@@ -2495,6 +2495,151 @@ __global__ __launch_bounds__(THREADS) void gemv_q4_chain_kernel(GemvParams p, in
     }
 }
 
+// ------------------------------------- Q4_0, a row's chains as batons ----
+// Long rows in a number that leaves most SIMDs idle with one lane per chain: L lanes
+// per chain, so a wave takes 8 / L rows (L = 8: one, L = 4: two) and a workgroup's
+// four waves share the activations.  A chain's steps are cut into phases of 32 (two
+// packed groups), and in tile t (L phases) lane L r + j holds the 32 dequantised
+// weights and activations of phase L t + j of chain (r - t) mod (64 / L) in
+// registers (chain 8 q + l: chain l of the wave's row q).  At phase p every lane
+// runs 32 dependent fmas on its own values, the first taking its sum from the lane
+// before (DPP wave_ror:1), so chain c's running sum travels through lanes L c + p
+// (mod 64) in step order and the sums of the other lanes are discarded: the chain
+// is the reference's, fma by fma, but its L lanes share the dequantisation and the
+// operand reads, 2.4 instructions per step when one lane walks a chain alone and
+// 2.4 / L here.  (Reading values that other waves dequantised into LDS costs about
+// 11 cycles a step against 5.7 here, and its LDS footprint ran 1536 x 8960 in two
+// rounds of workgroups: 22.5 us against 11.4 with L = 8.)
+constexpr int BT_LONG = 12;  // packed groups past which it serves (launch_gemv)
+// Floats of a chain's activations: phases of 32 steps, 4 floats apart in the
+// banks, neighbouring chains 16 apart.
+__host__ __device__ constexpr int64_t baton_stride(int64_t K) {
+    return (36 * (((K / 32 + 3) / 4 + 1) / 2) + 15) / 32 * 32 + 16;
+}
+
+template <int MODE, int L>
+__global__ __launch_bounds__(THREADS) void gemv_q4_baton_kernel(GemvParams p) {
+    constexpr int RW = 8 / L;  // rows of a wave
+    extern __shared__ __align__(16) float xs[];  // [8][baton_stride(K)]
+    DevState *st = p.st;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nb = p.nb, G = (nb + 3) >> 2, P = (G + 1) >> 1;  // phases
+    const int CS = (int)baton_stride(p.K);
+    const int64_t row0 = ((int64_t)blockIdx.x * (THREADS / WAVE) + wave) * RW;  // the wave's first row
+    const int64_t rows = min(p.N, p.rows_valid);
+    const bool any_row = row0 < rows;  // (uniform in the wave)
+    const int r = lane / L, j = lane % L;
+    // chain (and row) of this lane in tile t
+    auto chain = [&](int t) { return (r - t) & (WAVE / L - 1); };
+
+    vu2 n[2][2];  // two tiles' weights in flight
+    vu4 s[2][2];
+    const uint8_t *w = p.w + (size_t)(any_row ? row0 : 0) * G * 80;
+    const int last = any_row ? (int)min((int64_t)RW, rows - row0) - 1 : 0;
+    auto load = [&](vu2 (&n)[2], vu4 (&s)[2], int t) {  // (clamped; a group past the row's end is made zeros when it is used)
+        const int c = chain(t);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint8_t *g = w + ((size_t)min(c >> 3, last) * G + min(2 * (L * t + j) + h, G - 1)) * 80;
+            n[h] = *(const vu2 *)(g + 8 * (c & 7));
+            s[h] = *(const vu4 *)(g + 64);
+        }
+    };
+    if (any_row) {
+        load(n[0], s[0], 0);
+        load(n[1], s[1], 1);
+    }
+    const int64_t row = row0 + (lane >> 3);  // lanes 0 and (L = 4) 8 store
+    const bool stores = (lane & 7) == 0 && (lane >> 3) < RW && row < p.N;
+    float bias = 0.0f, old = 0.0f, kthr = -INFINITY;
+    if (stores) {
+        if (row < p.bias_len) bias = p.bias[row];
+        if constexpr (MODE == MODE_RESIDUAL) {
+            old = p.y[row];
+            if (p.kwta_k > 0) kthr = *p.kwta_thr;
+        }
+    }
+    // the activations, one row of steps per chain (element 32 q + 8 c + l: chain l,
+    // step 4 q + c), zero past the row's end
+    int bad = 0;
+    for (int q = tid; q < 8 * P; q += THREADS) {
+        float4 v[8];
+        if (p.x_cm) {
+#pragma unroll
+            for (int l = 0; l < 8; ++l)
+                v[l] = q < nb ? *(const float4 *)(p.x_cm + (size_t)l * p.cm_stride + 4 * q) : make_float4(0.f, 0.f, 0.f, 0.f);
+        } else {
+            float4 f[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                f[k] = q < nb ? *(const float4 *)(p.x + 32 * (size_t)q + 4 * k) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int l = 0; l < 8; ++l) {
+                const int h = l >> 2;
+                auto pick = [&](const float4 &a) { return (l & 3) == 0 ? a.x : (l & 3) == 1 ? a.y : (l & 3) == 2 ? a.z : a.w; };
+                v[l] = make_float4(pick(f[h]), pick(f[2 + h]), pick(f[4 + h]), pick(f[6 + h]));
+            }
+        }
+#pragma unroll
+        for (int l = 0; l < 8; ++l) {
+            bad |= isnan(v[l].x) | isnan(v[l].y) | isnan(v[l].z) | isnan(v[l].w);
+            *(float4 *)(xs + l * CS + 4 * q + 4 * (q >> 3)) = v[l];
+        }
+    }
+    if (st && s_load_i32(&st->halted)) return;  // uniform
+    if (p.st_in >= 0 && __any(bad) && lane == 0) nan_flag(st, p.layer, p.st_in);
+    lds_barrier();
+    float acc = 0.0f;
+    if (any_row) {
+        auto tile = [&](int t, vu2 (&n)[2], vu4 (&s)[2]) {
+            float4 x[8];
+            const float *xl = xs + (chain(t) & 7) * CS + 36 * min(L * t + j, P - 1);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[i] = *(const float4 *)(xl + 4 * i);
+            if (2 * (L * t + j) + 1 >= G) s[1] = (vu4){0u, 0u, 0u, 0u};  // a row of an odd number of groups
+            float d[8][4];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                q4_dequant_dw<0>(d[4 * h + 0], n[h].x, s[h].x);
+                q4_dequant_dw<1>(d[4 * h + 1], n[h].x, s[h].y);
+                q4_dequant_dw<0>(d[4 * h + 2], n[h].y, s[h].z);
+                q4_dequant_dw<1>(d[4 * h + 3], n[h].y, s[h].w);
+            }
+            load(n, s, t + 2);
+            const int np = min(L, P - L * t);
+            for (int ph = 0; ph < np; ++ph) {
+                acc = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, acc), 0x13C, 0xF, 0xF, false));
+#pragma unroll
+                for (int i = 0; i < 8; ++i) acc = q4_chain(acc, d[i], x[i]);
+            }
+        };
+        for (int t = 0; L * t < P; t += 2) {
+            tile(t, n[0], s[0]);
+            if (L * (t + 1) < P) tile(t + 1, n[1], s[1]);
+        }
+    }
+    // chain c's sum is in lane L c + P - 1 (mod 64)
+    const float a = __shfl(acc, (L * lane + P - 1) & 63, WAVE);
+    float y = row < rows ? flush_small(red8_dpp(a)) : 0.0f;
+    if (!stores) return;
+    if (p.a_ptr) {  // sparse anchors, then the bias (forward.rs:103-115)
+        for (int64_t k = p.a_ptr[row]; k < p.a_ptr[row + 1]; ++k) {
+            const int e = (int)p.a_col[k], c = e >> 3;
+            const float prod = xs[(e & 7) * CS + c + 4 * (c >> 5)] * half_bits(p.a_val[k]);
+            y = y + prod;
+        }
+    }
+    if (row < p.bias_len) y = y + bias;
+    if constexpr (MODE == MODE_RESIDUAL) {
+        if (isnan(y)) nan_flag(st, p.layer, p.st_a);
+        // the previous block's K-WTA on the residual (the MODE_QKV launch's threshold)
+        if (p.kwta_k > 0) old = old < kthr ? -1e9f : old;
+        y = old + y;
+        if (isnan(y)) nan_flag(st, p.layer, p.st_b);
+    }
+    p.y[row] = y;
+}
+
 // gemv_q4_chain_kernel for a mode, norm and row length (G packed groups).
 template <int MODE, bool NORM, int GX = CH_XREG_MAX>
 void (*chain_kernel_g(int G))(GemvParams, int64_t, int) {
@@ -2671,6 +2816,16 @@ static bool chain_ok(const GemvParams &p, int64_t npairs) {
            clds + 1024 <= max_lds_per_block();
 }
 
+// The baton kernel's: long Q4_0 rows without a norm, at most one wave per SIMD of
+// two rows each.  Rows of up to BT_LONG groups stay on the chain kernel (1536 x
+// 1536, 12 groups: 4.1 against 4.4 us; 1000 x 2080, 17 groups: 4.9 against 4.6; 896
+// x 4864: 8.0 against 6.0).
+static bool baton_ok(const GemvParams &p) {
+    return p.fmt == FMT_Q4_0 && (p.mode == MODE_STORE || p.mode == MODE_RESIDUAL) && !p.gnorm && !p.x_out && !p.norm_w &&
+           (p.nb + 3) / 4 > BT_LONG && p.N <= 8 * (int64_t)device_cu_count() && p.K <= (1 << 20) &&
+           (size_t)baton_stride(p.K) * 32 + 1024 <= max_lds_per_block();
+}
+
 bool gemv_chain_serves(const GemvParams &p) {
     if (p.N <= 0 || p.K <= 0 || p.nb != (int32_t)(p.K / 32)) return false;
     int64_t npairs;
@@ -2734,6 +2889,21 @@ int launch_gemv(const GemvParams &p, hipStream_t s) {
     if (p.kwta_k > 0 && (!chain || (p.mode != MODE_QKV && p.mode != MODE_RESIDUAL) || !p.kwta_thr || p.x_cm ||
                          (p.mode == MODE_QKV && p.K > INT32_MAX)))
         return set_error(GAJE_ERR_UNSUPPORTED, "gemv: the fused K-WTA runs only on the chain kernel (QKV / residual)");
+    if (baton_ok(p) && (p.kwta_k <= 0 || chain)) {
+        GemvParams pc = p;  // x_cm only where its rows are whole quads of this row's steps
+        if (pc.x_cm && (pc.cm_stride % 4 || pc.cm_stride < 4 * p.nb || ((uintptr_t)pc.x_cm & 15))) pc.x_cm = nullptr;
+        const size_t blds = (size_t)baton_stride(p.K) * 32;
+        // one row per wave while each has a SIMD of its own (its chains then
+        // have eight lanes), else two
+        const int rw = p.N <= 4 * (int64_t)device_cu_count() ? 1 : 2;
+        const dim3 grid((unsigned)((p.N + 4 * rw - 1) / (4 * rw)));
+        void (*fn)(GemvParams) =
+            p.mode == MODE_RESIDUAL ? (rw == 1 ? gemv_q4_baton_kernel<MODE_RESIDUAL, 8> : gemv_q4_baton_kernel<MODE_RESIDUAL, 4>)
+                                    : (rw == 1 ? gemv_q4_baton_kernel<MODE_STORE, 8> : gemv_q4_baton_kernel<MODE_STORE, 4>);
+        hipLaunchKernelGGL(fn, grid, dim3(THREADS), blds, s, pc);
+        GAJE_HIP_CHECK(hipGetLastError());
+        return GAJE_OK;
+    }
     // latency-bound Q4_0 matvecs (few rows): split waves
     if (chain) {
         const int64_t G = (p.nb + 3) / 4;

@@ -180,6 +180,11 @@ struct AttnParams {
     const int32_t *seq_pos, *row_seq;
     int64_t seq_kv_stride, seq_q_stride;
     int32_t n_seq;           // rows
+    // launch_attn_rows: tiles of consecutive tokens, {first row, rows <=
+    // ATTN_ROWS_TILE} each, the rows of one sequence at consecutive positions
+    // (row_seq null: one cache for all rows); no context is longer than ctx
+    const int32_t *tiles;
+    int32_t n_tiles;
     // where a kernel whose LDS producers and consumers wait on each other
     // reports a wait that ran out of its spin bound (layer * 8 + ST_WAIT):
     // st->nan_code for one sequence, seq_nan[z] for batched sequence z
@@ -187,6 +192,11 @@ struct AttnParams {
     int32_t layer;
 };
 int launch_attention(const AttnParams &p, hipStream_t s);
+// Rows of several tokens per sequence (a prompt's): tiles of up to
+// ATTN_ROWS_TILE consecutive tokens, where attn_rows_serves.
+constexpr int ATTN_ROWS_TILE = 16;
+bool attn_rows_serves(int head_dim, int64_t kv_cap, int64_t ctx);
+int launch_attn_rows(const AttnParams &p, hipStream_t s);
 size_t attention_lds_bytes(int head_dim, int64_t max_ctx);
 // Largest KV capacity whose scores fit the attention kernel's LDS buffer.
 constexpr int64_t MAX_CTX = 12288;

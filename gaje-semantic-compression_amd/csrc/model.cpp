@@ -266,7 +266,7 @@ int fuse_linears(std::vector<HostLinear> parts, const std::string &name, HostLin
 struct RowBufs {
     int64_t rows = 0;        // rows they hold
     float *H = nullptr, *XN = nullptr, *QKV = nullptr, *Q = nullptr, *ATT = nullptr, *GU = nullptr, *ACT = nullptr;
-    uint32_t *ids = nullptr;  // [3][rows]: embedding rows, then each row's position and sequence
+    uint32_t *ids = nullptr;  // embedding rows, then each row's position and sequence, then the attention's tiles
     uint32_t *nan_codes = nullptr;  // [rows] guards
 };
 
@@ -1012,8 +1012,8 @@ namespace {
 
 // Rows of one bit-exact pass: enough that the products' tiles fill the chip
 // several times, few enough that the buffers stay small (the gate/up rows of a
-// 1.5B-parameter model: 73 MB).
-constexpr int64_t ROWS_CHUNK = 1024;
+// 1.5B-parameter model: 147 MB).
+constexpr int64_t ROWS_CHUNK = 2048;
 
 // Token rows whose blocks run together (rows_blocks): row r is a token of
 // sequence seq[r] at position pos[r] of its cache (pos[r] < 0: computed and
@@ -1023,6 +1023,9 @@ struct RowPass {
     int64_t R = 0;
     const int32_t *pos = nullptr, *seq = nullptr;
     int64_t pos0 = 0;
+    const int32_t *tiles = nullptr;  // the attention's tiles of consecutive tokens (AttnParams), or null
+    int32_t n_tiles = 0;
+    int64_t max_ctx = 0;             // longest context of the rows
     float *k_cache = nullptr, *v_cache = nullptr;  // layer 0
     int64_t layer_kv = 0, seq_kv = 0, cap = 0;     // floats per layer and per sequence, positions
     const float *rope_cos = nullptr, *rope_sin = nullptr;
@@ -1056,7 +1059,7 @@ int rows_reserve(Owner *o, const gaje_hip_model *m, RowBufs &b, int64_t rows) {
     GAJE_TRY(o->alloc(&b.ATT, (size_t)(rows * m->q_rows)));
     GAJE_TRY(o->alloc(&b.GU, (size_t)(rows * L0.gate_up.N)));
     GAJE_TRY(o->alloc(&b.ACT, (size_t)(rows * m->ffn)));
-    GAJE_TRY(o->alloc(&b.ids, (size_t)(3 * rows)));
+    GAJE_TRY(o->alloc(&b.ids, (size_t)(5 * rows)));  // at most one tile per row, two words each
     GAJE_TRY(o->alloc(&b.nan_codes, (size_t)rows));
     b.rows = rows;
     return GAJE_OK;
@@ -1159,7 +1162,14 @@ int rows_blocks(gaje_hip_model *m, const RowPass &c) {
         ap.n_seq = (int32_t)R;
         ap.seq_nan = b.nan_codes;
         ap.layer = li;
-        GAJE_TRY(launch_attention(ap, s));
+        if (c.tiles && attn_rows_serves((int)m->hd, c.cap, c.max_ctx)) {
+            ap.tiles = c.tiles;
+            ap.n_tiles = c.n_tiles;
+            ap.ctx = c.max_ctx;
+            GAJE_TRY(launch_attn_rows(ap, s));
+        } else {
+            GAJE_TRY(launch_attention(ap, s));
+        }
         BatchGemvParams g = rows_gemv(Ly.o, b.ATT, m->q_rows, b.H, E, R, b.nan_codes);
         g.mode = MODE_RESIDUAL;
         GAJE_TRY(launch_gemv_batch(g, s));
@@ -1182,6 +1192,16 @@ int rows_blocks(gaje_hip_model *m, const RowPass &c) {
         if (const int64_t k = block_kwta_k(m)) GAJE_TRY(launch_kwta_rows(b.H, E, E, R, k, s));
     }
     return GAJE_OK;
+}
+
+// Appends the attention's tiles of n consecutive tokens (rows row0 ..): {first
+// row, rows}; returns their number.
+int64_t attn_tiles(std::vector<uint32_t> &tiles, int64_t row0, int64_t n) {
+    for (int64_t i = 0; i < n; i += ATTN_ROWS_TILE) {
+        tiles.push_back((uint32_t)(row0 + i));
+        tiles.push_back((uint32_t)std::min<int64_t>(ATTN_ROWS_TILE, n - i));
+    }
+    return (n + ATTN_ROWS_TILE - 1) / ATTN_ROWS_TILE;
 }
 
 // n tokens one step at a time from m->pos (the captured token graph).
@@ -1212,6 +1232,7 @@ int prefill_rows(gaje_hip_model *m, const uint32_t *ids, int64_t n, bool &clean)
         up[i] = ids[i];
         up[n + i] = (uint32_t)(m->pos + i);
     }
+    const int64_t nt = attn_tiles(up, 0, n);
     GAJE_HIP_CHECK(hipMemcpyAsync(b.ids, up.data(), up.size() * 4, hipMemcpyHostToDevice, s));
     GAJE_TRY(launch_fill_u32(b.nan_codes, NAN_NONE, n, s));
     GAJE_TRY(launch_embed_rows(embed_params(m, b.H), b.ids, n, s));
@@ -1220,6 +1241,9 @@ int prefill_rows(gaje_hip_model *m, const uint32_t *ids, int64_t n, bool &clean)
     c.R = n;
     c.pos = (const int32_t *)(b.ids + n);
     c.pos0 = m->pos;
+    c.tiles = (const int32_t *)(b.ids + 2 * n);
+    c.n_tiles = (int32_t)nt;
+    c.max_ctx = m->pos + n;
     c.k_cache = m->k_cache;
     c.v_cache = m->v_cache;
     c.layer_kv = m->n_kv * m->cap * m->hd;
@@ -1711,26 +1735,36 @@ int batch_feed_rows(gaje_hip_batch *b, const uint32_t *ids, int64_t n, int64_t i
     std::vector<uint32_t> up;
     for (int64_t c0 = i0; c0 < i1; c0 += per) {
         const int64_t c1 = std::min(i1, c0 + per);
-        std::vector<uint32_t> tok, pos, seq;
+        std::vector<uint32_t> tok, pos, seq, tiles;
         std::vector<int32_t> end(b->pos);
-        for (int64_t q = 0; q < b->nseq; ++q)
+        int64_t nt = 0, max_ctx = 0;
+        for (int64_t q = 0; q < b->nseq; ++q) {
+            const int64_t row0 = (int64_t)tok.size();
             for (int64_t i = c0; i < c1 && !b->halted[q]; ++i)
                 if (ids[q * n + i] != BATCH_INACTIVE) {
                     tok.push_back(ids[q * n + i]);
                     pos.push_back((uint32_t)end[q]++);
                     seq.push_back((uint32_t)q);
                 }
+            nt += attn_tiles(tiles, row0, (int64_t)tok.size() - row0);
+            max_ctx = std::max<int64_t>(max_ctx, end[q]);
+        }
         const int64_t R = (int64_t)tok.size();
         if (R == 0) continue;
         GAJE_TRY(rows_reserve(b, m, b->rb, R));
         up.assign(tok.begin(), tok.end());
         up.insert(up.end(), pos.begin(), pos.end());
         up.insert(up.end(), seq.begin(), seq.end());
+        up.insert(up.end(), tiles.begin(), tiles.end());
         GAJE_HIP_CHECK(hipMemcpyAsync(b->rb.ids, up.data(), up.size() * 4, hipMemcpyHostToDevice, s));
         GAJE_TRY(launch_fill_u32(b->rb.nan_codes, NAN_NONE, R, s));
         GAJE_TRY(launch_embed_rows(embed_params(m, b->rb.H), b->rb.ids, R, s));
         const int32_t *dpos = (const int32_t *)(b->rb.ids + R);
-        GAJE_TRY(rows_blocks(m, batch_rows(b, b->rb, R, dpos, dpos + R)));
+        RowPass c = batch_rows(b, b->rb, R, dpos, dpos + R);
+        c.tiles = dpos + 2 * R;
+        c.n_tiles = (int32_t)nt;
+        c.max_ctx = max_ctx;
+        GAJE_TRY(rows_blocks(m, c));
         GAJE_HIP_CHECK(hipMemcpyAsync(up.data(), b->rb.nan_codes, (size_t)R * 4, hipMemcpyDeviceToHost, s));
         GAJE_HIP_CHECK(hipStreamSynchronize(s));
         bool clean = true;

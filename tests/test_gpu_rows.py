@@ -18,6 +18,7 @@ TINY = dict(n_embd=128, n_head=4, n_head_kv=2, n_blocks=2, ffn=256, vocab_size=1
             rope_base=1e4, arch_family=1, qkv_bias=1, tied_embeddings=0)
 HD64 = dict(TINY, n_embd=256, ffn=544)
 HD128 = dict(TINY, n_embd=384, n_head=3, n_head_kv=1, ffn=512, n_blocks=1)
+LONG = dict(TINY, n_embd=128, n_head=2, n_head_kv=1, ffn=128, n_blocks=1, vocab_size=300)
 NAN_TOKEN = 42
 
 
@@ -103,10 +104,12 @@ def _oracle(O, path, kwta):
 
 
 # prompts of two tokens, of a few tiles, and of more rows than one pass takes, on an
-# empty cache and after it
+# empty cache and after it; the last one's second prompt has contexts past what
+# the rows' attention holds in LDS
 @pytest.mark.parametrize("name,cfg,kwta,lengths", [("tiny", TINY, 0.0, [2, 33, 1]), ("tiny", TINY, 0.5, [19]),
                                                    ("hd64", HD64, 0.0, [65, 3]), ("hd128", HD128, 0.0, [130]),
-                                                   ("gnorm", GNORM_MODEL, 0.0, [17]), ("tiny", TINY, 0.0, [1040])])
+                                                   ("gnorm", GNORM_MODEL, 0.0, [17]), ("tiny", TINY, 0.0, [2060]),
+                                                   ("long", LONG, 0.0, [2490, 20])])
 def test_prompt_rows_match_the_oracle(hip, O, tmp_models, name, cfg, kwta, lengths):
     p = _write(hip, tmp_models, name, cfg)
     g, r = hip.load_genomic_auto(p), _oracle(O, p, kwta)

@@ -1743,102 +1743,122 @@ void *q8l_kernel(int G) {
 }
 
 // LUT-4bit rows stored whole (MODE_STORE, optional bias, no anchors or
-// prologue), LDS-staged: one wave per workgroup takes 16 rows (lane 4 r + c:
-// row r, chain c) and copies, all at once with LDS-direct loads, x, the 16
-// rows' codes (16 B per block, contiguous) and their 16-entry tables (one per
-// row and block, or the one shared table); then each lane walks its chain
-// (elements e of a block with e % 4 == c, blocks in order: genomic.rs:148-204)
-// with its table lookups and x reads from LDS.  Against row_lut4, which waits
-// for each block's table before its lookups, every byte of the tile is in
-// flight from the start.
-constexpr int LUTL_ROWS = 16;
-// Tables in LDS: row q's nb tables at q nb 64 bytes, as the tile lies in
-// memory (one copy per KiB).  For even nb every row's tables then begin on the
-// same LDS bank, so a block's lookups from the 16 rows conflict; padding the
-// rows apart (one copy per row and KiB) measured slower (9.2 against 7.3 us
-// per C0-LUT launch).
-__host__ __device__ constexpr int64_t lut4_trow_bytes(int64_t nb) { return nb * 64; }
-size_t lut4_lds_bytes(int64_t K, int64_t nb, bool shared_table) {
-    const size_t xb = (size_t)K * 4, cb = (size_t)LUTL_ROWS * nb * 16;
-    const size_t tb = shared_table ? 64 : (size_t)LUTL_ROWS * lut4_trow_bytes(nb);
-    return (xb + 1023) / 1024 * 1024 + (cb + 1023) / 1024 * 1024 + (tb + 1023) / 1024 * 1024;
+// prologue), LDS-staged: W waves of four rows, each wave copying its own rows'
+// codes (16 B per block, contiguous) and 16-entry tables (one per row and block, or
+// the one shared table) with LDS-direct loads, all at once; x is shared, one row of
+// steps per chain.
+//
+// A row's four chains (elements e of a block with e % 4 == c, blocks in order:
+// genomic.rs:148-204) run as batons: four lanes per chain, each holding the
+// products of one phase (two blocks, 16 steps) of the tile in registers, the running
+// sum handed to the next lane every 16 adds (DPP wave_ror:1).  In tile t lane 4 r +
+// j holds phase 4 t + j of chain (r - t) mod 16 (chain 4 q + c: chain c of the
+// wave's row q); chain g's sum is in lane 4 g + p after phase p (mod 64).  So the
+// lookups and products, about four instructions per step, are spread over four
+// lanes and only the add is serial, and four times as many waves share the rows:
+// 4864 x 896 with a table per block 7.5 us with one lane per chain and 16 rows per
+// wave.
+constexpr int LUTL_WR = 4;  // rows per wave
+// LDS: the chains' activations (phases of 16 floats, 20 apart; chains 16 banks
+// apart), then per wave the codes and the tables, in whole KiB copies.
+__host__ __device__ constexpr int lut4_chain_floats(int64_t nb) { return (int)((20 * ((nb + 1) / 2) + 15) / 32 * 32 + 16); }
+__host__ __device__ constexpr int64_t lut4_kib(int64_t bytes) { return (bytes + 1023) / 1024 * 1024; }
+size_t lut4_lds_bytes(int waves, int64_t nb, bool shared_table) {
+    return (size_t)lut4_chain_floats(nb) * 16 +
+           (size_t)waves * (lut4_kib(LUTL_WR * nb * 16) + lut4_kib(shared_table ? 64 : LUTL_WR * nb * 64));
 }
 
-template <bool SHARED>
-__global__ __launch_bounds__(WAVE) void gemv_lut4_lds_kernel(GemvParams p) {
+template <int W, bool SHARED>
+__global__ __launch_bounds__(W * WAVE) void gemv_lut4_lds_kernel(GemvParams p) {
     extern __shared__ __align__(16) float smem[];
-    const int lane = threadIdx.x, r = lane >> 2, c = lane & 3, base = lane & ~3;
-    const int nb = p.nb;
-    const int64_t K = p.K;
-    const int64_t r0 = (int64_t)blockIdx.x * LUTL_ROWS;
-    float *xs = smem;
-    const int64_t xb = K * 4, cb = (int64_t)LUTL_ROWS * nb * 16;
-    const int64_t trs = lut4_trow_bytes(nb);
-    uint8_t *codes = (uint8_t *)smem + (xb + 1023) / 1024 * 1024;
-    float *tabs = (float *)(codes + (cb + 1023) / 1024 * 1024);
-    // ---- every copy at once: x, the codes, the tables ----
-    lds_copy_bytes(p.x, xb, lds_addr(xs), lane);
-    {
-        // codes of rows r0 .. r0 + 15 (contiguous); lanes past the tensor re-read its start
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane >> 2, j = lane & 3;
+    const int nb = p.nb, P = (nb + 1) >> 1, CS = lut4_chain_floats(nb);  // phases, floats of a chain
+    const int64_t r0 = ((int64_t)blockIdx.x * W + wave) * LUTL_WR;  // the wave's first row
+    const int64_t cb = LUTL_WR * (int64_t)nb * 16, tb = SHARED ? 64 : LUTL_WR * (int64_t)nb * 64;
+    uint8_t *codes = (uint8_t *)(smem + 4 * CS) + wave * (lut4_kib(cb) + lut4_kib(tb));
+    const float *tabs = (const float *)(codes + lut4_kib(cb));
+    // ---- every copy at once: the codes, the tables; rows past the tensor copy its last ----
+    if (r0 < p.N) {  // (uniform in the wave)
         const uint8_t *cw = p.w + r0 * nb * 16;
         const int64_t cend = (p.N - r0) * nb * 16;
         for (int64_t o = 0; o < cb; o += 1024) {
             const int64_t a = o + lane * 16;
             lds_dma16(cw + (a + 16 <= cend ? a : 0), lds_addr(codes) + (uint32_t)o);
         }
-    }
-    if constexpr (SHARED) {
-        if (lane < 4) lds_dma16<true>(p.lut + 4 * lane, lds_addr(tabs));
-    } else {
-        // row q's table set (nb 64 bytes) starts at q nb 64 bytes if q < lut_rows_own,
-        // else at 0; rows past the tensor copy row r0's
-        const uint32_t rs = (uint32_t)nb * 64;
-        const uint8_t *lb = (const uint8_t *)p.lut;
-        const int64_t tb = (int64_t)LUTL_ROWS * rs;
-        if (r0 + LUTL_ROWS <= p.lut_rows_own && r0 + LUTL_ROWS <= p.N) {
-            for (int64_t o = 0; o < tb; o += 1024) lds_dma16(lb + r0 * rs + o + lane * 16, lds_addr(tabs) + (uint32_t)o);
+        if constexpr (SHARED) {
+            if (lane < 4) lds_dma16<true>(p.lut + 4 * lane, lds_addr(tabs));
         } else {
+            // row q's table set (nb 64 bytes) starts at q nb 64 bytes if q < lut_rows_own, else at 0
+            const uint32_t rs = (uint32_t)nb * 64;
+            const uint8_t *lb = (const uint8_t *)p.lut;
+            const bool own = r0 + LUTL_WR <= p.lut_rows_own && r0 + LUTL_WR <= p.N;
             for (int64_t o = 0; o < tb; o += 1024) {
                 const uint32_t a = (uint32_t)o + lane * 16;
-                int64_t q = r0 + a / rs;
-                q = q < p.N ? q : r0;
-                const int64_t src = (q < p.lut_rows_own ? q * rs : 0) + a % rs;
-                lds_dma16(lb + src, lds_addr(tabs) + (uint32_t)o);
+                if (own) {
+                    lds_dma16(lb + r0 * rs + (a < tb ? a : 0), lds_addr(tabs) + (uint32_t)o);
+                } else {
+                    int64_t q = r0 + (a < tb ? a / rs : 0);
+                    q = q < p.N ? q : r0;
+                    lds_dma16(lb + (q < p.lut_rows_own ? q * rs : 0) + a % rs, lds_addr(tabs) + (uint32_t)o);
+                }
             }
         }
     }
-    if (p.st && s_load_i32(&p.st->halted)) {
-        wait_vmcnt<0>();
-        return;
+    // ---- x: element 32 b + 4 u + c is step 8 b + u of chain c; zero past the row ----
+    for (int m = tid; m < 16 * P; m += W * WAVE) {
+        const float4 v = m < 8 * nb ? *(const float4 *)(p.x + 4 * (size_t)m) : make_float4(0.f, 0.f, 0.f, 0.f);
+        float *d = smem + 20 * (m >> 4) + (m & 15);
+        d[0] = v.x;
+        d[CS] = v.y;
+        d[2 * CS] = v.z;
+        d[3 * CS] = v.w;
     }
+    const bool stores = (lane & 3) == 0 && (lane >> 2) < LUTL_WR && r0 + (lane >> 2) < p.N;
+    const int64_t row = r0 + (lane >> 2);
+    const float bias = stores && row < p.bias_len ? p.bias[row] : 0.0f;
+    const bool halted = p.st && s_load_i32(&p.st->halted);
     wait_vmcnt<0>();
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    __builtin_amdgcn_wave_barrier();
-    // ---- the chain: acc = acc + tbl[code] * x[e], mul then add, blocks in order ----
+    lds_barrier();
+    if (halted || r0 >= p.N) return;
     float acc = 0.0f;
-    const uint8_t *crow = codes + (size_t)r * nb * 16;
-    const float *trow = SHARED ? tabs : (const float *)((const uint8_t *)tabs + r * trs);
-    for (int j = 0; j < nb; ++j) {
-        const vu4 cw = *(const vu4 *)(crow + (size_t)j * 16);
-        const float *t = SHARED ? trow : trow + (size_t)j * 16;
-        const float *xj = xs + (size_t)j * 32 + c;
+    for (int t = 0; 4 * t < P; ++t) {
+        const int g = (r - t) & 15, q = g >> 2, c = g & 3, ph = min(4 * t + j, P - 1);
+        vf4 x[4];
+        const float *xl = smem + c * CS + 20 * ph;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            // element e = 4 u + c; even e is the high nibble of byte e / 2
-            const uint32_t word = (u >> 1) == 0 ? cw.x : (u >> 1) == 1 ? cw.y : (u >> 1) == 2 ? cw.z : cw.w;
-            // byte e / 2 = 2 u + c / 2 of the block: bits 8 ((2u + c/2) & 3) of word u / 2
-            const uint32_t idx = __builtin_amdgcn_ubfe(word, 8 * ((2 * u + (c >> 1)) & 3) + ((c & 1) ? 0 : 4), 4);
-            const float prod = t[idx] * xj[4 * u];
-            acc = acc + prod;
+        for (int i = 0; i < 4; ++i) x[i] = *(const vf4 *)(xl + 4 * i);
+        float prod[16];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const bool in = 2 * ph + h < nb;  // the last phase of an odd row has one block
+            const int b = in ? 2 * ph + h : nb - 1;
+            const vu4 cw = *(const vu4 *)(codes + ((size_t)q * nb + b) * 16);
+            const float *tt = SHARED ? tabs : tabs + ((size_t)q * nb + b) * 16;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                // element e = 4 u + c; even e is the high nibble of byte e / 2: bits
+                // 8 ((2 u + c / 2) & 3) of word u / 2
+                const uint32_t idx = __builtin_amdgcn_ubfe(cw[u >> 1], 8 * ((2 * u + (c >> 1)) & 3) + ((c & 1) ? 0 : 4), 4);
+                const float pr = tt[idx] * x[2 * h + (u >> 2)][u & 3];
+                prod[8 * h + u] = in ? pr : 0.0f;  // (+0 leaves a sum that started at +0 as it is)
+            }
+        }
+        const int np = min(4, P - 4 * t);
+        for (int k = 0; k < np; ++k) {
+            acc = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, acc), 0x13C, 0xF, 0xF, false));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc = acc + prod[i];
         }
     }
-    const float s1 = shfl(acc, base + 1), s2 = shfl(acc, base + 2), s3 = shfl(acc, base + 3);
-    float total = flush_small(((acc + s1) + s2) + s3);  // s0 + s1 + s2 + s3, left to right
-    const int64_t row = r0 + r;
-    if (c == 0 && row < p.N) {
-        if (row < p.bias_len) total = total + p.bias[row];
-        p.y[row] = total;
-    }
+    // row q's chains are g = 4 q + c, their sums in lanes 4 g + P - 1 (mod 64): to lane 4 q + c
+    const float a = shfl(acc, (4 * lane + P - 1) & 63);
+    const int base = lane & ~3;
+    const float s1 = shfl(a, base + 1), s2 = shfl(a, base + 2), s3 = shfl(a, base + 3);
+    float total = flush_small(((a + s1) + s2) + s3);  // s0 + s1 + s2 + s3, left to right
+    if (!stores) return;
+    if (row < p.bias_len) total = total + bias;
+    p.y[row] = total;
 }
 
 template <int MODE, int WAVES, int STAGES, int ROWS, bool TOL = false>
@@ -3022,11 +3042,16 @@ int launch_gemv(const GemvParams &p, hipStream_t s) {
         p.rows_valid == p.N && p.st_in < 0 && (p.lut_block_stride == 0 || p.lut_block_stride == 16) &&
         ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.lut & 15) == 0 && ((uintptr_t)p.w & 15) == 0) {
         const bool shared = p.lut_block_stride == 0;
-        const size_t llds = lut4_lds_bytes(p.K, p.nb, shared);
+        // two waves of four rows (4864 x 896: 6.6 us against 7.0 with four, whose
+        // 304 workgroups load the compute units unevenly); one where the LDS
+        // holds no more (rows past 5888 with a table per block)
+        const int waves = lut4_lds_bytes(2, p.nb, shared) + 1024 <= max_lds_per_block() ? 2 : 1;
+        const size_t llds = lut4_lds_bytes(waves, p.nb, shared);
         if (llds + 1024 <= max_lds_per_block()) {
-            const int64_t grid = (p.N + LUTL_ROWS - 1) / LUTL_ROWS;
-            hipLaunchKernelGGL(shared ? gemv_lut4_lds_kernel<true> : gemv_lut4_lds_kernel<false>, dim3((unsigned)grid),
-                               dim3(WAVE), llds, s, p);
+            const dim3 grid((unsigned)((p.N + waves * LUTL_WR - 1) / (waves * LUTL_WR)));
+            void (*lf)(GemvParams) = waves == 2 ? (shared ? gemv_lut4_lds_kernel<2, true> : gemv_lut4_lds_kernel<2, false>)
+                                                : (shared ? gemv_lut4_lds_kernel<1, true> : gemv_lut4_lds_kernel<1, false>);
+            hipLaunchKernelGGL(lf, grid, dim3(waves * WAVE), llds, s, p);
             GAJE_HIP_CHECK(hipGetLastError());
             return GAJE_OK;
         }

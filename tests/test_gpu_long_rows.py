@@ -60,3 +60,20 @@ def test_long_rows_in_a_decode_step(hip, O, tmp_models, kwta):
             a, b = g.forward(t, i == 0), r.forward_core(t, i == 0)
             assert np.array_equal(a.view(np.uint32), np.asarray(b, np.float32).view(np.uint32)), (name, i)
         g.close()
+
+
+# odd numbers of blocks, partial workgroups, a table per row and block or the shared
+# one, tables of only the first rows, and rows that leave LDS for one wave a workgroup
+@pytest.mark.parametrize("n,k,own", [(9, 96, 9), (6, 32, 3), (21, 928, 21), (13, 928, -1), (7, 6016, 7), (10, 8960, 5),
+                                     (5, 8992, -1)])
+def test_lut4_rows_match_the_oracle(hip, O, n, k, own):
+    codes, lut = hip.synth.lut4_tensor(41, f"long.{n}.{k}", n, k)
+    lut = lut[:16 if own < 0 else own * (k // 32) * 16].copy()
+    x, b = hip.synth.normal(42, f"x.{k}", k), hip.synth.normal(43, f"b.{n}", n)
+    ops = hip.ops
+    y = ops.DeviceBuffer(n * 4)
+    dev = ops.DeviceBuffer.from_array
+    ops.lut4_gemv(dev(codes), dev(lut), lut.size, dev(x), y, n, k, bias=dev(b), bias_len=n)
+    ops.synchronize()
+    want = O.GenomicLinear(codes, b"", lut, n, k, b, 4).forward_core(x)
+    assert np.array_equal(y.read(np.float32, n).view(np.uint32), np.asarray(want, np.float32).view(np.uint32))

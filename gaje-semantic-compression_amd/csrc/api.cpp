@@ -286,6 +286,17 @@ struct GemmWorkspace {
     size_t bytes;
 };
 
+// Whether m rows run straight from the packed rows (launch_gemm_q4_dir), without
+// building the block-scaled product's operands first: up to 64 rows always (8 x
+// 2048 x 1536 21.3 -> 14.3 us, 64 x 17920 x 1536 52.9 -> 36.1, 64 x 896 x 896 19.6 ->
+// 18.4), up to 96 where the weights are not few (96 x 17920 x 1536 57.4 -> 45.9, 96 x
+// 2048 x 1536 28.2 -> 28.0, but 96 x 896 x 896 20.4 -> 22.4); past that the tiles'
+// activation reads cost more than the operands (128 x 9728 x 4096 67 -> 71).
+bool gemm_direct(int64_t m, int64_t n, int64_t k) { return m <= 64 || (m <= 96 && n * k >= (int64_t)3 << 20); }
+GemmBsPlan gemm_plan(int64_t m, int64_t n, int64_t k) {
+    return gemm_direct(m, n, k) ? plan_gemm_q4_dir(m, n, k) : plan_gemm_q4_bs(m, n, k);
+}
+
 GemmWorkspace gemm_workspace(char *base, int64_t m, int64_t n, int64_t k, const GemmBsPlan &pl) {
     GemmWorkspace w{};
     size_t off = 0;
@@ -301,6 +312,8 @@ GemmWorkspace gemm_workspace(char *base, int64_t m, int64_t n, int64_t k, const 
     off = align256(off + (size_t)(m * w.ldsum) * 2);
     w.part = (float *)(base + off);
     off = align256(off + (size_t)pl.part_floats * 4);
+    // the weight operands, also where the rows run without them: a workspace sized for
+    // more rows serves fewer
     w.mins = (uint16_t *)(base + off);  // [n][ldsum]: the weight rows' block mins
     off = align256(off + (size_t)(n * w.ldsum) * 2);
     w.wf = (uint16_t *)(base + off);    // the weight rows' code fragments and scales
@@ -316,7 +329,7 @@ GemmWorkspace gemm_workspace(char *base, int64_t m, int64_t n, int64_t k, const 
 extern "C" int64_t gaje_hip_q4_0_gemm_mfma_workspace(int64_t m, int64_t n, int64_t k) {
     if (m < 0 || n <= 0 || k <= 0 || k % 32 != 0) return -1;
     if (m == 0) return 0;
-    return (int64_t)gemm_workspace(nullptr, m, n, k, plan_gemm_q4_bs(m, n, k)).bytes;
+    return (int64_t)gemm_workspace(nullptr, m, n, k, gemm_plan(m, n, k)).bytes;
 }
 
 extern "C" int gaje_hip_q4_0_gemm_mfma(const void *packed, const float *X, const float *bias, int64_t bias_len,
@@ -327,7 +340,7 @@ extern "C" int gaje_hip_q4_0_gemm_mfma(const void *packed, const float *X, const
         return set_error(GAJE_ERR_INVALID_ARG, "bad gemm arguments");
     if (m == 0 || n == 0) return GAJE_OK;
     if (((uintptr_t)workspace & 15) != 0) return set_error(GAJE_ERR_INVALID_ARG, "gemm workspace must be 16-byte aligned");
-    const GemmBsPlan pl = plan_gemm_q4_bs(m, n, k);
+    const GemmBsPlan pl = gemm_plan(m, n, k);
     const GemmWorkspace w = gemm_workspace((char *)workspace, m, n, k, pl);
     if ((int64_t)w.bytes > workspace_bytes)
         return set_error(GAJE_ERR_INVALID_ARG, "gemm workspace of %lld bytes is smaller than the %zu needed",
@@ -345,8 +358,10 @@ extern "C" int gaje_hip_q4_0_gemm_mfma(const void *packed, const float *X, const
     sp.sl = w.sl;
     sp.ldsum = w.ldsum;
     GAJE_TRY(launch_split_rows(sp, s));
-    GAJE_TRY(launch_q4_operands((const uint8_t *)packed, n, k, w.wf, w.wsc, w.mins, w.ldsum, s));
+    const bool direct = gemm_direct(m, n, k);
+    if (!direct) GAJE_TRY(launch_q4_operands((const uint8_t *)packed, n, k, w.wf, w.wsc, w.mins, w.ldsum, s));
     GemmBsParams p{};
+    p.wq = (const uint8_t *)packed;
     p.wf = w.wf;
     p.wsc = w.wsc;
     p.nbp4 = q4_frag_nbp4(k);
@@ -367,7 +382,7 @@ extern "C" int gaje_hip_q4_0_gemm_mfma(const void *packed, const float *X, const
     p.M = m;
     p.N = n;
     p.nb = (int32_t)(k / 32);
-    return launch_gemm_q4_bs(p, pl, s);
+    return direct ? launch_gemm_q4_dir(p, pl, s) : launch_gemm_q4_bs(p, pl, s);
 }
 
 namespace {
@@ -570,12 +585,14 @@ namespace {
 // The prepared experts of gaje_hip_moe_prepare: for each of the two products
 // (gate_up: N = 2 ffn, K = h; down: N = h, K = ffn) every expert's code
 // fragments, fragment scales and dense block mins (the block-scaled product's
-// weight operands), one expert after the other at fixed strides.
+// weight operands) and its packed rows, one expert after the other at fixed
+// strides.
 struct MoePrepared {
-    int64_t wf_stride[2], wsc_stride[2], mins_stride[2], ldm[2];
+    int64_t wf_stride[2], wsc_stride[2], mins_stride[2], ldm[2], wq_stride[2];
     uint16_t *wf[2];
     float *wsc[2];
     uint16_t *mins[2];
+    uint8_t *wq[2];
     size_t bytes;
 };
 
@@ -593,13 +610,21 @@ MoePrepared moe_prepared(char *base, int64_t h, int64_t ffn, int64_t E) {
         w.wf_stride[i] = (q4_frag_halves(NN[i], KK[i]) + 511) / 512 * 512;
         w.wsc_stride[i] = (q4_frag_scale_floats(NN[i], KK[i]) + 63) / 64 * 64;
         w.mins_stride[i] = (NN[i] * w.ldm[i] + 127) / 128 * 128;
+        w.wq_stride[i] = (int64_t)align256((size_t)q4_0_packed_bytes(NN[i], KK[i]));
         w.wf[i] = (uint16_t *)take((size_t)(E * w.wf_stride[i]) * 2);
         w.wsc[i] = (float *)take((size_t)(E * w.wsc_stride[i]) * 4);
         w.mins[i] = (uint16_t *)take((size_t)(E * w.mins_stride[i]) * 2);
+        w.wq[i] = (uint8_t *)take((size_t)(E * w.wq_stride[i]));
     }
     w.bytes = off;
     return w;
 }
+
+// Whether R dispatched rows over E experts run straight from the packed rows: up
+// to 56 per expert (8 x 4096, h 1536: 16 tokens 127 -> 86 us a layer, 128 tokens 136
+// -> 117, 192 tokens 160 -> 128; 256 tokens 157.6 -> 162, 512 tokens 253 -> 271).
+constexpr int64_t moe_direct_rows(int64_t E) { return 56 * E; }
+bool moe_direct(int64_t R, int64_t E) { return R <= moe_direct_rows(E); }
 
 // Workspace of gaje_hip_moe_ffn_prepared: the routing, the block-scaled
 // activation planes of the dispatched rows, the two products' results and
@@ -618,13 +643,21 @@ struct MoeBsWorkspace {
 MoeBsWorkspace moe_bs_workspace(char *base, int64_t T, int64_t h, int64_t ffn, int64_t E) {
     MoeBsWorkspace w{};
     const int64_t R = 2 * T, kmax = std::max(h, ffn);
-    w.pgu = plan_gemm_q4_bs_grouped(R, E, T, 2 * ffn, h);
-    w.pdn = plan_gemm_q4_bs_grouped(R, E, T, h, ffn);
+    const auto plan = moe_direct(R, E) ? plan_gemm_q4_dir_grouped : plan_gemm_q4_bs_grouped;
+    w.pgu = plan(R, E, T, 2 * ffn, h);
+    w.pdn = plan(R, E, T, h, ffn);
     const int64_t mt = BS_WR_ROWS * std::max(w.pgu.waves, w.pdn.waves);
     const int64_t gm = std::max(w.pgu.mtiles, w.pdn.mtiles) / E;  // row tiles per group
     w.plane_rows = gemm_bs_plane_rows(R + gm * mt);
     w.ldsum = gemm_bs_sum_cols(kmax);
-    const int64_t part = std::max(w.pgu.part_floats, w.pdn.part_floats);
+    // partials: those of fewer rows too (a direct plan's grow up to each multiple of
+    // DR_ROWS), so that a workspace sized for more tokens serves fewer
+    int64_t part = std::max(w.pgu.part_floats, w.pdn.part_floats);
+    for (int64_t r = DR_ROWS; r - DR_ROWS < std::min(R, moe_direct_rows(E)); r += DR_ROWS) {
+        const int64_t Rd = std::min({r, R, moe_direct_rows(E)});
+        part = std::max({part, plan_gemm_q4_dir_grouped(Rd, E, Rd / 2, 2 * ffn, h).part_floats,
+                         plan_gemm_q4_dir_grouped(Rd, E, Rd / 2, h, ffn).part_floats});
+    }
     size_t off = 0;
     auto take = [&](size_t bytes) {
         char *p = base + off;
@@ -674,6 +707,8 @@ extern "C" int gaje_hip_moe_prepare(const void *const *gate_up, const void *cons
             const uint8_t *pk = (const uint8_t *)(i == 0 ? gate_up[e] : down[e]);
             GAJE_TRY(launch_q4_operands(pk, NN[i], KK[i], w.wf[i] + e * w.wf_stride[i], w.wsc[i] + e * w.wsc_stride[i],
                                         w.mins[i] + e * w.mins_stride[i], w.ldm[i], s));
+            GAJE_HIP_CHECK(hipMemcpyAsync(w.wq[i] + e * w.wq_stride[i], pk, (size_t)q4_0_packed_bytes(NN[i], KK[i]) - Q4_TAIL_PAD,
+                                          hipMemcpyDeviceToDevice, s));
         }
     return GAJE_OK;
 }
@@ -738,6 +773,11 @@ extern "C" int gaje_hip_moe_ffn_prepared(const float *x, int64_t T, int64_t h, c
         p.nbp4 = q4_frag_nbp4(K);
         p.mins = pw.mins[i];
         p.ldm = pw.ldm[i];
+        p.wq = pw.wq[i];
+        p.g_wq_stride = pw.wq_stride[i];
+        p.g_wf_stride = pw.wf_stride[i];
+        p.g_wsc_stride = pw.wsc_stride[i];
+        p.g_mins_stride = pw.mins_stride[i];
         p.xh = w.xh;
         p.plane_rows = w.plane_rows;
         p.sh = w.sh;
@@ -755,11 +795,8 @@ extern "C" int gaje_hip_moe_ffn_prepared(const float *x, int64_t T, int64_t h, c
         p.g_offsets = w.offsets;
         p.g_groups = (int32_t)n_expert;
         p.g_mtiles = (int32_t)(pl.mtiles / n_expert);
-        p.g_wf_stride = pw.wf_stride[i];
-        p.g_wsc_stride = pw.wsc_stride[i];
-        p.g_mins_stride = pw.mins_stride[i];
         p.defer_reduce = i == 1 && pl.splits > 1;  // down: the combine sums its partials
-        return launch_gemm_q4_bs(p, pl, s);
+        return moe_direct(R, n_expert) ? launch_gemm_q4_dir(p, pl, s) : launch_gemm_q4_bs(p, pl, s);
     };
     GAJE_TRY(gemm(0, w.pgu, 2 * ffn, h, w.GU));
     // swiglu of every dispatched row into the planes, then down

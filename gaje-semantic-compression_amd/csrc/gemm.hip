@@ -95,6 +95,23 @@ __global__ __launch_bounds__(256) void q4_row_exp_kernel(const uint8_t *w, int64
     if (lane == 0) ew[row] = split_exponent(mx);
 }
 
+// The block-scaled activation plane: the 128 bytes (hi | lo) of a row's block b lie
+// with those of the seven other rows of its group of eight, block after block, so
+// that a tile's copy of a block is whole contiguous KiB.  (With whole rows one after
+// the other, the lines that a tile needs of a block are K * 4 bytes apart and fall
+// on few of the L2's channels: the products of a 512-token prompt, 1.5B widths, 41.5
+// us on average against 40.4.)
+// Halves to row m's block b; ldh = 64 halves per block, times the blocks.
+__device__ __forceinline__ int64_t bs_plane_half(int64_t m, int64_t b, int64_t ldh) {
+    return (m >> 3) * 8 * ldh + b * 512 + (m & 7) * 64;
+}
+// Byte offset of the row that lane's copy takes of the 8 rows m0 + 8 q .., from
+// bs_plane_half((m0 & ~7) + 8 q, b): m0 may start inside a group of eight.
+__device__ __forceinline__ uint32_t bs_plane_lane(int64_t m0, int lane, int64_t ldh) {
+    const int r = (int)(m0 & 7) + (lane >> 3);
+    return (uint32_t)((r >> 3) * 16 * ldh + (r & 7) * 128);
+}
+
 // One activation row per workgroup: a prologue (none, rms_norm (norm.rs:52-88),
 // or swiglu_balanced of a gate/up pair (activation.rs:35-51) with the optional
 // use_genomic_norm scaling of block/forward.rs:115-123; or the deferred
@@ -311,7 +328,7 @@ __global__ __launch_bounds__(NTH) void split_rows_kernel(SplitParams p) {
         if (b & 2) nan_flag(p.st, p.layer, p.st_b);
     }
     if (p.sh) {
-        // block-scaled layout: one plane, block b at halves 64 b.. holding its
+        // block-scaled layout (bs_plane_half): one plane, per row and block its
         // 32 hi halves then its 32 lo halves; position 8 kg + t of each holds
         // element 32 b + 2 kg + 8 (t & 3) + (t >> 2).  Chunk u (8 halves) is
         // (block u >> 2, kg = u & 3); the block sum 2^-5 sum x' (|x'| < 2^15)
@@ -330,7 +347,7 @@ __global__ __launch_bounds__(NTH) void split_rows_kernel(SplitParams p) {
                     lo[t] = (_Float16)(a - (float)hi[t]);
                     s8 += a;
                 }
-                _Float16 *row = (_Float16 *)p.xh + m * p.ldh + 64 * (u >> 2) + 8 * (u & 3);
+                _Float16 *row = (_Float16 *)p.xh + bs_plane_half(m, u >> 2, p.ldh) + 8 * (u & 3);
                 *(h8 *)row = hi;
                 *(h8 *)(row + 32) = lo;
             }
@@ -759,19 +776,19 @@ __global__ __launch_bounds__(64 * W, (BsShape<W, BPI, R, NB>::WG_PER_CU)) void g
     uint8_t *bfr = bs_mem + W * R * BS_ABLK;  // [NB][PB]: fragments, then scales (block e at 144 e floats)
 
     // activation copies: per block a wave copies its 32 rows x 128 bytes (the
-    // block's hi | lo halves, one cache line per row).  Instruction q takes rows
+    // block's hi | lo halves, one cache line per row, eight rows contiguous).  Instruction q takes rows
     // 8q..8q+7: lane -> row R = 8q + (lane >> 3), LDS chunk lane & 7, holding
     // global chunk (lane & 7) ^ ((R >> 1) & 7), so that the fragment reads of
     // 16 consecutive rows fall in distinct banks.  (R >> 1) & 7 is
     // (lane >> 4) ^ 4 (q & 1): one lane offset for even q, one for odd.  The
     // plane holds plane_rows >= the tile's rows, so no row is clamped, and its
     // byte offsets fit 32 bits (both checked by the launcher).
-    const uint32_t arow = (uint32_t)((lane >> 3) * 2 * p.ldh);
+    const uint32_t arow = bs_plane_lane(m0, lane, p.ldh);
     const uint32_t aoffs[2] = {arow + 16 * ((lane & 7) ^ (lane >> 4)), arow + 16 * ((lane & 7) ^ (lane >> 4) ^ 4)};
     auto dma_a = [&](int kk, int slot) {
         const int64_t b = b0 + min(kk, nblk - 1);
         const uint32_t dst = lds_addr(ring + slot * BS_ABLK);
-        const uint8_t *base = (const uint8_t *)p.xh + m0 * 2 * p.ldh + 128 * b;
+        const uint8_t *base = (const uint8_t *)p.xh + 2 * bs_plane_half(m0 & ~(int64_t)7, b, p.ldh);
 #pragma unroll
         for (int q = 0; q < BS_ADMA; ++q) lds_dma16_so(base + q * 16 * p.ldh, aoffs[q & 1], dst + q * 1024);
     };
@@ -1057,6 +1074,284 @@ __global__ __launch_bounds__(64 * W, (BsShape<W, BPI, R, NB>::WG_PER_CU)) void g
     }
 }
 
+// ---------------------------------------------------------------------------
+// The block-scaled product straight from the packed rows (few activation rows,
+// dense or of MoE experts): the same terms and operands as gemm_q4_bs_kernel,
+// without fragments.
+//
+// A workgroup is eight waves, one per compute unit; each wave takes all of the
+// tile's activation rows (up to 128) against its own 16 DR_J weight rows, so that
+// every weight is read and expanded once per row tile, by the one wave that uses
+// it: a lane's 16 code bytes and its row's 16 scale and min bytes per group go from
+// memory to registers, 0.625 bytes per weight where the fragments, scales and mins
+// take 2.2, and one group expands into four blocks' fragments with about 11 VALU
+// instructions each, beside 2 NI MFMAs and 4 NI fmas.  The activations (the split
+// pass's plane) are shared: a ring of DR_S stages of two blocks in LDS, one barrier
+// per stage.  Vector memory completes in order, so both kinds of load wait for the
+// slower one; activations are copied three stages ahead and weights loaded three
+// groups ahead, which covers a trip to HBM (four waves, three blocks ahead: 32 x
+// 17920 x 1536 ran at 0.6 us a block).  NI, the tile's 16-row units, is a template
+// argument chosen by the tile's own rows, so that an expert's product costs what
+// its rows need.
+constexpr int DR_W = 8;                     // waves
+constexpr int DR_J = 2;                     // 16-row weight units per wave
+constexpr int DR_NT = 16 * DR_J * DR_W;     // weight rows per workgroup
+constexpr int DR_S = 4;                     // stages in the ring
+constexpr int DR_BLK = DR_ROWS * 128;       // bytes of a block's rows (hi | lo)
+constexpr size_t DR_LDS = (size_t)DR_S * 2 * DR_BLK;
+
+template <int NI>
+__device__ __forceinline__ void dir_tile(const GemmBsParams &p, const uint8_t *wq, int z, int kb_per, int64_t n0, int64_t m0,
+                                         int64_t mend, uint8_t *ring) {
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, kg = lane >> 4;
+    const int G = (p.nb + 3) >> 2;
+    const int b0 = z * kb_per, nblk = min(p.nb, b0 + kb_per) - b0, g0 = b0 >> 2, ng = (nblk + 3) >> 2;
+    constexpr int CP = (4 * NI + DR_W - 1) / DR_W;  // activation copies per wave and stage (8 rows of a block each)
+
+    // activation copies: instruction c of a stage takes rows 8q .. 8q + 7 (q = c mod
+    // 2 NI) of its block c / (2 NI), the chunks of a row XORed by (row >> 1) & 7, as in
+    // gemm_q4_bs_kernel; in place of one past the stage's 4 NI a wave copies its first
+    // again (same bytes, same place)
+    const uint32_t arow = bs_plane_lane(m0, lane, p.ldh);
+    const uint32_t aoffs[2] = {arow + 16 * ((lane & 7) ^ (lane >> 4)), arow + 16 * ((lane & 7) ^ (lane >> 4) ^ 4)};
+    auto dma_a = [&](int st, int slot) {
+#pragma unroll
+        for (int i = 0; i < CP; ++i) {
+            int c = w + DR_W * i;
+            c = c < 4 * NI ? c : w < 4 * NI ? w : 0;
+            const int e = c >= 2 * NI ? 1 : 0, q = c - 2 * NI * e;
+            const int64_t b = b0 + min(2 * st + e, nblk - 1);
+            lds_dma16_so((const uint8_t *)p.xh + 2 * bs_plane_half((m0 & ~(int64_t)7) + 8 * q, b, p.ldh), q & 1 ? aoffs[1] : aoffs[0],
+                         lds_addr(ring + (2 * slot + e) * DR_BLK) + q * 1024);
+        }
+    };
+    // weights: unit j's row n0 + 16 j + fr (rows past N read the last, not stored)
+    const uint8_t *wrow[DR_J];
+#pragma unroll
+    for (int j = 0; j < DR_J; ++j) wrow[j] = wq + (size_t)min(n0 + 16 * j + fr, p.N - 1) * G * 80;
+    struct Group {
+        vu4 q[DR_J], s[DR_J];
+    };
+    auto load_g = [&](Group &r, int g) {
+        const size_t at = (size_t)(g0 + min(g, ng - 1)) * 80;
+#pragma unroll
+        for (int j = 0; j < DR_J; ++j) {
+            r.q[j] = *(const vu4 *)(wrow[j] + at + 16 * kg);
+            r.s[j] = *(const vu4 *)(wrow[j] + at + 64);
+        }
+    };
+    Group gr[4];
+#pragma unroll
+    for (int g = 0; g < 3; ++g) load_g(gr[g], g);
+#pragma unroll
+    for (int st = 0; st < DR_S - 1; ++st) dma_a(st, st);
+
+    f4 acc[NI][DR_J];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < DR_J; ++j) acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
+    // the min term over this split's blocks, 32 blocks a step (see gemm_q4_bs_kernel)
+    {
+        const _Float16 *sh = (const _Float16 *)p.sh, *sl = (const _Float16 *)p.sl;
+        for (int c = b0 >> 5; c <= (b0 + nblk - 1) >> 5; ++c) {
+            const int bl = 32 * c + 8 * kg;  // this lane's first block
+            h8 mh[DR_J];
+#pragma unroll
+            for (int j = 0; j < DR_J; ++j) {
+                const vu4 lo = *(const vu4 *)(wrow[j] + (size_t)min(bl >> 2, G - 1) * 80 + 64);
+                const vu4 hi = *(const vu4 *)(wrow[j] + (size_t)min((bl >> 2) + 1, G - 1) * 80 + 64);
+                vu4 mn;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t a = q < 2 ? lo[2 * q] : hi[2 * q - 4], b = q < 2 ? lo[2 * q + 1] : hi[2 * q - 3];
+                    const int blk = bl + 2 * q;  // the halves of blocks blk, blk + 1 inside [b0, b0 + nblk)
+                    mn[q] = (blk >= b0 && blk < b0 + nblk ? a >> 16 : 0u) |
+                            (blk + 1 >= b0 && blk + 1 < b0 + nblk ? b & 0xFFFF0000u : 0u);
+                }
+                mh[j] = __builtin_bit_cast(h8, mn);
+            }
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                const int64_t srow = min(m0 + 16 * i + fr, p.M - 1) * p.ldsum + bl;
+                const h8 x0 = *(const h8 *)(sh + srow), x1 = *(const h8 *)(sl + srow);
+#pragma unroll
+                for (int j = 0; j < DR_J; ++j) {
+                    f4 tm = __builtin_amdgcn_mfma_f32_16x16x32_f16(x0, mh[j], (f4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    tm = __builtin_amdgcn_mfma_f32_16x16x32_f16(x1, mh[j], tm, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf(32.0f, tm[r], acc[i][j][r]);
+                }
+            }
+        }
+    }
+
+    // fragment (i, plane P) of lane (fr, kg): row 16 i + fr, chunk (4 P + kg) ^ ((fr >> 1) & 7)
+    const uint32_t aoff0 = fr * 128 + 16 * (kg ^ ((fr >> 1) & 7)), aoff1 = aoff0 ^ 64;
+    // block u of group r, from ring block rb
+    auto block = [&](const Group &r, auto uc, int rb) {
+        constexpr int u = decltype(uc)::value;
+        h8 bf[DR_J];
+        float sc[DR_J];
+#pragma unroll
+        for (int j = 0; j < DR_J; ++j) {
+            uint32_t wa = u & 2 ? r.q[j][1] : r.q[j][0], wb = u & 2 ? r.q[j][3] : r.q[j][2];
+            if (u & 1) {
+                wa >>= 4;
+                wb >>= 4;
+            }
+            wa &= 0x0F0F0F0Fu;
+            wb &= 0x0F0F0F0Fu;
+            const vu4 f = {code_pair<0>(wa), code_pair<1>(wa), code_pair<0>(wb), code_pair<1>(wb)};
+            bf[j] = __builtin_bit_cast(h8, f);
+            sc[j] = half_lo(r.s[j][u]);
+        }
+        const uint8_t *ab = ring + rb * DR_BLK;
+        h8 a[2][2];
+        a[0][0] = *(const h8 *)(ab + aoff0);
+        a[0][1] = *(const h8 *)(ab + aoff1);
+        f4 pr[2][DR_J];
+        // the fmas of unit i - 1 issue between the MFMAs of unit i
+#pragma unroll
+        for (int i = 0; i <= NI; ++i) {
+            if (i + 1 < NI) {
+                a[(i + 1) & 1][0] = *(const h8 *)(ab + (i + 1) * 2048 + aoff0);
+                a[(i + 1) & 1][1] = *(const h8 *)(ab + (i + 1) * 2048 + aoff1);
+            }
+            if (i < NI) {
+#pragma unroll
+                for (int j = 0; j < DR_J; ++j)
+                    pr[i & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i & 1][0], bf[j], (f4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < DR_J; ++j)
+                    pr[i & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i & 1][1], bf[j], pr[i & 1][j], 0, 0, 0);
+            }
+            if (i > 0) {
+#pragma unroll
+                for (int j = 0; j < DR_J; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) acc[i - 1][j][q] = fmaf(sc[j], pr[(i - 1) & 1][j][q], acc[i - 1][j][q]);
+            }
+            if (i > 0 && i < NI) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // the next unit's fragments
+#pragma unroll
+                for (int q = 0; q < 2 * DR_J; ++q) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+                    __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // two fmas
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // Stage st, a group's first or second half (odd): the copies of stages st + 1 and
+    // st + 2 may be in flight, and the weight loads issued since st's copies went out
+    // (after every first half: one group's when st is even, two groups' when odd).
+    auto enter = [&](int st, int slot, auto odd) {
+        wait_vmcnt<(DR_S - 2) * CP + (decltype(odd)::value ? 4 : 2) * DR_J>();
+        lds_barrier();  // stage st has landed for every wave, and stage st - 1 has been read
+        dma_a(st + DR_S - 1, (slot + DR_S - 1) & (DR_S - 1));
+    };
+    // group g from set r, in ring stages slot, slot + 1; set next3 takes group g + 3
+    auto group = [&](const Group &r, Group &next3, int g, auto slotc) {
+        constexpr int slot = decltype(slotc)::value;
+        const int left = nblk - 4 * g;  // (uniform)
+        enter(2 * g, slot, std::false_type{});
+        block(r, std::integral_constant<int, 0>{}, 2 * slot);
+        if (left > 1) block(r, std::integral_constant<int, 1>{}, 2 * slot + 1);
+        load_g(next3, g + 3);
+        if (left <= 2) return;
+        enter(2 * g + 1, slot + 1, std::true_type{});
+        block(r, std::integral_constant<int, 2>{}, 2 * slot + 2);
+        if (left > 3) block(r, std::integral_constant<int, 3>{}, 2 * slot + 3);
+    };
+    const std::integral_constant<int, 0> s0{};
+    const std::integral_constant<int, 2> s2{};
+    for (int g = 0; g < ng; g += 4) {
+        group(gr[0], gr[3], g, s0);
+        if (g + 1 >= ng) break;
+        group(gr[1], gr[0], g + 1, s2);
+        if (g + 2 >= ng) break;
+        group(gr[2], gr[1], g + 2, s0);
+        if (g + 3 >= ng) break;
+        group(gr[3], gr[2], g + 3, s2);
+    }
+    wait_vmcnt<0>();  // no copy into LDS outlives the workgroup
+
+    // epilogue: lane holds rows 16 i + 4 kg + r of column 16 j + fr
+    int bad_a = 0, bad_b = 0;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        int exr[4];
+        int64_t mrow[4];
+        bool mok[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t m = m0 + 16 * i + 4 * kg + r;
+            mok[r] = m < mend;
+            mrow[r] = mok[r] ? m : p.M - 1;
+            exr[r] = p.ex[mrow[r]];
+        }
+#pragma unroll
+        for (int j = 0; j < DR_J; ++j) {
+            const int64_t n = n0 + 16 * j + fr;
+            if (n >= p.N) continue;
+            const float bias = n < p.bias_len ? p.bias[n] : 0.0f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float v = ldexpf(acc[i][j][r], -exr[r]);
+                if (!mok[r]) continue;
+                if (p.part) {
+                    p.part[((int64_t)z * p.M + mrow[r]) * p.N + n] = v;
+                    continue;
+                }
+                v = flush_small(v);
+                if (n < p.bias_len) v = v + bias;
+                bad_a |= isnan(v);
+                if (p.resid) v = p.resid[mrow[r] * p.ldr + n] + v;
+                bad_b |= isnan(v);
+                p.y[mrow[r] * p.ldy + n] = v;
+            }
+        }
+    }
+    if (p.st && !p.part) {
+        if (__any(bad_a) && lane == 0) nan_flag(p.st, p.layer, p.st_a);
+        if (__any(bad_b) && lane == 0) nan_flag(p.st, p.layer, p.st_b);
+    }
+}
+
+__global__ __launch_bounds__(64 * DR_W) void gemm_q4_dir_kernel(GemmBsParams p, BsGrid gd) {
+    extern __shared__ __align__(16) uint8_t bs_mem[];
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    // XCD x takes the x-th contiguous run of (row tile, split, weight tile) indices
+    const int Q = (int)(gridDim.x >> 3);
+    const int idx = (int)(blockIdx.x & 7) * Q + (int)(blockIdx.x >> 3);
+    if (idx >= gd.total) return;
+    const int t = idx % gd.ntiles, mz = idx / gd.ntiles;
+    const int z = mz % gd.splits, mt = mz / gd.splits;
+    int64_t m0 = (int64_t)mt * DR_ROWS, mend = p.M;
+    const uint8_t *wq = p.wq;
+    if (p.g_counts) {  // grouped (uniform)
+        const int e = mt / p.g_mtiles, mtl = mt - e * p.g_mtiles;
+        const int64_t cnt = p.g_counts[e];
+        if ((int64_t)mtl * DR_ROWS >= cnt) return;  // before any copy or barrier
+        m0 = p.g_offsets[e] + (int64_t)mtl * DR_ROWS;
+        mend = p.g_offsets[e] + cnt;
+        wq += e * p.g_wq_stride;
+    }
+    const int64_t n0 = (int64_t)t * DR_NT + 16 * DR_J * w;
+    switch ((min(mend - m0, (int64_t)DR_ROWS) + 15) >> 4) {
+    case 1: dir_tile<1>(p, wq, z, gd.kb_per, n0, m0, mend, bs_mem); break;
+    case 2: dir_tile<2>(p, wq, z, gd.kb_per, n0, m0, mend, bs_mem); break;
+    case 3: dir_tile<3>(p, wq, z, gd.kb_per, n0, m0, mend, bs_mem); break;
+    case 4: dir_tile<4>(p, wq, z, gd.kb_per, n0, m0, mend, bs_mem); break;
+    case 5: dir_tile<5>(p, wq, z, gd.kb_per, n0, m0, mend, bs_mem); break;
+    case 6: dir_tile<6>(p, wq, z, gd.kb_per, n0, m0, mend, bs_mem); break;
+    case 7: dir_tile<7>(p, wq, z, gd.kb_per, n0, m0, mend, bs_mem); break;
+    default: dir_tile<8>(p, wq, z, gd.kb_per, n0, m0, mend, bs_mem); break;
+    }
+}
+
 // The product's weight operands from packed Q4_0 rows: per 16-row tile and
 // block, the MFMA fragment of its codes as f16 (lane (fr, kg) holds the codes
 // of row 16 tile + fr, block b, elements 2 kg + 8 (t & 3) + (t >> 2), t =
@@ -1147,7 +1442,7 @@ int launch_split_rows(const SplitParams &p, hipStream_t s) {
     if (p.M < 0 || p.K <= 0 || p.K % 32 || (p.M > 0 && (!p.x || !p.xh || (!p.xl && !p.sh) || !p.ex)) || p.ldx < p.K ||
         p.ldh < (p.sh ? 2 : 1) * p.K)
         return set_error(GAJE_ERR_INVALID_ARG, "split rows: bad arguments");
-    if (p.sh && (!p.sl || p.ldsum < gemm_bs_sum_cols(p.K) || p.ldh % 8))
+    if (p.sh && (!p.sl || p.ldsum < gemm_bs_sum_cols(p.K) || p.ldh % 64))
         return set_error(GAJE_ERR_INVALID_ARG, "split rows: bad block-sum planes");
     if (p.M == 0) return GAJE_OK;
     const size_t lds = (size_t)p.K * 4;
@@ -1283,6 +1578,32 @@ GemmBsPlan plan_gemm_q4_bs_grouped(int64_t R, int64_t E, int64_t T, int64_t N, i
     return pl;
 }
 
+namespace {
+// The split-K partials of a block-scaled product into its outputs.
+int reduce_splits(const GemmBsParams &p, int splits, hipStream_t s) {
+    GemmQ4Params r{};
+    r.bias = p.bias;
+    r.bias_len = p.bias_len;
+    r.resid = p.resid;
+    r.ldr = p.ldr;
+    r.y = p.y;
+    r.ldy = p.ldy;
+    r.part = p.part;
+    r.M = p.M;
+    r.N = p.N;
+    r.st = p.st;
+    r.layer = p.layer;
+    r.st_a = p.st_a;
+    r.st_b = p.st_b;
+    const int64_t elems = p.M * p.N;
+    int64_t g = (elems + 255) / 256;
+    if (g > 4096) g = 4096;
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)g), dim3(256), 0, s, r, splits);
+    GAJE_HIP_CHECK(hipGetLastError());
+    return GAJE_OK;
+}
+}  // namespace
+
 int launch_gemm_q4_bs(const GemmBsParams &p, const GemmBsPlan &pl, hipStream_t s) {
     if (p.M < 0 || p.N <= 0 || p.nb <= 0 || !p.wf || !p.wsc || p.nbp4 != q4_frag_nbp4(32 * (int64_t)p.nb) ||
         (p.M > 0 && (!p.xh || !p.sh || !p.sl || !p.ex || !p.y || p.ldh < 64 * (int64_t)p.nb ||
@@ -1290,7 +1611,7 @@ int launch_gemm_q4_bs(const GemmBsParams &p, const GemmBsPlan &pl, hipStream_t s
         return set_error(GAJE_ERR_INVALID_ARG, "q4 block-scaled gemm: bad arguments");
     if (p.M > 0 && (!p.mins || p.ldm < gemm_bs_sum_cols(32 * (int64_t)p.nb)))
         return set_error(GAJE_ERR_INVALID_ARG, "q4 block-scaled gemm: no block mins");
-    if ((((uintptr_t)p.xh | (uintptr_t)p.sh | (uintptr_t)p.sl | (uintptr_t)p.mins) & 15) || p.ldh % 8 || p.ldsum % 8 ||
+    if ((((uintptr_t)p.xh | (uintptr_t)p.sh | (uintptr_t)p.sl | (uintptr_t)p.mins) & 15) || p.ldh % 64 || p.ldsum % 8 ||
         p.ldm % 8)
         return set_error(GAJE_ERR_INVALID_ARG, "q4 block-scaled gemm: planes must be 16-byte aligned");
     if (p.M == 0) return GAJE_OK;
@@ -1345,27 +1666,77 @@ int launch_gemm_q4_bs(const GemmBsParams &p, const GemmBsPlan &pl, hipStream_t s
         break;
     }
     GAJE_HIP_CHECK(hipGetLastError());
-    if (pl.splits > 1 && !p.defer_reduce) {
-        GemmQ4Params r{};
-        r.bias = p.bias;
-        r.bias_len = p.bias_len;
-        r.resid = p.resid;
-        r.ldr = p.ldr;
-        r.y = p.y;
-        r.ldy = p.ldy;
-        r.part = p.part;
-        r.M = p.M;
-        r.N = p.N;
-        r.st = p.st;
-        r.layer = p.layer;
-        r.st_a = p.st_a;
-        r.st_b = p.st_b;
-        const int64_t elems = p.M * p.N;
-        int64_t g = (elems + 255) / 256;
-        if (g > 4096) g = 4096;
-        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)g), dim3(256), 0, s, r, pl.splits);
-        GAJE_HIP_CHECK(hipGetLastError());
-    }
+    if (pl.splits > 1 && !p.defer_reduce) return reduce_splits(p, pl.splits, s);
+    return GAJE_OK;
+}
+
+namespace {
+// Splits for `tiles` output tiles: one workgroup per compute unit.
+void dir_splits(GemmBsPlan &pl, int64_t tiles, int64_t M, int64_t N, int64_t K) {
+    const int64_t nb = K / 32, slots = (int64_t)device_cu_count(), S = tiles < slots ? slots / tiles : 1;
+    const int64_t kb = std::max<int64_t>(((nb + S - 1) / S + 3) / 4 * 4, 4);  // splits start on group boundaries
+    pl.kb_per = (int)kb;
+    pl.splits = (int)((nb + kb - 1) / kb);
+    pl.part_floats = pl.splits > 1 ? (int64_t)pl.splits * M * N : 0;
+}
+}  // namespace
+
+GemmBsPlan plan_gemm_q4_dir(int64_t M, int64_t N, int64_t K) {
+    GemmBsPlan pl{};
+    pl.waves = DR_ROWS / BS_WR;
+    pl.mtiles = (int)((M + DR_ROWS - 1) / DR_ROWS);
+    pl.ntiles = (int)((N + DR_NT - 1) / DR_NT);
+    dir_splits(pl, (int64_t)pl.mtiles * pl.ntiles, M, N, K);
+    return pl;
+}
+
+GemmBsPlan plan_gemm_q4_dir_grouped(int64_t R, int64_t E, int64_t T, int64_t N, int64_t K) {
+    GemmBsPlan pl{};
+    pl.waves = DR_ROWS / BS_WR;
+    pl.mtiles = (int)(E * ((T + DR_ROWS - 1) / DR_ROWS));  // a group holds at most T rows; empty tiles return at once
+    pl.ntiles = (int)((N + DR_NT - 1) / DR_NT);
+    // tiles holding rows, at most; and a group's rows cost what they fill
+    dir_splits(pl, ((R + DR_ROWS - 1) / DR_ROWS + E - 1) * pl.ntiles, R, N, K);
+    return pl;
+}
+
+int launch_gemm_q4_dir(const GemmBsParams &p, const GemmBsPlan &pl, hipStream_t s) {
+    if (p.M < 0 || p.N <= 0 || p.nb <= 0 || !p.wq ||
+        (p.M > 0 && (!p.xh || !p.sh || !p.sl || !p.ex || !p.y || p.ldh < 64 * (int64_t)p.nb ||
+                     p.ldsum < gemm_bs_sum_cols(32 * (int64_t)p.nb))))
+        return set_error(GAJE_ERR_INVALID_ARG, "q4 direct gemm: bad arguments");
+    if ((((uintptr_t)p.xh | (uintptr_t)p.sh | (uintptr_t)p.sl) & 15) || p.ldh % 64 || p.ldsum % 8)
+        return set_error(GAJE_ERR_INVALID_ARG, "q4 direct gemm: planes must be 16-byte aligned");
+    if (p.M == 0) return GAJE_OK;
+    const bool grouped = p.g_counts != nullptr;
+    if (grouped && (!p.g_offsets || p.g_groups <= 0 || p.g_groups > MOE_MAX_EXPERTS || p.g_mtiles <= 0 ||
+                    pl.mtiles != (int64_t)p.g_groups * p.g_mtiles || p.g_wq_stride < q4_0_packed_bytes(p.N, 32 * (int64_t)p.nb)))
+        return set_error(GAJE_ERR_INVALID_ARG, "q4 direct gemm: bad groups");
+    // rows read: a grouped tile starts inside the M rows and reads one tile on
+    const int64_t rows_read = grouped ? p.M + (int64_t)p.g_mtiles * DR_ROWS : (int64_t)pl.mtiles * DR_ROWS;
+    if (p.plane_rows < rows_read)
+        return set_error(GAJE_ERR_INVALID_ARG, "q4 direct gemm: the activation plane holds %lld rows, the tiles read %lld",
+                         (long long)p.plane_rows, (long long)rows_read);
+    if (2 * p.plane_rows * p.ldh >= ((int64_t)1 << 32) ||  // the products launch_gemm_q4_bs takes
+        2 * q4_frag_halves(p.N, 32 * (int64_t)p.nb) >= ((int64_t)1 << 32))
+        return set_error(GAJE_ERR_UNSUPPORTED, "q4 direct gemm: operands beyond 4 GiB");
+    if (pl.waves * BS_WR != DR_ROWS || (!grouped && pl.mtiles != (p.M + DR_ROWS - 1) / DR_ROWS) ||
+        pl.ntiles != (p.N + DR_NT - 1) / DR_NT || pl.kb_per % 4 || pl.kb_per <= 0 || (int64_t)pl.splits * pl.kb_per < p.nb ||
+        (int64_t)(pl.splits - 1) * pl.kb_per >= p.nb || (pl.splits > 1 && !p.part))
+        return set_error(GAJE_ERR_INVALID_ARG, "q4 direct gemm: bad plan");
+    if (DR_LDS > max_lds_per_block()) return set_error(GAJE_ERR_UNSUPPORTED, "q4 direct gemm: LDS");
+    GemmBsParams q = p;
+    if (pl.splits == 1) q.part = nullptr;
+    BsGrid gd{};
+    gd.ntiles = pl.ntiles;
+    gd.splits = pl.splits;
+    gd.kb_per = pl.kb_per;
+    const int64_t total = (int64_t)pl.mtiles * pl.splits * pl.ntiles;
+    if (total > (1 << 30)) return set_error(GAJE_ERR_UNSUPPORTED, "q4 direct gemm: too many tiles");
+    gd.total = (int32_t)total;
+    gemm_q4_dir_kernel<<<dim3((unsigned)((total + 7) / 8 * 8)), dim3(64 * DR_W), DR_LDS, s>>>(q, gd);
+    GAJE_HIP_CHECK(hipGetLastError());
+    if (pl.splits > 1 && !p.defer_reduce) return reduce_splits(p, pl.splits, s);
     return GAJE_OK;
 }
 

@@ -319,7 +319,7 @@ struct GemmBsParams {
     int64_t nbp4;            // q4_frag_nbp4(K)
     const uint16_t *mins;    // the rows' block mins as f16, [N][ldm] (launch_q4_operands)
     int64_t ldm;             // >= gemm_bs_sum_cols(K)
-    const uint16_t *xh;      // activation plane [plane_rows][ldh] (hi | lo per block, ldh >= 2K)
+    const uint16_t *xh;      // activation plane (hi | lo per block, by eight rows; ldh >= 2K, % 64)
     int64_t plane_rows;      // rows allocated: >= gemm_bs_plane_rows(M) (rows past M are read, not used)
     const uint16_t *sh, *sl; // block-sum planes [M][ldsum]
     const int *ex;           // [M] activation row exponents
@@ -346,6 +346,10 @@ struct GemmBsParams {
     const int32_t *g_counts, *g_offsets;
     int32_t g_groups, g_mtiles;
     int64_t g_wf_stride, g_wsc_stride, g_mins_stride;
+    // launch_gemm_q4_dir: the packed rows (group e's at wq + e * g_wq_stride)
+    // in place of wf, wsc and mins
+    const uint8_t *wq;
+    int64_t g_wq_stride;
 };
 struct GemmBsPlan {
     int waves;               // 32-row wave tiles per workgroup (2, 4 or 8)
@@ -359,6 +363,11 @@ GemmBsPlan plan_gemm_q4_bs(int64_t M, int64_t N, int64_t K);
 // tiles of T rows; the tile height follows the mean group size).
 GemmBsPlan plan_gemm_q4_bs_grouped(int64_t R, int64_t E, int64_t T, int64_t N, int64_t K);
 int launch_gemm_q4_bs(const GemmBsParams &p, const GemmBsPlan &plan, hipStream_t s);
+// The same product straight from the packed rows, DR_ROWS activation rows a tile.
+constexpr int DR_ROWS = 128;
+GemmBsPlan plan_gemm_q4_dir(int64_t M, int64_t N, int64_t K);
+GemmBsPlan plan_gemm_q4_dir_grouped(int64_t R, int64_t E, int64_t T, int64_t N, int64_t K);
+int launch_gemm_q4_dir(const GemmBsParams &p, const GemmBsPlan &plan, hipStream_t s);
 // Columns of the block-sum planes for a K: K/32 rounded up to a multiple of 32.
 int64_t gemm_bs_sum_cols(int64_t K);
 // The block-scaled product's weight operands from packed Q4_0 rows: per

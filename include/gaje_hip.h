@@ -130,9 +130,10 @@ int gaje_hip_q4_0_gemm(const void *packed, const float *X, const float *bias, in
  * linear/forward.rs:84-92,113-115) to about fp32 accuracy in a different
  * summation order.  `workspace` is 16-byte aligned device memory of at least
  * gaje_hip_q4_0_gemm_mfma_workspace(m, n, k) bytes (-1 for an invalid shape);
- * it also holds the weight rows' codes as f16 MFMA fragments (about two bytes
- * per weight), rebuilt from `packed` on each call; calls that share a
- * workspace must not overlap. */
+ * it has room for the weight rows' codes as f16 MFMA fragments (about two bytes
+ * per weight), rebuilt from `packed` on each call of more than 64 to 96 rows
+ * (fewer run from the packed rows themselves); calls that share a workspace must
+ * not overlap. */
 int64_t gaje_hip_q4_0_gemm_mfma_workspace(int64_t m, int64_t n, int64_t k);
 int gaje_hip_q4_0_gemm_mfma(const void *packed, const float *X, const float *bias, int64_t bias_len,
                             float *Y, int64_t m, int64_t n, int64_t k, void *workspace,
@@ -173,11 +174,11 @@ int gaje_hip_moe_ffn(const float *x, int64_t T, int64_t h, const float *router, 
 /* The same layer over prepared experts: gaje_hip_moe_prepare builds, once per
  * set of experts, the block-scaled product's weight operands (per expert and
  * product: the codes as f16 MFMA fragments, the fragment scales and the dense
- * block mins; about 3.3x the packed bytes) into a caller-owned, 256-byte
+ * block mins, and the packed rows; about 4.3x the packed bytes) into a caller-owned, 256-byte
  * aligned device buffer of gaje_hip_moe_prepared_bytes; gaje_hip_moe_ffn_
  * prepared then runs the layer with one grouped block-scaled product per
- * projection (a row tile per ~64 dispatched rows, no dequantisation per
- * tile).  Routing, composition, accuracy and arguments as gaje_hip_moe_ffn;
+ * projection: over the fragments, or for up to 56 dispatched rows per expert
+ * from the packed rows.  Routing, composition, accuracy and arguments as gaje_hip_moe_ffn;
  * no reference counterpart.  The prepared buffer depends only on the experts'
  * packed rows: prepare again after changing them. */
 int64_t gaje_hip_moe_prepared_bytes(int64_t h, int64_t ffn, int64_t n_expert);

@@ -86,6 +86,20 @@ def test_q4_0_gemm_mfma(hip, O, m, n, k):
     _check(got, _oracle(O, blocks, X, n, k, bias), _exact(O, blocks, X, n, k, bias), f"gemm m={m} n={n} k={k}")
 
 
+# up to 64 rows (96 over weights of 3M and more) the product runs from the packed
+# rows: every count of 16-row units, weight rows about a wave's 32 and a workgroup's
+# 256, groups of one to four blocks at the end, one group and split chains
+@pytest.mark.parametrize("m,n,k", [(1, 1, 32), (2, 31, 128), (16, 32, 160), (17, 33, 4096), (33, 255, 64), (48, 256, 224),
+                                   (49, 257, 1120), (64, 300, 96), (65, 2049, 1536), (81, 3072, 1056), (96, 1537, 8960),
+                                   (97, 2049, 1536)])
+def test_q4_0_gemm_mfma_few_rows(hip, O, m, n, k):
+    blocks = hip.synth.q4_0_tensor(25, f"gemm.few.{n}.{k}", n, k)
+    X = hip.synth.normal(26, f"gemm.few.x.{m}.{k}", m * k).reshape(m, k)
+    bias = hip.synth.normal(27, f"gemm.few.b.{n}", n - n // 3, 0.0, 0.02)
+    got = _run(hip, blocks, X, n, k, bias)
+    _check(got, _oracle(O, blocks, X, n, k, bias), _exact(O, blocks, X, n, k, bias), f"gemm m={m} n={n} k={k}")
+
+
 def test_q4_0_gemm_mfma_row_scales(hip, O):
     # rows of very different magnitude, and weight rows whose scales and mins span
     # f16's range: the per-row power-of-two scaling keeps every row at fp32 accuracy

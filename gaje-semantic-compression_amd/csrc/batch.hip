@@ -6,6 +6,9 @@
 // step and consumed by every sequence's chains.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 #include "device_util.h"
 #include "kernels.h"
@@ -76,29 +79,95 @@ __global__ __launch_bounds__(256) void gemv_batch_f32_kernel(BatchGemvParams p) 
     }
 }
 
-// The same products for a batch of 16, register-blocked over rows: lanes 2r,
-// 2r+1 of a wave own rows r + 32j (j < RB; one 32-row tile each) of the
-// wave's 32*RB rows, chains 0..3 and 4..7 as above, and a workgroup takes VG
-// of the vectors, so each activation quad read from LDS feeds RB rows.
-// VG = 16 (all vectors, when their activations fit LDS): every weight row is
-// read once.  VG = 4: the batch splits over the grid, workgroups b, b+8,
-// b+16, b+24 taking one row block's four vector groups; consecutive
-// workgroups go to the eight XCDs in turn, so the four land on one XCD and its
-// L2 serves the block's rows three times of four (measured: 372 us for the
-// 151936 x 1536 lm_head of batch 16, its L2-to-CU traffic four times the
-// weights; VG = 16 reads them once).
-constexpr int F32B_AHEAD = 4;
-template <int RB, int NT> constexpr int64_t f32b_rows() { return NT / 2 * RB; }  // rows per workgroup
+// The same products on the f32 matrix cores, up to 16 vectors in LDS.  A matrix
+// instruction with one k step is one fma per output (see rows.hip): block b of
+// v_mfma_f32_16x16x1 runs chain 2b (and, in a second one, 2b + 1) of 16 rows x
+// 16 vectors, so a lane's operand is two neighbouring floats of its row's
+// chunk, a wave's load of 16 rows one contiguous 512 bytes, and every output's
+// eight chains end in one lane.  No VALU work per weight, so the weights' bytes
+// bind it: 16 vectors, 151936 x 1536 322 us with one chain per VALU lane -> 159 (5.9
+// TB/s; 32768 rows 106 -> 37), 8 vectors 173 -> 150, 4 vectors 148 -> 146 (32768 rows
+// 45 -> 35); reading 16 chunks ahead instead of 8 the same or 1-2 us more.
+// One workgroup of eight waves per compute unit walks 128-row blocks, each wave
+// 16 rows of them, F32M_AHEAD chunks ahead across the end of a block; rows of x
+// sit K + 4 floats apart (K a multiple of 8: the 16 rows' reads hit all banks).
+constexpr int F32M_AHEAD = 8, F32M_NT = 512, F32M_ROWS = 128;
+typedef float vf2 __attribute__((ext_vector_type(2)));
+typedef float vf16 __attribute__((ext_vector_type(16)));
 
-template <int RB, int VG, int NT>
-__global__ __launch_bounds__(NT) void gemv_batch_f32_rb_kernel(BatchGemvParams p, int64_t nblk) {
-    constexpr int AHEAD = F32B_AHEAD, NVG = 16 / VG;
-    constexpr int64_t F32B_ROWS = f32b_rows<RB, NT>();
+__global__ __launch_bounds__(F32M_NT) void gemv_batch_f32_mfma_kernel(BatchGemvParams p, int nv, int64_t nblk) {
+    extern __shared__ __align__(16) float xs[];  // [16][K + 4], rows past nv zero
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 15, b = lane >> 4;
+    const int64_t K = p.K;
+    const int chunks = (int)(K / 8), K4 = (int)(K / 4);
+    // this wave's 16 rows of block blk (past the padded last tile: the last tile's)
+    const int64_t tiles = (p.N + 31) / 32;
+    auto rows_at = [&](int64_t blk) {
+        const int64_t r = blk * F32M_ROWS + 16 * wave, tile = min(r >> 5, tiles - 1);
+        return (const float *)p.w + tile * K * 32 + (r & 16) * 8 + fr * 8 + 2 * b;
+    };
+    const float *w = rows_at(blockIdx.x);
+    vf2 ring[F32M_AHEAD];
+#pragma unroll
+    for (int u = 0; u < F32M_AHEAD; ++u) ring[u] = __builtin_nontemporal_load((const vf2 *)(w + 256 * min(u, chunks - 1)));
+    for (int i = tid; i < 16 * K4; i += F32M_NT) {
+        const int v = i / K4, q = i - v * K4;
+        const float4 t = v < nv ? *(const float4 *)(p.x + (size_t)v * p.ldx + 4 * q) : make_float4(0.f, 0.f, 0.f, 0.f);
+        *(float4 *)(xs + v * (K + 4) + 4 * q) = t;
+    }
+    __syncthreads();
+    const float *xl = xs + fr * (K + 4) + 2 * b;
+    for (int64_t blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
+        const float *wn = rows_at(blk + gridDim.x < nblk ? blk + gridDim.x : blk);
+        vf16 a0 = {}, a1 = {};
+        auto group = [&](int c0, auto full) {
+            const bool last = c0 + F32M_AHEAD >= chunks;
+            const float *src = last ? wn : w;
+#pragma unroll
+            for (int u = 0; u < F32M_AHEAD; ++u) {
+                const vf2 wv = ring[u];
+                ring[u] = __builtin_nontemporal_load((const vf2 *)(src + 256 * min(last ? u : c0 + F32M_AHEAD + u, chunks - 1)));
+                if (decltype(full)::value || c0 + u < chunks) {
+                    const vf2 x = *(const vf2 *)(xl + 8 * (c0 + u));
+                    a0 = __builtin_amdgcn_mfma_f32_16x16x1f32(wv.x, x.x, a0, 0, 0, 0);
+                    a1 = __builtin_amdgcn_mfma_f32_16x16x1f32(wv.y, x.y, a1, 0, 0, 0);
+                }
+            }
+        };
+        int c0 = 0;
+        for (; c0 + F32M_AHEAD <= chunks; c0 += F32M_AHEAD) group(c0, std::true_type{});
+        if (c0 < chunks) group(c0, std::false_type{});
+        w = wn;
+        // lane (fr, b): vector fr, rows 4b + r; ((s0+s4)+(s1+s5)) + ((s2+s6)+(s3+s7))
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t row = blk * F32M_ROWS + 16 * wave + 4 * b + r;
+            if (row >= p.N || fr >= p.nv) continue;
+            float y = ((a0[r] + a0[8 + r]) + (a1[r] + a1[8 + r])) + ((a0[4 + r] + a0[12 + r]) + (a1[4 + r] + a1[12 + r]));
+            if (row < p.bias_len) y = y + p.bias[row];
+            p.y[(size_t)fr * p.ldy + row] = y;
+        }
+    }
+}
+
+// The same products for a batch of 16 whose activations exceed LDS, register-
+// blocked over rows: lanes 2r, 2r+1 of a wave own rows r + 32j (j < RB; one 32-row
+// tile each) of the wave's 32*RB rows, chains 0..3 and 4..7 as above, and a
+// workgroup takes VG of the vectors, so each activation quad read from LDS feeds
+// RB rows.  The batch splits over the grid, workgroups b, b+8, b+16, b+24 taking
+// one row block's four vector groups; consecutive workgroups go to the eight XCDs
+// in turn, so the four land on one XCD and its L2 serves the block's rows three
+// times of four.
+constexpr int F32B_AHEAD = 4, F32B_RB = 4, F32B_VG = 4, F32B_NT = 256;
+constexpr int64_t F32B_ROWS = F32B_NT / 2 * F32B_RB;  // rows per workgroup
+
+__global__ __launch_bounds__(F32B_NT) void gemv_batch_f32_rb_kernel(BatchGemvParams p, int64_t nblk) {
+    constexpr int AHEAD = F32B_AHEAD, RB = F32B_RB, VG = F32B_VG, NT = F32B_NT;
     extern __shared__ __align__(16) float xs[];  // [VG][K]
     const int b = blockIdx.x;
-    const int64_t blk = NVG == 1 ? (int64_t)b : (((int64_t)(b >> 5) << 3) | (b & 7));
-    if (blk >= nblk) return;  // whole workgroup: the grid is rounded up to 32 (NVG = 4)
-    const int vz = NVG == 1 ? 0 : ((b >> 3) & 3) * VG;
+    const int64_t blk = ((int64_t)(b >> 5) << 3) | (b & 7);
+    if (blk >= nblk) return;  // whole workgroup: the grid is rounded up to 32
+    const int vz = ((b >> 3) & 3) * VG;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t K = p.K, K4 = K / 4;
     for (int64_t i = tid; i < VG * K4; i += NT) {
@@ -419,24 +488,20 @@ int launch_gemv_batch(const BatchGemvParams &p, hipStream_t s) {
     if (p.fmt == FMT_F32) {
         if (!p.f32_tiled || p.K % 8) return set_error(GAJE_ERR_UNSUPPORTED, "batched matvec: f32 rows must be tiled");
         if (p.mode != MODE_STORE) return set_error(GAJE_ERR_UNSUPPORTED, "batched matvec: f32 rows store only");
-        if (nv == 4) return launch_f32<4>(p, s);
-        if (nv == 8) return launch_f32<8>(p, s);
+        // 16 vectors in LDS (K to 2540 or so): the matrix cores, at any count faster
         if ((size_t)16 * p.K * 4 + 1024 <= max_lds_per_block()) {
-            // all 16 vectors in one workgroup of 8 waves (two per SIMD: the
-            // workgroup's LDS allows one per compute unit), one row per lane
-            constexpr int RB = 1, NT = 512;
-            const int64_t nblk = (p.N + f32b_rows<RB, NT>() - 1) / f32b_rows<RB, NT>();
-            hipLaunchKernelGGL((gemv_batch_f32_rb_kernel<RB, 16, NT>), dim3((unsigned)nblk), dim3(NT),
-                               (size_t)16 * p.K * 4, s, p, nblk);
+            const int64_t nblk = (p.N + F32M_ROWS - 1) / F32M_ROWS;
+            hipLaunchKernelGGL(gemv_batch_f32_mfma_kernel, dim3((unsigned)std::min<int64_t>(nblk, device_cu_count())),
+                               dim3(F32M_NT), (size_t)16 * (p.K + 4) * 4, s, p, nv, nblk);
             GAJE_HIP_CHECK(hipGetLastError());
             return GAJE_OK;
         }
+        if (nv == 4) return launch_f32<4>(p, s);
+        if (nv == 8) return launch_f32<8>(p, s);
         if ((size_t)4 * p.K * 4 + 1024 <= max_lds_per_block()) {
-            constexpr int RB = 4, NT = 256;
-            const int64_t nblk = (p.N + f32b_rows<RB, NT>() - 1) / f32b_rows<RB, NT>();
+            const int64_t nblk = (p.N + F32B_ROWS - 1) / F32B_ROWS;
             const int64_t grid = (nblk + 7) / 8 * 32;  // 4 vector groups per block
-            hipLaunchKernelGGL((gemv_batch_f32_rb_kernel<RB, 4, NT>), dim3((unsigned)grid), dim3(NT), (size_t)4 * p.K * 4,
-                               s, p, nblk);
+            hipLaunchKernelGGL(gemv_batch_f32_rb_kernel, dim3((unsigned)grid), dim3(F32B_NT), (size_t)4 * p.K * 4, s, p, nblk);
             GAJE_HIP_CHECK(hipGetLastError());
             return GAJE_OK;
         }

@@ -210,3 +210,23 @@ def test_batch_nan_guard_halts_one_sequence(hip, O, tmp_models):
         hip.GenomicBatch(g2, 2, 64)
     g2.close()
     g.close()
+
+
+@pytest.mark.parametrize("heads,vocab,n_seq", [(3, 293, 16), (5, 33, 9), (3, 32900, 16), (1, 33000, 2), (2, 1025, 5)])
+def test_batch_lm_head_edges(hip, O, tmp_models, heads, vocab, n_seq):
+    """The batched f32 head: vocabularies about its 16, 32 and 128-row tiles and past one 128-row block
+    per compute unit, widths that end a read-ahead group early, 2 to 16 vectors."""
+    cfg = dict(HD64, n_embd=64 * heads, n_head=heads, n_head_kv=1, n_blocks=1, ffn=64, vocab_size=vocab)
+    p = _write(hip, tmp_models / f"batch_head_{heads}_{vocab}.flat", seed=25, **cfg)
+    prompts = _prompts(n_seq, [2], vocab, 26)
+    g = hip.load_genomic_auto(p)
+    g.set_k_wta_ratio(0.0)
+    b = hip.GenomicBatch(g, n_seq, 8)
+    logits = b.feed(_padded(prompts, hip.BATCH_INACTIVE), want_logits=True)
+    out = b.decode_greedy(np.argmax(logits, axis=1).astype(np.uint32), 1)
+    for s, pr in enumerate(prompts):
+        last, toks = _oracle_run(O, p, pr, 2)
+        assert same_bits(logits[s], last), f"sequence {s}"
+        assert int(out[s][0]) == toks[1], f"sequence {s}"
+    b.close()
+    g.close()

@@ -248,7 +248,7 @@ def cpu_baseline(path: str, prompt, seconds: float, threads: int):
 
 def decode_workload(d: str, seed: int, preset: str, prompt_len: int, gen: int, steps: int, warmup: int = 1,
                     kwta: float = 0.0, quant_embed: int = 0, body_format: int = 1, stages=None):
-    """Batch-1 greedy decode: prompt fed token by token once, then `steps` timed runs
+    """Batch-1 greedy decode: prompt fed once, then `steps` timed runs
     of the fixed-length greedy loop from the prompt state (cache rewound each time)."""
     import gaje_hip
     from gaje_hip import ops

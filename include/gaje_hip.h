@@ -174,7 +174,7 @@ int gaje_hip_moe_ffn(const float *x, int64_t T, int64_t h, const float *router, 
 /* The same layer over prepared experts: gaje_hip_moe_prepare builds, once per
  * set of experts, the block-scaled product's weight operands (per expert and
  * product: the codes as f16 MFMA fragments, the fragment scales and the dense
- * block mins, and the packed rows; about 4.3x the packed bytes) into a caller-owned, 256-byte
+ * block mins, and the packed rows; about 4.5x the packed bytes) into a caller-owned, 256-byte
  * aligned device buffer of gaje_hip_moe_prepared_bytes; gaje_hip_moe_ffn_
  * prepared then runs the layer with one grouped block-scaled product per
  * projection: over the fragments, or for up to 56 dispatched rows per expert
@@ -304,8 +304,9 @@ int gaje_hip_get_kwta(const gaje_hip_model *m, float *ratio);
  * cache is an unbounded Vec; this only pre-sizes the device buffers). */
 int gaje_hip_reserve(gaje_hip_model *m, int64_t positions);
 
-/* Token-by-token prefill (nn/llm/forward.rs:229-232): ids[0..n) through
- * forward_core in order; last_logits_host (may be NULL) gets the last
+/* Prefill with the results of the token-by-token loop (nn/llm/forward.rs:229-232:
+ * ids[0..n) through forward_core in order), bit for bit; where the body is Q4_0
+ * the tokens run together as rows.  last_logits_host (may be NULL) gets the last
  * token's K-WTA-filtered logits. */
 int gaje_hip_prefill(gaje_hip_model *m, const uint32_t *ids, int64_t n, float *last_logits_host);
 
@@ -323,9 +324,9 @@ int gaje_hip_prefill_mfma(gaje_hip_model *m, const uint32_t *ids, int64_t n, flo
 /* Batched decode: n_seq (1..16) independent sequences over one model's
  * weights, each with its own KV cache of `capacity` positions, as n_seq
  * GenomicLLM instances (llm/forward.rs:7-64) stepping together.  Every
- * sequence's logits are bit-identical to its own forward_core: the matvecs
- * read each weight row once per step and run every sequence's accumulation
- * chains in the reference order.  Needs Q4_0 body tensors and an f32 lm_head
+ * sequence's logits are bit-identical to its own forward_core: the products
+ * share each weight row between the sequences (and, feeding prompts, their
+ * tokens) and run every accumulation chain in the reference order.  Needs Q4_0 body tensors and an f32 lm_head
  * (GAJE_ERR_UNSUPPORTED otherwise).  No reference function batches
  * sequences. */
 typedef struct gaje_hip_batch gaje_hip_batch;

@@ -1186,6 +1186,10 @@ __device__ __forceinline__ void dir_tile(const GemmBsParams &p, const uint8_t *w
             }
         }
     }
+    // Stages 0 and 1: the counts at enter allow for weight loads issued since a stage's
+    // copies, and theirs has none (one group's less for stage 1).  So everything issued
+    // so far has landed first; the min term's operands, the last of it, were waited for.
+    wait_vmcnt<0>();
 
     // fragment (i, plane P) of lane (fr, kg): row 16 i + fr, chunk (4 P + kg) ^ ((fr >> 1) & 7)
     const uint32_t aoff0 = fr * 128 + 16 * (kg ^ ((fr >> 1) & 7)), aoff1 = aoff0 ^ 64;
@@ -1246,7 +1250,8 @@ __device__ __forceinline__ void dir_tile(const GemmBsParams &p, const uint8_t *w
     };
     // Stage st, a group's first or second half (odd): the copies of stages st + 1 and
     // st + 2 may be in flight, and the weight loads issued since st's copies went out
-    // (after every first half: one group's when st is even, two groups' when odd).
+    // (after every first half: from stage 2 on one group's when st is even, two
+    // groups' when odd; the copies of stages 0 and 1 have landed before the loop).
     auto enter = [&](int st, int slot, auto odd) {
         wait_vmcnt<(DR_S - 2) * CP + (decltype(odd)::value ? 4 : 2) * DR_J>();
         lds_barrier();  // stage st has landed for every wave, and stage st - 1 has been read

@@ -246,7 +246,7 @@ extern "C" int gaje_hip_q4_0_gemm(const void *packed, const float *X, const floa
                                   int64_t m, int64_t n, int64_t k, void *stream) {
     GAJE_TRY(check_dims(n, k));
     if (m < 0 || (m > 0 && (!X || !Y))) return set_error(GAJE_ERR_INVALID_ARG, "bad gemm arguments");
-    if (m >= 2 && n > 0 && k % 32 == 0 && packed && gemv_lds_bytes(k, FMT_Q4_0, false) + 1024 <= max_lds_per_block() &&
+    if (q4_rows_serve(m, n, k) && n > 0 && k % 32 == 0 && packed && gemv_lds_bytes(k, FMT_Q4_0, false) + 1024 <= max_lds_per_block() &&
         !(((uintptr_t)packed | (uintptr_t)X) & 15)) {
         BatchGemvParams p{};
         p.w = (const uint8_t *)packed;

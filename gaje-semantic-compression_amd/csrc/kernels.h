@@ -463,6 +463,19 @@ struct BatchGemvParams {
 int launch_gemv_batch(const BatchGemvParams &p, hipStream_t s);
 // Its Q4_0 products (any nv).
 int launch_q4_rows(const BatchGemvParams &p, hipStream_t s);
+// Whether m plain rows against n weight rows of length k run as row products rather
+// than as m matvecs: from three rows on always.  Two, past the weight rows that the
+// 4-row tiles take (80 per compute unit), use an eighth of a 16-row tile, and two
+// matvecs cost less where the matvec runs near its rate: rows of 2848 and more
+// (21504 x 4096: 33.9 us against 37.7, 24576 x 8960: 58.6 against 78.3; at 2560,
+// 26.2 us against 24.9, and at 32768 x 2816, 36.9 against 34.0, it is the other way),
+// and rows of up to 1024, which it stages, 128 of them per compute unit in a round,
+// where its round is full enough: in the second and later (65536 x 896: 21.9 against
+// 23.6, 151936 x 896: 39.3 against 51.2, 61440 x 512: 13.8 against 15.8; 49152 x 896:
+// 20.8 against 18.5, x 512: 13.1 against 12.5), and in the first for 672 to 992
+// (26624 x 896: 12.2 against 13.3; 24576 x 896: 12.1 against 10.7; 30720 x 512: 9.5
+// against 9.2, x 1024: 15.6 against 14.7).
+bool q4_rows_serve(int64_t m, int64_t n, int64_t k);
 // Activation lanes a batch of n sequences is padded to (4, 8 or 16).
 int batch_lanes(int64_t n);
 // Per-sequence row passes of the batched step.

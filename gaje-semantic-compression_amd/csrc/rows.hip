@@ -445,6 +445,15 @@ int launch_rows4(const BatchGemvParams &p, hipStream_t s) {
 
 }  // namespace
 
+bool q4_rows_serve(int64_t m, int64_t n, int64_t k) {
+    const int64_t cu = device_cu_count();
+    if (m != 2 || n <= 80 * cu) return m >= 2;
+    if (k > 2816) return false;
+    if (k <= 640) return n <= 192 * cu;
+    if (k <= 1024) return n <= 224 * cu && !(k < 1024 && n > 96 * cu && n <= 128 * cu);
+    return true;
+}
+
 int launch_q4_rows(const BatchGemvParams &p, hipStream_t s) {
     if (!p.w || !p.x || !p.y || p.N <= 0 || p.nv <= 0 || p.ldx < p.K || p.ldx % 4 || p.ldy < p.N || p.nb <= 0 ||
         (int64_t)p.nb * 32 != p.K || p.K > (1 << 20) || (((uintptr_t)p.x | (uintptr_t)p.w) & 15) ||
@@ -460,8 +469,11 @@ int launch_q4_rows(const BatchGemvParams &p, hipStream_t s) {
     // a weight row's once for 32 activations (1536 x 17920 x 1536: 834 us
     // against 999 with 16 x 32 tiles; 1536 x 1536 x 8960: 405 against 476), but
     // need enough tiles to fill the chip: at 1064 of them (201 x 9728 x 896)
-    // 53 us against 48, at 560 (64 x 17920 x 1536) 51 against 47.
-    if (((p.nv + 31) / 32) * ((p.N + 63) / 64) >= 9 * (int64_t)device_cu_count() / 2) return launch_rows<32, 64, 2>(p, s);
+    // 53 us against 48, at 560 (64 x 17920 x 1536) 51 against 47.  Up to 16 rows
+    // would leave half of each unused (5 x 151936 x 896: 89 us against 51, x 1536:
+    // 145 against 82).
+    if (p.nv > 16 && ((p.nv + 31) / 32) * ((p.N + 63) / 64) >= 9 * (int64_t)device_cu_count() / 2)
+        return launch_rows<32, 64, 2>(p, s);
     return launch_rows<16, 32, 2>(p, s);
 }
 

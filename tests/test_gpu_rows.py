@@ -55,11 +55,14 @@ def _blocks(rng, n, k):
 
 # rows below, at and past the 4-, 8-, 16- and 32-row tiles; last groups of 1, 2, 3 and 4
 # blocks; one weight row; long sums; then products large enough for the 16 x 32 tiles,
-# and one for the 32 x 64
+# for the 32 x 64, of wide matrices at and past 16 rows, and of two rows on either side
+# of the lines to two matvecs
 @pytest.mark.parametrize("m,n,k", [(2, 1, 32), (3, 37, 96), (4, 8, 128), (5, 200, 160), (8, 33, 576), (9, 64, 896),
                                    (16, 65, 1536), (17, 31, 64), (31, 40, 224), (33, 129, 1152), (4, 24, 8960),
                                    (7, 40, 5888), (64, 16, 4864), (17, 4200, 64), (16, 5153, 1152),
-                                   (33, 2600, 224), (66, 1310, 576), (100, 1000, 32), (70, 24608, 96), (65, 24610, 160)])
+                                   (33, 2600, 224), (66, 1310, 576), (100, 1000, 32), (70, 24608, 96), (65, 24610, 160),
+                                   (16, 73794, 32), (17, 73794, 32), (2, 49152, 64), (2, 49153, 64), (2, 24577, 672),
+                                   (2, 20481, 2816), (2, 20481, 2848), (3, 20481, 2848)])
 def test_row_products_match_the_oracle(hip, O, m, n, k):
     rng = np.random.default_rng(m * 1000003 + n * 1009 + k)
     blocks, X = _blocks(rng, n, k), rng.standard_normal((m, k)).astype(np.float32)

@@ -2530,7 +2530,7 @@ __global__ __launch_bounds__(THREADS) void gemv_q4_chain_kernel(GemvParams p, in
 // 2.4 / L here.  (Reading values that other waves dequantised into LDS costs about
 // 11 cycles a step against 5.7 here, and its LDS footprint ran 1536 x 8960 in two
 // rounds of workgroups: 22.5 us against 11.4 with L = 8.)
-constexpr int BT_LONG = 12;  // packed groups past which it serves (launch_gemv)
+constexpr int BT_SHORT = 12, BT_LONG = 18;  // packed groups past which it serves (baton_ok)
 // Floats of a chain's activations: phases of 32 steps, 4 floats apart in the
 // banks, neighbouring chains 16 apart.
 __host__ __device__ constexpr int64_t baton_stride(int64_t K) {
@@ -2837,12 +2837,16 @@ static bool chain_ok(const GemvParams &p, int64_t npairs) {
 }
 
 // The baton kernel's: long Q4_0 rows without a norm, at most one wave per SIMD of
-// two rows each.  Rows of up to BT_LONG groups stay on the chain kernel (1536 x
-// 1536, 12 groups: 4.1 against 4.4 us; 1000 x 2080, 17 groups: 4.9 against 4.6; 896
-// x 4864: 8.0 against 6.0).
+// two rows each.  The chain kernel keeps rows of up to 12 groups (1536 x 1536: 4.1
+// against 4.4 us) and, while one row per wave leaves it the same workgroups per
+// compute unit, of up to 18 (kernel times: 1024 x 2048 4.66 against 4.82, 1025 x 2176
+// 5.04 against 5.48; past the line 1056 x 2048 4.88 against 4.92, 2048 x 2048 5.26
+// against 5.10, and 1024 x 2336, 19 groups, 5.40 against 5.22; 896 x 4864 8.0 against
+// 6.0 a call).
 static bool baton_ok(const GemvParams &p) {
+    const int64_t G = (p.nb + 3) / 4, cu = device_cu_count();
     return p.fmt == FMT_Q4_0 && (p.mode == MODE_STORE || p.mode == MODE_RESIDUAL) && !p.gnorm && !p.x_out && !p.norm_w &&
-           (p.nb + 3) / 4 > BT_LONG && p.N <= 8 * (int64_t)device_cu_count() && p.K <= (1 << 20) &&
+           (G > BT_LONG || (G > BT_SHORT && 8 * p.N >= 33 * cu)) && p.N <= 8 * cu && p.K <= (1 << 20) &&
            (size_t)baton_stride(p.K) * 32 + 1024 <= max_lds_per_block();
 }
 

@@ -1,6 +1,7 @@
-"""Bit parity of the long-row Q4_0 matvec (rows of more than 12 packed groups, at
-most eight per compute unit) with the CPU oracle: a row's chains run as batons
-handed from lane to lane, fma by fma in the reference's order."""
+"""Bit parity of the long-row Q4_0 matvec (rows of more than 18 packed groups, of more
+than 12 in matrices of 1056 rows and more, at most eight per compute unit) with the CPU
+oracle: a row's chains run as batons handed from lane to lane, fma by fma in the
+reference's order."""
 import numpy as np
 import pytest
 
@@ -21,9 +22,11 @@ def O():
     return oracle
 
 
-# the shortest rows it serves (13 groups, an odd number; the last of 1 and 4 blocks), one
-# and several tiles of phases, one and two rows per wave, ragged numbers of rows
-@pytest.mark.parametrize("n,k", [(1, 1568), (5, 1664), (33, 1760), (1023, 2080), (1025, 2048), (2047, 1632), (7, 4096),
+# the shortest rows it serves and the longest before them (12, 13, 18 and 19 groups; the
+# last of 1 and 4 blocks), one and several tiles of phases, one and two rows per wave,
+# ragged numbers of rows
+@pytest.mark.parametrize("n,k", [(3, 2304), (3, 2336), (1055, 1568), (1056, 1568), (1057, 1536), (1024, 2432),
+                                 (1, 1568), (5, 1664), (33, 1760), (1023, 2080), (1025, 2048), (2047, 1632), (7, 4096),
                                  (1030, 4128), (64, 8960), (1026, 8960)])
 def test_long_rows_match_the_oracle(hip, O, n, k):
     rng = np.random.default_rng(n * 10007 + k)

@@ -312,8 +312,10 @@ GemmWorkspace gemm_workspace(char *base, int64_t m, int64_t n, int64_t k, const 
     off = align256(off + (size_t)(m * w.ldsum) * 2);
     w.part = (float *)(base + off);
     off = align256(off + (size_t)pl.part_floats * 4);
-    // the weight operands, also where the rows run without them: a workspace sized for
-    // more rows serves fewer
+    // the weight operands' room, also where the rows run without them: the size then
+    // differs between numbers of rows by what the activations and partials do.  (It can
+    // fall with m, where the plan has fewer splits: 128 rows of 1536 x 8960 67.0 MB,
+    // 129 rows 53.7.)
     w.mins = (uint16_t *)(base + off);  // [n][ldsum]: the weight rows' block mins
     off = align256(off + (size_t)(n * w.ldsum) * 2);
     w.wf = (uint16_t *)(base + off);    // the weight rows' code fragments and scales
@@ -643,21 +645,39 @@ struct MoeBsWorkspace {
 MoeBsWorkspace moe_bs_workspace(char *base, int64_t T, int64_t h, int64_t ffn, int64_t E) {
     MoeBsWorkspace w{};
     const int64_t R = 2 * T, kmax = std::max(h, ffn);
-    const auto plan = moe_direct(R, E) ? plan_gemm_q4_dir_grouped : plan_gemm_q4_bs_grouped;
-    w.pgu = plan(R, E, T, 2 * ffn, h);
-    w.pdn = plan(R, E, T, h, ffn);
-    const int64_t mt = BS_WR_ROWS * std::max(w.pgu.waves, w.pdn.waves);
-    const int64_t gm = std::max(w.pgu.mtiles, w.pdn.mtiles) / E;  // row tiles per group
-    w.plane_rows = gemm_bs_plane_rows(R + gm * mt);
+    // of r rows: the plans, the plane's rows and the partials
+    auto plans = [&](int64_t r, GemmBsPlan &pgu, GemmBsPlan &pdn, int64_t &plane, int64_t &part) {
+        const auto plan = moe_direct(r, E) ? plan_gemm_q4_dir_grouped : plan_gemm_q4_bs_grouped;
+        pgu = plan(r, E, r / 2, 2 * ffn, h);
+        pdn = plan(r, E, r / 2, h, ffn);
+        const int64_t mt = BS_WR_ROWS * std::max(pgu.waves, pdn.waves);
+        const int64_t gm = std::max(pgu.mtiles, pdn.mtiles) / E;  // row tiles per group
+        plane = gemm_bs_plane_rows(r + gm * mt);
+        part = std::max(pgu.part_floats, pdn.part_floats);
+    };
+    int64_t part;
+    plans(R, w.pgu, w.pdn, w.plane_rows, part);
     w.ldsum = gemm_bs_sum_cols(kmax);
-    // partials: those of fewer rows too (a direct plan's grow up to each multiple of
-    // DR_ROWS), so that a workspace sized for more tokens serves fewer
-    int64_t part = std::max(w.pgu.part_floats, w.pdn.part_floats);
-    for (int64_t r = DR_ROWS; r - DR_ROWS < std::min(R, moe_direct_rows(E)); r += DR_ROWS) {
-        const int64_t Rd = std::min({r, R, moe_direct_rows(E)});
-        part = std::max({part, plan_gemm_q4_dir_grouped(Rd, E, Rd / 2, 2 * ffn, h).part_floats,
-                         plan_gemm_q4_dir_grouped(Rd, E, Rd / 2, h, ffn).part_floats});
-    }
+    // A workspace sized for more tokens serves fewer, whose plans may need more of
+    // either: their needs grow up to each change of plan (the direct line, the tile
+    // heights, a tile more) and can fall there, so those are the rows to look at,
+    // as long as a tile height splits at all.
+    auto fewer = [&](int64_t lo, int64_t hi, int64_t step) {  // plans of (lo, hi] rows change every `step`
+        for (int64_t r = lo; r < std::min(hi, R);) {
+            r = std::min({(r / step + 1) * step, hi, R});
+            GemmBsPlan pgu, pdn;
+            int64_t pl, pa;
+            plans(r, pgu, pdn, pl, pa);
+            w.plane_rows = std::max(w.plane_rows, pl);
+            part = std::max(part, pa);
+            if (pgu.splits == 1 && pdn.splits == 1) break;  // (and the plane grows with the rows)
+        }
+    };
+    const int64_t d = moe_direct_rows(E);
+    fewer(0, d, DR_ROWS);
+    fewer(d, 32 * E, 2 * BS_WR_ROWS);
+    fewer(std::max(d, 32 * E), 96 * E, 4 * BS_WR_ROWS);
+    fewer(96 * E, R, 8 * BS_WR_ROWS);
     size_t off = 0;
     auto take = [&](size_t bytes) {
         char *p = base + off;

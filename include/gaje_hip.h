@@ -133,7 +133,8 @@ int gaje_hip_q4_0_gemm(const void *packed, const float *X, const float *bias, in
  * it has room for the weight rows' codes as f16 MFMA fragments (about two bytes
  * per weight), rebuilt from `packed` on each call of more than 64 to 96 rows
  * (fewer run from the packed rows themselves); calls that share a workspace must
- * not overlap. */
+ * not overlap.  The size does not always grow with m: a workspace for several m
+ * takes the largest of their sizes. */
 int64_t gaje_hip_q4_0_gemm_mfma_workspace(int64_t m, int64_t n, int64_t k);
 int gaje_hip_q4_0_gemm_mfma(const void *packed, const float *X, const float *bias, int64_t bias_len,
                             float *Y, int64_t m, int64_t n, int64_t k, void *workspace,
@@ -177,9 +178,10 @@ int gaje_hip_moe_ffn(const float *x, int64_t T, int64_t h, const float *router, 
  * block mins, and the packed rows; about 4.5x the packed bytes) into a caller-owned, 256-byte
  * aligned device buffer of gaje_hip_moe_prepared_bytes; gaje_hip_moe_ffn_
  * prepared then runs the layer with one grouped block-scaled product per
- * projection: over the fragments, or for up to 56 dispatched rows per expert
- * from the packed rows.  Routing, composition, accuracy and arguments as gaje_hip_moe_ffn;
- * no reference counterpart.  The prepared buffer depends only on the experts'
+ * projection: over the fragments, or for up to 56 dispatched rows per
+ * expert from the packed rows.  A workspace for T tokens serves fewer.
+ * Routing, composition, accuracy and arguments as gaje_hip_moe_ffn; no reference
+ * counterpart.  The prepared buffer depends only on the experts'
  * packed rows: prepare again after changing them. */
 int64_t gaje_hip_moe_prepared_bytes(int64_t h, int64_t ffn, int64_t n_expert);
 int gaje_hip_moe_prepare(const void *const *gate_up, const void *const *down, int64_t h, int64_t ffn,

@@ -622,11 +622,20 @@ MoePrepared moe_prepared(char *base, int64_t h, int64_t ffn, int64_t E) {
     return w;
 }
 
-// Whether R dispatched rows over E experts run straight from the packed rows: up
-// to 56 per expert (8 x 4096, h 1536: 16 tokens 127 -> 86 us a layer, 128 tokens 136
-// -> 117, 192 tokens 160 -> 128; 256 tokens 157.6 -> 162, 512 tokens 253 -> 271).
-constexpr int64_t moe_direct_rows(int64_t E) { return 56 * E; }
-bool moe_direct(int64_t R, int64_t E) { return R <= moe_direct_rows(E); }
+// Whether R dispatched rows over E experts run straight from the packed rows: up to
+// 32 per expert, 16 where an expert's matrices are small (h * ffn below 4M).  The lines
+// hold for uneven loads, which the host does not see: the direct product gives a tile
+// of a busy expert's rows to one workgroup and has the lower rate on many rows.  Packed
+// rows against fragments, us a layer, even loads and ones whose busiest expert has
+// about twice the mean:
+//   8 x 4096, h 1536   32 per expert  115 / 132, 141 / 191;  40  118 / 150, 153 / 150;
+//                      52  137 / 152, 203 / 152
+//   4 x 4096, h 2048   32   95 / 112, 102 / 113;  36  122 / 114, 132 / 114
+//   16 x 2048, h 2048  32  164 / 179, 216 / 220;  36  177 / 214, 257 / 214
+//   8 x 2048, h 1024   16   64 / 76, 72 / 77;  24  71 / 78, 90 / 79;  28  82 / 76
+//   8 x 2048, h 512    16   58 / 60, 63 / 61;  24  56 / 61, 69 / 62
+constexpr int64_t moe_direct_rows(int64_t h, int64_t ffn, int64_t E) { return (h * ffn >= (int64_t)1 << 22 ? 32 : 16) * E; }
+bool moe_direct(int64_t R, int64_t h, int64_t ffn, int64_t E) { return R <= moe_direct_rows(h, ffn, E); }
 
 // Workspace of gaje_hip_moe_ffn_prepared: the routing, the block-scaled
 // activation planes of the dispatched rows, the two products' results and
@@ -647,7 +656,7 @@ MoeBsWorkspace moe_bs_workspace(char *base, int64_t T, int64_t h, int64_t ffn, i
     const int64_t R = 2 * T, kmax = std::max(h, ffn);
     // of r rows: the plans, the plane's rows and the partials
     auto plans = [&](int64_t r, GemmBsPlan &pgu, GemmBsPlan &pdn, int64_t &plane, int64_t &part) {
-        const auto plan = moe_direct(r, E) ? plan_gemm_q4_dir_grouped : plan_gemm_q4_bs_grouped;
+        const auto plan = moe_direct(r, h, ffn, E) ? plan_gemm_q4_dir_grouped : plan_gemm_q4_bs_grouped;
         pgu = plan(r, E, r / 2, 2 * ffn, h);
         pdn = plan(r, E, r / 2, h, ffn);
         const int64_t mt = BS_WR_ROWS * std::max(pgu.waves, pdn.waves);
@@ -673,7 +682,7 @@ MoeBsWorkspace moe_bs_workspace(char *base, int64_t T, int64_t h, int64_t ffn, i
             if (pgu.splits == 1 && pdn.splits == 1) break;  // (and the plane grows with the rows)
         }
     };
-    const int64_t d = moe_direct_rows(E);
+    const int64_t d = moe_direct_rows(h, ffn, E);
     fewer(0, d, DR_ROWS);
     fewer(d, 32 * E, 2 * BS_WR_ROWS);
     fewer(std::max(d, 32 * E), 96 * E, 4 * BS_WR_ROWS);
@@ -816,7 +825,7 @@ extern "C" int gaje_hip_moe_ffn_prepared(const float *x, int64_t T, int64_t h, c
         p.g_groups = (int32_t)n_expert;
         p.g_mtiles = (int32_t)(pl.mtiles / n_expert);
         p.defer_reduce = i == 1 && pl.splits > 1;  // down: the combine sums its partials
-        return moe_direct(R, n_expert) ? launch_gemm_q4_dir(p, pl, s) : launch_gemm_q4_bs(p, pl, s);
+        return moe_direct(R, h, ffn, n_expert) ? launch_gemm_q4_dir(p, pl, s) : launch_gemm_q4_bs(p, pl, s);
     };
     GAJE_TRY(gemm(0, w.pgu, 2 * ffn, h, w.GU));
     // swiglu of every dispatched row into the planes, then down

@@ -178,7 +178,7 @@ int gaje_hip_moe_ffn(const float *x, int64_t T, int64_t h, const float *router, 
  * block mins, and the packed rows; about 4.5x the packed bytes) into a caller-owned, 256-byte
  * aligned device buffer of gaje_hip_moe_prepared_bytes; gaje_hip_moe_ffn_
  * prepared then runs the layer with one grouped block-scaled product per
- * projection: over the fragments, or for up to 56 dispatched rows per
+ * projection: over the fragments, or for up to 16 to 32 dispatched rows per
  * expert from the packed rows.  A workspace for T tokens serves fewer.
  * Routing, composition, accuracy and arguments as gaje_hip_moe_ffn; no reference
  * counterpart.  The prepared buffer depends only on the experts'

@@ -121,10 +121,12 @@ def test_moe_ffn_prepared(hip, O, T, h, ffn, E, skew):
     assert err <= TOL
 
 
-# up to 56 dispatched rows per expert the products run from the packed rows: either
-# side of the line, a skewed load of several row tiles in one expert, ragged widths
-# and groups
-@pytest.mark.parametrize("T,h,ffn,E,skew", [(2, 32, 32, 2, 0.0), (56, 160, 224, 2, 0.0), (57, 160, 224, 2, 0.0),
+# up to 32 dispatched rows per expert (16 of matrices below 4M) the products run from the
+# packed rows: either side of the lines, a skewed load of several row tiles in one
+# expert, ragged widths and groups
+@pytest.mark.parametrize("T,h,ffn,E,skew", [(16, 160, 224, 2, 0.0), (17, 160, 224, 2, 0.0), (32, 2048, 2048, 2, 0.0),
+                                            (33, 2048, 2048, 2, 0.0), (128, 96, 160, 16, 6.0), (96, 2048, 2080, 6, 6.0),
+                                            (2, 32, 32, 2, 0.0), (56, 160, 224, 2, 0.0), (57, 160, 224, 2, 0.0),
                                             (200, 288, 96, 8, 6.0), (448, 96, 160, 16, 6.0), (449, 96, 160, 16, 6.0),
                                             (17, 1536, 1120, 3, 0.0)])
 def test_moe_ffn_prepared_few_rows(hip, O, T, h, ffn, E, skew):

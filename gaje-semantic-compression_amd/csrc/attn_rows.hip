@@ -179,14 +179,25 @@ __global__ __launch_bounds__(HD * 4) void attn_rows_kernel(AttnParams p) {
 
 }  // namespace
 
-bool attn_rows_serves(int head_dim, int64_t kv_cap, int64_t ctx) {
+static bool attn_rows_fits(int head_dim, int64_t kv_cap, int64_t ctx) {
     return (head_dim == 64 || head_dim == 128) && kv_cap % 16 == 0 && (size_t)ar_floats(ctx) * 4 + 2048 <= max_lds_per_block();
+}
+
+// Against one workgroup per (head, row), which costs by the round of workgroups, a
+// tile costs a longer serial pass whatever its rows: it takes about two rounds, three
+// at 64 dimensions over a long context, to pay.  Prompts of n tokens over a cache, us
+// (8 layers), tiles against rows: 12 heads of 128: 32 tokens at 1024 1358 / 1264, 48
+// 1552 / 1623; 14 of 64: 32 at 1024 1001 / 830, 48 1087 / 1041, 64 1127 / 1209, 48 at 0
+// 723 / 767; 9 of 64: 2 at 2200 1124 / 649, 64 1336 / 1186, 96 1380 / 1453.
+bool attn_rows_serves(int head_dim, int n_head, int64_t kv_cap, int64_t ctx, int64_t rows) {
+    const int64_t rounds = ctx <= 64 ? 1 : head_dim == 128 || ctx <= 256 ? 2 : 3;
+    return rows * n_head >= rounds * device_cu_count() && attn_rows_fits(head_dim, kv_cap, ctx);
 }
 
 int launch_attn_rows(const AttnParams &p, hipStream_t s) {
     if (!p.q || !p.k_cache || !p.v_cache || !p.out || !p.seq_pos || !p.tiles || p.n_tiles <= 0 || p.n_head <= 0 ||
         p.n_head_kv <= 0 || p.n_head % p.n_head_kv || p.kv_cap <= 0 || p.kv_head_stride != p.kv_cap * p.head_dim ||
-        p.ctx <= 0 || p.ctx > p.kv_cap || !attn_rows_serves(p.head_dim, p.kv_cap, p.ctx) ||
+        p.ctx <= 0 || p.ctx > p.kv_cap || !attn_rows_fits(p.head_dim, p.kv_cap, p.ctx) ||
         (((uintptr_t)p.k_cache | (uintptr_t)p.v_cache) & 15) || p.seq_kv_stride % 4 ||
         (int64_t)p.n_tiles * p.n_head > INT32_MAX)
         return set_error(GAJE_ERR_INVALID_ARG, "attention rows: bad arguments");

@@ -193,9 +193,10 @@ struct AttnParams {
 };
 int launch_attention(const AttnParams &p, hipStream_t s);
 // Rows of several tokens per sequence (a prompt's): tiles of up to
-// ATTN_ROWS_TILE consecutive tokens, where attn_rows_serves.
+// ATTN_ROWS_TILE consecutive tokens, where attn_rows_serves (rows of the pass, its
+// longest context).
 constexpr int ATTN_ROWS_TILE = 16;
-bool attn_rows_serves(int head_dim, int64_t kv_cap, int64_t ctx);
+bool attn_rows_serves(int head_dim, int n_head, int64_t kv_cap, int64_t ctx, int64_t rows);
 int launch_attn_rows(const AttnParams &p, hipStream_t s);
 size_t attention_lds_bytes(int head_dim, int64_t max_ctx);
 // Largest KV capacity whose scores fit the attention kernel's LDS buffer.

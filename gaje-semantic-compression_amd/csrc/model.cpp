@@ -1162,7 +1162,7 @@ int rows_blocks(gaje_hip_model *m, const RowPass &c) {
         ap.n_seq = (int32_t)R;
         ap.seq_nan = b.nan_codes;
         ap.layer = li;
-        if (c.tiles && attn_rows_serves((int)m->hd, c.cap, c.max_ctx)) {
+        if (c.tiles && attn_rows_serves((int)m->hd, (int)m->n_head, c.cap, c.max_ctx, R)) {
             ap.tiles = c.tiles;
             ap.n_tiles = c.n_tiles;
             ap.ctx = c.max_ctx;

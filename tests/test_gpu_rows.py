@@ -107,12 +107,16 @@ def _oracle(O, path, kwta):
 
 
 # prompts of two tokens, of a few tiles, and of more rows than one pass takes, on an
-# empty cache and after it; the last one's second prompt has contexts past what
-# the rows' attention holds in LDS
+# empty cache and after it; `long`'s second prompt has contexts past what the rows'
+# attention holds in LDS; then numbers of rows and contexts on either side of the lines
+# between that attention (whole tiles, ragged ones, on a cache) and one row at a time
 @pytest.mark.parametrize("name,cfg,kwta,lengths", [("tiny", TINY, 0.0, [2, 33, 1]), ("tiny", TINY, 0.5, [19]),
                                                    ("hd64", HD64, 0.0, [65, 3]), ("hd128", HD128, 0.0, [130]),
                                                    ("gnorm", GNORM_MODEL, 0.0, [17]), ("tiny", TINY, 0.0, [2060]),
-                                                   ("long", LONG, 0.0, [2490, 20])])
+                                                   ("long", LONG, 0.0, [2490, 20]),
+                                                   ("hd64", HD64, 0.0, [63, 1, 64, 64]), ("hd64", HD64, 0.0, [64, 127]),
+                                                   ("hd64", HD64, 0.0, [128, 128, 192, 191]),
+                                                   ("hd128", HD128, 0.0, [171, 170, 175, 186])])
 def test_prompt_rows_match_the_oracle(hip, O, tmp_models, name, cfg, kwta, lengths):
     p = _write(hip, tmp_models, name, cfg)
     g, r = hip.load_genomic_auto(p), _oracle(O, p, kwta)

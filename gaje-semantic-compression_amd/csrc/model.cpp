@@ -1747,7 +1747,7 @@ int batch_feed_rows(gaje_hip_batch *b, const uint32_t *ids, int64_t n, int64_t i
                     seq.push_back((uint32_t)q);
                 }
             nt += attn_tiles(tiles, row0, (int64_t)tok.size() - row0);
-            max_ctx = std::max<int64_t>(max_ctx, end[q]);
+            if ((int64_t)tok.size() > row0) max_ctx = std::max<int64_t>(max_ctx, end[q]);
         }
         const int64_t R = (int64_t)tok.size();
         if (R == 0) continue;

@@ -174,3 +174,27 @@ def test_batch_rows_with_gaps_and_a_guard(hip, O, tmp_models):
         assert b.cache_len(2) == 0
         b.close()
     g.close()
+
+
+def test_batch_rows_past_the_tiled_attention(hip, O, tmp_models):
+    """Two sequences in one pass, one with contexts past what the tiled attention holds
+    in LDS (one row at a time, each in its own cache); then a prompt of whole tiles for
+    the short one while the long one is idle."""
+    p = _write(hip, tmp_models, "long", LONG)
+    g = hip.load_genomic_auto(p)
+    g.set_k_wta_ratio(0.0)
+    X, rng = hip.BATCH_INACTIVE, np.random.default_rng(12)
+    b, r = hip.GenomicBatch(g, 2, 2800), [_oracle(O, p, 0.0) for _ in range(2)]
+    for lengths in ((2490, 3), (20, 17), (0, 257)):
+        n = max(lengths)
+        ids = np.full((2, n), X, np.uint32)
+        for s, k in enumerate(lengths):
+            ids[s, n - k:] = rng.integers(0, LONG["vocab_size"], k)
+        logits = b.feed(ids, want_logits=True)
+        for s, k in enumerate(lengths):
+            for t in ids[s, n - k:]:
+                want = r[s].forward_core(int(t))
+            assert k == 0 or _same(logits[s], want), (lengths, s)
+    assert (b.cache_len(0), b.cache_len(1)) == (2510, 277)
+    b.close()
+    g.close()

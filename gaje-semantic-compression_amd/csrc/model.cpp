@@ -28,6 +28,7 @@
 #include "common.h"
 #include "flat.h"
 #include "kernels.h"
+#include "rows_fit.h"
 
 namespace gaje {
 namespace {
@@ -1044,13 +1045,15 @@ bool rows_supported(const gaje_hip_model *m) {
 
 // Owner: gaje_hip_model or gaje_hip_batch (alloc and release).
 template <class Owner>
-int rows_reserve(Owner *o, const gaje_hip_model *m, RowBufs &b, int64_t rows) {
-    if (rows <= b.rows) return GAJE_OK;
-    GAJE_HIP_CHECK(hipStreamSynchronize(m->stream));
+void rows_release(Owner *o, RowBufs &b) {
     for (void *p : {(void *)b.H, (void *)b.XN, (void *)b.QKV, (void *)b.Q, (void *)b.ATT, (void *)b.GU, (void *)b.ACT,
                     (void *)b.ids, (void *)b.nan_codes})
         if (p) o->release(p);
     b = RowBufs();
+}
+
+template <class Owner>
+int rows_reserve(Owner *o, const gaje_hip_model *m, RowBufs &b, int64_t rows) {
     const Layer &L0 = m->layers[0];
     GAJE_TRY(o->alloc(&b.H, (size_t)(rows * m->n_embd)));
     GAJE_TRY(o->alloc(&b.XN, (size_t)(rows * m->n_embd)));
@@ -1063,6 +1066,23 @@ int rows_reserve(Owner *o, const gaje_hip_model *m, RowBufs &b, int64_t rows) {
     GAJE_TRY(o->alloc(&b.nan_codes, (size_t)rows));
     b.rows = rows;
     return GAJE_OK;
+}
+
+// Rows of a pass over `want` rows that b has room for, after growing it: want (at most
+// ROWS_CHUNK), fewer where the device's memory does not hold that many, 0 where it
+// holds no more than one, when the tokens go one step at a time instead.
+template <class Owner>
+int64_t rows_room(Owner *o, const gaje_hip_model *m, RowBufs &b, int64_t want) {
+    want = std::min(want, ROWS_CHUNK);
+    if (want > b.rows && hipStreamSynchronize(m->stream) != hipSuccess) return 0;  // (the steps report it)
+    return rows_fit(want, b.rows, ROWS_CHUNK, [&](int64_t rows) {
+        rows_release(o, b);
+        if (rows_reserve(o, m, b, rows) == GAJE_OK) return true;
+        rows_release(o, b);
+        (void)hipGetLastError();  // (the next launch's check would report it)
+        clear_error();
+        return false;
+    });
 }
 
 BatchGemvParams rows_gemv(const DevLinear &D, const float *x, int64_t ldx, float *y, int64_t ldy, int64_t rows,
@@ -1218,15 +1238,14 @@ int prefill_steps(gaje_hip_model *m, const uint32_t *ids, int64_t n, DevState &s
     return s.halted || s.nan_code != NAN_NONE ? nan_error(s) : GAJE_OK;
 }
 
-// n tokens (at most ROWS_CHUNK) as rows of one pass at positions m->pos..: the
+// n tokens (at most m->rb.rows) as rows of one pass at positions m->pos..: the
 // keys and values appended, the rows' hidden states in m->rb.H.  `clean` tells
 // whether every guard held; if one fired nothing is committed (the cache length
 // stays), and the caller runs the tokens one by one, which stops at the token
 // that the reference stops at.
 int prefill_rows(gaje_hip_model *m, const uint32_t *ids, int64_t n, bool &clean) {
-    RowBufs &b = m->rb;
+    const RowBufs &b = m->rb;
     hipStream_t s = m->stream;
-    GAJE_TRY(rows_reserve(m, m, b, n));
     std::vector<uint32_t> up((size_t)(2 * n));
     for (int64_t i = 0; i < n; ++i) {
         up[i] = ids[i];
@@ -1267,9 +1286,9 @@ extern "C" int gaje_hip_prefill(gaje_hip_model *m, const uint32_t *ids, int64_t 
     if (n == 0) return GAJE_OK;
     GAJE_TRY(reserve_ctx(m, m->pos + n));
     DevState s;
-    const bool rows = n > 1 && !m->profile && rows_supported(m);
+    const int64_t rows = n > 1 && !m->profile && rows_supported(m) ? rows_room(m, m, m->rb, n) : 0;
     for (int64_t c0 = 0; c0 < n;) {
-        const int64_t P = rows ? std::min(ROWS_CHUNK, n - c0) : n;
+        const int64_t P = rows ? std::min(rows, n - c0) : n;
         bool clean = false;
         if (rows) GAJE_TRY(prefill_rows(m, ids + c0, P, clean));
         if (!clean) {
@@ -1725,13 +1744,13 @@ int batch_sync(gaje_hip_batch *b, int32_t *status) {
 
 // Steps i0 .. i1 - 1 of a feed (ids on the host and in b->ids, [seq][n]) as
 // rows of shared passes: every running sequence's tokens at once, up to
-// ROWS_CHUNK rows a pass.  Nothing of a pass in which a guard fired is
+// `room` rows a pass (at least one per sequence).  Nothing of a pass in which a guard fired is
 // committed: its steps run one at a time instead, where the sequence halts at
 // its own token and the others go on.
-int batch_feed_rows(gaje_hip_batch *b, const uint32_t *ids, int64_t n, int64_t i0, int64_t i1) {
+int batch_feed_rows(gaje_hip_batch *b, const uint32_t *ids, int64_t n, int64_t i0, int64_t i1, int64_t room) {
     gaje_hip_model *m = b->m;
     hipStream_t s = m->stream;
-    const int64_t per = std::max<int64_t>(1, ROWS_CHUNK / b->nseq);
+    const int64_t per = room / b->nseq;
     std::vector<uint32_t> up;
     for (int64_t c0 = i0; c0 < i1; c0 += per) {
         const int64_t c1 = std::min(i1, c0 + per);
@@ -1751,7 +1770,6 @@ int batch_feed_rows(gaje_hip_batch *b, const uint32_t *ids, int64_t n, int64_t i
         }
         const int64_t R = (int64_t)tok.size();
         if (R == 0) continue;
-        GAJE_TRY(rows_reserve(b, m, b->rb, R));
         up.assign(tok.begin(), tok.end());
         up.insert(up.end(), pos.begin(), pos.end());
         up.insert(up.end(), seq.begin(), seq.end());
@@ -1930,8 +1948,9 @@ extern "C" int gaje_hip_batch_feed(gaje_hip_batch *b, const uint32_t *ids, int64
     // The last step gives the logits; the steps before it run as rows, from two on (one is
     // a step without its head, but waits for the guards: 4 sequences of SmolLM2-135M
     // widths, two tokens each, 943 us as two steps and 971 that way)
-    if (n > 2 && rows_supported(m)) {
-        GAJE_TRY(batch_feed_rows(b, ids, n, 0, n - 1));
+    const int64_t room = n > 2 && rows_supported(m) ? rows_room(b, m, b->rb, b->nseq * (n - 1)) : 0;
+    if (room >= b->nseq) {
+        GAJE_TRY(batch_feed_rows(b, ids, n, 0, n - 1, room));
         GAJE_TRY(batch_enqueue_step(b, b->ids, n, n - 1, nullptr, false));
     } else {
         for (int64_t i = 0; i < n; ++i) GAJE_TRY(batch_enqueue_step(b, b->ids, n, i, nullptr, false));

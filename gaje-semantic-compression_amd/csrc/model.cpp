@@ -1941,6 +1941,7 @@ extern "C" int gaje_hip_batch_feed(gaje_hip_batch *b, const uint32_t *ids, int64
     const size_t need = (size_t)(b->nseq * n);
     if ((int64_t)need > b->ids_cap) {
         if (b->ids) b->release(b->ids);
+        b->ids_cap = 0;
         GAJE_TRY(b->alloc(&b->ids, need));
         b->ids_cap = (int64_t)need;
     }
@@ -1975,6 +1976,7 @@ extern "C" int gaje_hip_batch_decode_greedy(gaje_hip_batch *b, const uint32_t *f
     const size_t need = (size_t)(b->nseq * n);
     if ((int64_t)need > b->out_cap) {
         if (b->out) b->release(b->out);
+        b->out_cap = 0;
         GAJE_TRY(b->alloc(&b->out, need));
         b->out_cap = (int64_t)need;
     }
@@ -2003,10 +2005,11 @@ extern "C" int gaje_hip_decode_greedy(gaje_hip_model *m, uint32_t first_token, i
     if (n == 0) return GAJE_OK;
     GAJE_TRY(reserve_ctx(m, m->pos + n));
     if (n > m->out_cap) {
+        drop_graph(m);  // (it writes the old buffer)
         m->release(m->out_tokens);
-        m->out_cap = n;
+        m->out_cap = 0;
         GAJE_TRY(m->alloc(&m->out_tokens, (size_t)n));
-        drop_graph(m);
+        m->out_cap = n;
     }
     if (!m->profile) GAJE_TRY(ensure_graph(m));
     GAJE_TRY(launch_state_set(m->st, (int32_t)m->pos, first_token, (int32_t)m->out_cap, 0, 1, m->stream));

@@ -17,6 +17,8 @@
 // independent MFMAs, against 67 for v_fma_f32).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "common.h"
 #include "device_util.h"
 #include "kernels.h"
@@ -272,13 +274,24 @@ __global__ __launch_bounds__(TN * 8) void rows_q4_kernel(BatchGemvParams p, int6
     }
 }
 
+// A launch holds at most 2^32 - 1 threads in a dimension, so a product of more tiles
+// goes in several (33.5M activation rows x 64).
 template <int TM, int TN, int S>
 int launch_rows(const BatchGemvParams &p, hipStream_t s) {
     const int64_t ntiles = (p.N + TN - 1) / TN, mtiles = (p.nv + TM - 1) / TM;
-    const int64_t grid = (ntiles + 7) / 8 * 8 * mtiles;
-    if (grid > INT32_MAX) return set_error(GAJE_ERR_UNSUPPORTED, "q4_0 rows: %lld tiles", (long long)grid);
-    hipLaunchKernelGGL((rows_q4_kernel<TM, TN, S>), dim3((unsigned)grid), dim3(TN * 8), rq_lds(TM, TN, S), s, p, ntiles, mtiles);
-    GAJE_HIP_CHECK(hipGetLastError());
+    const int64_t ngrid = (ntiles + 7) / 8 * 8, most = (int64_t)UINT32_MAX / (TN * 8) / ngrid;  // row tiles a launch takes
+    if (most < 1) return set_error(GAJE_ERR_UNSUPPORTED, "q4_0 rows: %lld weight rows", (long long)p.N);
+    for (int64_t t = 0; t < mtiles; t += most) {
+        BatchGemvParams q = p;
+        const int64_t n = std::min(most, mtiles - t), m0 = t * TM;
+        q.x += m0 * p.ldx;
+        q.y += m0 * p.ldy;
+        if (q.nan_codes) q.nan_codes += m0;
+        q.nv = std::min(p.nv - m0, n * TM);
+        hipLaunchKernelGGL((rows_q4_kernel<TM, TN, S>), dim3((unsigned)(ngrid * n)), dim3(TN * 8), rq_lds(TM, TN, S), s, q,
+                           ntiles, n);
+        GAJE_HIP_CHECK(hipGetLastError());
+    }
     return GAJE_OK;
 }
 

@@ -81,6 +81,29 @@ def test_row_products_match_the_oracle(hip, O, m, n, k):
         assert _same(got[r], L.forward_core(X[r])), f"row {r}"
 
 
+def test_row_products_past_one_launch(hip, O):
+    """More tiles than one launch holds (1048575 of 32 rows x 64): 33.6M activation rows, of
+    which those at the ends and about the line are compared."""
+    from gaje_hip._lib import check, lib
+    line, n, k = 1048575 * 32, 64, 32
+    m = line + 65
+    rng = np.random.default_rng(3)
+    blocks = _blocks(rng, n, k)
+    ops = hip.ops
+    X, Y = ops.DeviceBuffer(m * k * 4), ops.DeviceBuffer(m * n * 4)
+    parts = {r0: rng.standard_normal((c, k)).astype(np.float32) for r0, c in ((0, 5), (line - 33, 70), (m - 20, 20))}
+    for r0, x in parts.items():
+        X.write(x, r0 * k * 4)
+    ops.q4_0_gemm(ops.q4_0_upload(blocks, n, k), X, Y, m, n, k)
+    ops.synchronize()
+    L = O.GenomicLinear(blocks, b"", None, n, k, np.zeros(0, np.float32), 4)
+    for r0, x in parts.items():
+        got = np.empty((len(x), n), np.float32)
+        check(lib().gaje_hip_memcpy_d2h(got.ctypes.data, Y.ptr + r0 * n * 4, got.nbytes))
+        for r in range(len(x)):
+            assert _same(got[r], L.forward_core(x[r])), f"row {r0 + r}"
+
+
 def _write(hip, tmp_models, name, cfg):
     if cfg is GNORM_MODEL:
         return write_genomic_norm_model(str(tmp_models), seed=17)

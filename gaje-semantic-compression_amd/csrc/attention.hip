@@ -735,102 +735,6 @@ __global__ __launch_bounds__(WIDE) void attn_batch_wide(AttnParams p) {
     }
 }
 
-// Batched decode (several sequences per launch): one workgroup per (query
-// head, sequence) computes the head's scores once; after the softmax each
-// output dimension's chain runs in its own thread (threads 0..HD-1), reading
-// its V row straight from memory (the row is contiguous and the loads run
-// ahead of the adds).  Same rounding sequence as attn_decode_wide.
-template <int HD>
-__global__ __launch_bounds__(THREADS) void attn_decode_batch(AttnParams p) {
-    extern __shared__ __align__(16) float smem[];  // chain_row(cap): scores, exponentials, weights
-    __shared__ float red[THREADS / WAVE];
-    __shared__ float inv_slot;
-    __shared__ uint64_t tab[32];
-    const int tid = threadIdx.x;
-    const int h = blockIdx.x, z = blockIdx.z;
-    const int pos = p.seq_pos[z];
-    if (pos < 0) return;
-    const int64_t kvz = p.row_seq ? p.row_seq[z] : z;
-    const int ctx = pos + 1;
-    if (tid < 32) tab[tid] = kExp2Tab[tid];
-    const int g = h / (p.n_head / p.n_head_kv);
-    const float scale = 1.0f / sqrtf((float)HD);
-    const int64_t cap = p.kv_cap;
-    const int n = chain_len(ctx);
-    float *sc = smem;
-    const float *qg = p.q + z * p.seq_q_stride + (size_t)h * HD;
-    const float *Kh = p.k_cache + kvz * p.seq_kv_stride + (size_t)g * p.kv_head_stride;
-    const float *Vh = p.v_cache + kvz * p.seq_kv_stride + (size_t)g * p.kv_head_stride;
-    // q: uniform (scalar) loads for HD = 64; a 128-float q does not fit the
-    // scalar registers (the compiler spills them), so it is read from LDS
-    __shared__ float qs[HD > 64 ? HD : 1];
-    if constexpr (HD > 64) {
-        if (tid < HD / 4) *(float4 *)(qs + 4 * tid) = *(const float4 *)(qg + 4 * tid);
-        __syncthreads();
-    }
-
-    // scores: thread j takes positions 4j..4j+3 of each round
-    const uint32_t rowb = (uint32_t)cap * 4;
-    float mx = -INFINITY;
-    for (int t4 = 4 * tid; t4 < ctx; t4 += 4 * THREADS) {
-        float acc[4][8];
-        key_round<HD>(acc, (const char *)Kh, rowb, (uint32_t)t4 * 4, qg, qs);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const float u0 = acc[u][0] + acc[u][4], u1 = acc[u][1] + acc[u][5];
-            const float u2 = acc[u][2] + acc[u][6], u3 = acc[u][3] + acc[u][7];
-            const float s = ((u0 + u1) + (u2 + u3)) * scale;
-            if (t4 + u < ctx) {
-                sc[t4 + u] = s;
-                mx = fmaxf(mx, s);
-            }
-        }
-    }
-    const float max_s = block_max(mx, red);
-    for (int t = tid; t < n; t += THREADS) sc[t] = t < ctx ? expf_ref_t(sc[t] - max_s, tab) : 0.0f;
-    __syncthreads();
-    if (tid == 0) inv_slot = 1.0f / (chain_lds(0.0f, sc, n) + 1e-12f);
-    __syncthreads();
-    const float inv = inv_slot;
-    for (int t = tid; t < ctx; t += THREADS) sc[t] = sc[t] * inv;
-    __syncthreads();
-
-    // out_i = ((w_0 v_0[i]) + (w_1 v_1[i])) + ..., products and sums rounded in t order.
-    // AH quads (4 AH positions) of the V row are in flight ahead of the chain, so
-    // a load issued one block ahead has the block's arithmetic to land.  Full
-    // blocks run without selects; the block holding ctx adds +0 past it (the
-    // chain starts at +0, so it is never -0 and +0 leaves it unchanged), and its
-    // w reads stay inside the scores' row: t < chain_len(ctx) (a multiple of 4 AH), where
-    // w_t = +0.
-    if (tid < HD) {
-        const float *v = Vh + (size_t)tid * cap;
-        float acc = 0.0f;
-        constexpr int AH = 16;
-        static_assert(64 % (4 * AH) == 0, "blocks must tile chain_len");
-        float4 vq[AH];
-#pragma unroll
-        for (int a = 0; a < AH; ++a) vq[a] = *(const float4 *)(v + (4 * a < ctx ? 4 * a : 0));
-        auto block = [&](int t0, auto full) {
-#pragma unroll
-            for (int a = 0; a < AH; ++a) {
-                const int t = t0 + 4 * a;
-                const float4 vv = vq[a];
-                const int tn = t + 4 * AH;
-                vq[a] = *(const float4 *)(v + (tn < ctx ? tn : 0));
-                const float4 w = *(const float4 *)(sc + t);
-                const float pr[4] = {w.x * vv.x, w.y * vv.y, w.z * vv.z, w.w * vv.w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc = acc + ((decltype(full)::value || t + j < ctx) ? pr[j] : 0.0f);
-            }
-        };
-        int t0 = 0;
-        for (; t0 + 4 * AH <= ctx; t0 += 4 * AH) block(t0, std::true_type{});
-        if (t0 < ctx) block(t0, std::false_type{});
-        const int64_t i = (int64_t)h * HD + tid;
-        p.out[z * p.seq_q_stride + i] = acc;
-    }
-}
-
 // Output dimensions per workgroup of the streaming kernel for this capacity,
 // or 0 if even one V row does not fit.
 size_t fast_lds_bytes(int64_t cap, int ds) { return (size_t)(chain_row(cap) + (size_t)ds * (chain_row(cap) + 4)) * 4; }
@@ -933,21 +837,14 @@ int launch_attention(const AttnParams &p, hipStream_t s) {
                          (long long)p.kv_cap);
     if (p.seq_pos && (p.n_seq <= 0 || p.n_seq > 65535)) return set_error(GAJE_ERR_INVALID_ARG, "attention: bad batch");
     const unsigned nz = p.seq_pos ? (unsigned)p.n_seq : 1u;
-    const bool batch_kernel = p.seq_pos && p.kv_cap % 4 == 0 && (p.head_dim == 64 || p.head_dim == 128) &&
-                              (size_t)chain_row(p.kv_cap) * 4 + 1024 <= max_lds_per_block();
-    if (batch_kernel && batch_wide_lds_bytes(p.head_dim, p.kv_cap) + 1024 <= max_lds_per_block()) {
+    // several rows: every capacity up to MAX_CTX fits its LDS
+    if (p.seq_pos && p.kv_cap % 4 == 0 && (p.head_dim == 64 || p.head_dim == 128) &&
+        batch_wide_lds_bytes(p.head_dim, p.kv_cap) + 1024 <= max_lds_per_block()) {
         const size_t blds = batch_wide_lds_bytes(p.head_dim, p.kv_cap);
         const int64_t groups = (int64_t)p.n_head_kv * nz, R = p.n_head / p.n_head_kv;
         const dim3 grid((unsigned)((groups + 7) / 8 * 8 * R));  // ids: (8 groups) x R per block of rows
         if (p.head_dim == 64) hipLaunchKernelGGL(attn_batch_wide<64>, grid, dim3(WIDE), blds, s, p);
         else hipLaunchKernelGGL(attn_batch_wide<128>, grid, dim3(WIDE), blds, s, p);
-        GAJE_HIP_CHECK(hipGetLastError());
-        return GAJE_OK;
-    }
-    if (batch_kernel) {
-        const size_t blds = (size_t)chain_row(p.kv_cap) * 4;
-        if (p.head_dim == 64) hipLaunchKernelGGL(attn_decode_batch<64>, dim3(p.n_head, 1, nz), dim3(THREADS), blds, s, p);
-        else hipLaunchKernelGGL(attn_decode_batch<128>, dim3(p.n_head, 1, nz), dim3(THREADS), blds, s, p);
         GAJE_HIP_CHECK(hipGetLastError());
         return GAJE_OK;
     }

@@ -1,9 +1,9 @@
-// Batched decode: one token for each of up to 16 independent sequences per
-// step, as if as many GenomicLLM instances (llm/forward.rs:7-64) stepped
-// together over shared weights.  Every product and reduction follows the
-// batch-1 decode kernels' order, so each sequence's values are bit-identical
-// to its own forward_core: the weight rows are read and dequantised once per
-// step and consumed by every sequence's chains.
+// Rows of several sequences or of a prompt, as if as many GenomicLLM instances
+// (llm/forward.rs:7-64) stepped over shared weights: the passes per row (norms, SwiGLU,
+// the steps' begin and end, argmax) and the batch's f32 lm_head.  Every product and
+// reduction follows the batch-1 decode kernels' order, so each row's values are
+// bit-identical to its own forward_core.  (The Q4_0 products are launch_q4_rows, where
+// the 4, 16 or 32 activation rows of a tile share each dequantised weight.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -505,7 +505,7 @@ int launch_gemv_batch(const BatchGemvParams &p, hipStream_t s) {
             GAJE_HIP_CHECK(hipGetLastError());
             return GAJE_OK;
         }
-        return launch_f32<16>(p, s);
+        return set_error(GAJE_ERR_UNSUPPORTED, "batched f32 matvec: 4 x %lld activations exceed LDS", (long long)p.K);
     }
     return set_error(GAJE_ERR_UNSUPPORTED, "batched matvec: weight format %d", p.fmt);
 }

@@ -6,7 +6,9 @@
 // 8c + l of each block's chunk c, in order) and one fixed reduction.  A matrix
 // instruction with a single k step, v_mfma_f32_{16x16x1_4b,32x32x1_2b}, is one
 // fma per output, rounded once: checked against fmaf over normal, subnormal,
-// infinite, NaN and zero operands, no difference.  So one MFMA block runs one
+// infinite, NaN and zero operands, no difference.  (Here a row's flush of |t| < 1e-6
+// hides what a subnormal could change; the f32 head and the attention of a prompt's
+// rows, which rest on the same property, have tests where it shows.)  So one MFMA block runs one
 // chain: block b of the instruction holds chain l(b) of a 16 x 16 or 32 x 32
 // tile of (weight row, activation row) pairs, each step feeds it one
 // dequantised weight and one activation per row, and the accumulators of the

@@ -212,10 +212,13 @@ def test_batch_nan_guard_halts_one_sequence(hip, O, tmp_models):
     g.close()
 
 
-@pytest.mark.parametrize("heads,vocab,n_seq", [(3, 293, 16), (5, 33, 9), (3, 32900, 16), (1, 33000, 2), (2, 1025, 5)])
+@pytest.mark.parametrize("heads,vocab,n_seq", [(3, 293, 16), (5, 33, 9), (3, 32900, 16), (1, 33000, 2), (2, 1025, 5),
+                                                 (39, 293, 16), (40, 293, 3), (40, 161, 7), (40, 1500, 16), (40, 33, 9)])
 def test_batch_lm_head_edges(hip, O, tmp_models, heads, vocab, n_seq):
     """The batched f32 head: vocabularies about its 16, 32 and 128-row tiles and past one 128-row block
-    per compute unit, widths that end a read-ahead group early, 2 to 16 vectors."""
+    per compute unit, widths that end a read-ahead group early, 2 to 16 vectors; the widest
+    whose 16 vectors fit LDS and the first past it, where 4, 8 and 16 lanes have kernels of
+    their own (512-row blocks for 16)."""
     cfg = dict(HD64, n_embd=64 * heads, n_head=heads, n_head_kv=1, n_blocks=1, ffn=64, vocab_size=vocab)
     p = _write(hip, tmp_models / f"batch_head_{heads}_{vocab}.flat", seed=25, **cfg)
     prompts = _prompts(n_seq, [2], vocab, 26)
@@ -228,5 +231,30 @@ def test_batch_lm_head_edges(hip, O, tmp_models, heads, vocab, n_seq):
         last, toks = _oracle_run(O, p, pr, 2)
         assert same_bits(logits[s], last), f"sequence {s}"
         assert int(out[s][0]) == toks[1], f"sequence {s}"
+    b.close()
+    g.close()
+
+
+def test_batch_lm_head_subnormals(hip, O, tmp_models):
+    """Logits whose products and whole sums are subnormal, beside ordinary rows."""
+    from oracle.flat import FlatFile
+    base = _write(hip, tmp_models / "batch_hd64.flat", seed=21, **HD64)
+    ff, data = FlatFile(base), bytearray(open(base, "rb").read())
+    e = ff.tensors["lm_head"]
+    w = np.frombuffer(data, np.float32, e["dna_len"] // 4, ff.weights_offset + e["dna_off"]).reshape(-1, HD64["n_embd"])
+    w[0::3] *= np.float32(1e-38)
+    w[1::3] *= np.float32(1e-41)
+    p = str(tmp_models / "batch_subnormal.flat")
+    open(p, "wb").write(bytes(data))
+    prompts = _prompts(5, [2], HD64["vocab_size"], 51)
+    g = hip.load_genomic_auto(p)
+    g.set_k_wta_ratio(0.0)
+    b = hip.GenomicBatch(g, 5, 8)
+    logits = b.feed(_padded(prompts, hip.BATCH_INACTIVE), want_logits=True)
+    for s, pr in enumerate(prompts):
+        last, _ = _oracle_run(O, p, pr, 0)
+        tiny = np.abs(last[last != 0]) < np.finfo(np.float32).tiny
+        assert np.mean(tiny) > 0.5  # subnormal sums that are not zero
+        assert same_bits(logits[s], last), f"sequence {s}"
     b.close()
     g.close()

@@ -66,7 +66,7 @@ def _blocks(rng, n, k):
 def test_row_products_match_the_oracle(hip, O, m, n, k):
     rng = np.random.default_rng(m * 1000003 + n * 1009 + k)
     blocks, X = _blocks(rng, n, k), rng.standard_normal((m, k)).astype(np.float32)
-    X[m - 1, :k // 2] *= np.float32(1e-38)     # subnormal products and sums
+    X[m - 1, :k // 2] *= np.float32(1e-38)     # no effect on bits: the row's flush hides subnormal sums
     if m > 2:
         X[1, k - 1], X[2, 0] = np.inf, np.nan  # stay in their own rows
     bias = rng.standard_normal(max(n - 3, 1)).astype(np.float32)
@@ -220,4 +220,49 @@ def test_batch_rows_past_the_tiled_attention(hip, O, tmp_models):
             assert k == 0 or _same(logits[s], want), (lengths, s)
     assert (b.cache_len(0), b.cache_len(1)) == (2510, 277)
     b.close()
+    g.close()
+
+
+def _subnormal_weights_model(hip, O, tmp_models, values):
+    """One block whose attention weights are subnormal wherever the values are not zero:
+    token 7 scores about 95 below token 9 (the query is a bias in the slowest RoPE pair,
+    the keys read elements 32.. of the normed embedding), token 9's values are zero and
+    token 7's about 1e36 (a huge norm weight on elements ..31, which only the values
+    read), or all zero without `values`."""
+    from oracle.flat import FlatFile
+    base = _write(hip, tmp_models, "hd64_1", dict(HD64, n_blocks=1))
+    ff, data = FlatFile(base), bytearray(open(base, "rb").read())
+
+    def view(name, dtype, what="dna"):
+        e = ff.tensors[name]
+        return np.frombuffer(data, dtype, e[what + "_len"] // np.dtype(dtype).itemsize, ff.weights_offset + e[what + "_off"])
+    emb = view("token_embd", np.float32).reshape(-1, 256)
+    norm, bias = view("blk.0.attn_norm", np.float32), view("blk.0.attn_qkv", np.float32, "bias")
+    qkv = view("blk.0.attn_qkv", np.uint8).reshape(512, 8, 20)  # rows: 4 x 64 queries, 2 x 64 keys, 2 x 64 values
+    emb[9, :32] = 0
+    norm[:32], norm[32:] = 1e37 if values else 0, 1
+    qkv[:256], qkv[256:384, 0], qkv[384:, 1:] = 0, 0, 0
+    bias[:] = 0
+    x = emb[[7, 9]] / np.sqrt((emb[[7, 9]].astype(np.float64) ** 2).mean(1, keepdims=True))
+    for h in range(4):
+        k = x @ O.q4_0_dequant(qkv[256 + 64 * (h // 2) + 31].reshape(-1).copy()).astype(np.float64)
+        bias[64 * h + 31] = -95 * 8 / (k[0] - k[1])
+    out = str(tmp_models / f"rows_subnormal_{int(values)}.flat")
+    open(out, "wb").write(bytes(data))
+    return out
+
+
+def test_prompt_attention_keeps_subnormal_weights(hip, O, tmp_models):
+    ids = np.full(130, 9, np.uint32)
+    ids[[3, 40, 77, 100]] = 7
+    want = []
+    for values in (True, False):
+        r = _oracle(O, _subnormal_weights_model(hip, O, tmp_models, values), 0.0)
+        for t in ids:
+            last = r.forward_core(int(t))
+        want.append(last)
+    assert np.mean(want[0] != want[1]) > 0.9  # what the subnormal weights carry reaches the logits
+    g = hip.load_genomic_auto(_subnormal_weights_model(hip, O, tmp_models, True))
+    g.set_k_wta_ratio(0.0)
+    assert _same(g.prefill(ids, want_logits=True), want[0])
     g.close()

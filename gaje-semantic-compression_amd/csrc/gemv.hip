@@ -1861,6 +1861,101 @@ __global__ __launch_bounds__(W * WAVE) void gemv_lut4_lds_kernel(GemvParams p) {
     p.y[row] = total;
 }
 
+// The same rows with one lane per chain: one wave per workgroup takes 16 rows (lane 4 r +
+// c: row r, chain c) and copies x, the rows' codes and their tables at once; then each lane
+// walks its chain with its table lookups and x reads from LDS.  A row takes a quarter of
+// the waves that it takes as batons, at about twice the time: for matrices of more rows than
+// the chip takes at once (launch_gemv).
+constexpr int LUTR_ROWS = 16;
+// Tables in LDS: row q's nb tables at q nb 64 bytes, as the tile lies in
+// memory (one copy per KiB).  For even nb every row's tables then begin on the
+// same LDS bank, so a block's lookups from the 16 rows conflict; padding the
+// rows apart (one copy per row and KiB) measured slower (9.2 against 7.3 us
+// per C0-LUT launch).
+__host__ __device__ constexpr int64_t lut4_trow_bytes(int64_t nb) { return nb * 64; }
+size_t lut4_rows_lds_bytes(int64_t K, int64_t nb, bool shared_table) {
+    const size_t xb = (size_t)K * 4, cb = (size_t)LUTR_ROWS * nb * 16;
+    const size_t tb = shared_table ? 64 : (size_t)LUTR_ROWS * lut4_trow_bytes(nb);
+    return (xb + 1023) / 1024 * 1024 + (cb + 1023) / 1024 * 1024 + (tb + 1023) / 1024 * 1024;
+}
+
+template <bool SHARED>
+__global__ __launch_bounds__(WAVE) void gemv_lut4_rows_kernel(GemvParams p) {
+    extern __shared__ __align__(16) float smem[];
+    const int lane = threadIdx.x, r = lane >> 2, c = lane & 3, base = lane & ~3;
+    const int nb = p.nb;
+    const int64_t K = p.K;
+    const int64_t r0 = (int64_t)blockIdx.x * LUTR_ROWS;
+    float *xs = smem;
+    const int64_t xb = K * 4, cb = (int64_t)LUTR_ROWS * nb * 16;
+    const int64_t trs = lut4_trow_bytes(nb);
+    uint8_t *codes = (uint8_t *)smem + (xb + 1023) / 1024 * 1024;
+    float *tabs = (float *)(codes + (cb + 1023) / 1024 * 1024);
+    // ---- every copy at once: x, the codes, the tables ----
+    lds_copy_bytes(p.x, xb, lds_addr(xs), lane);
+    {
+        // codes of rows r0 .. r0 + 15 (contiguous); lanes past the tensor re-read its start
+        const uint8_t *cw = p.w + r0 * nb * 16;
+        const int64_t cend = (p.N - r0) * nb * 16;
+        for (int64_t o = 0; o < cb; o += 1024) {
+            const int64_t a = o + lane * 16;
+            lds_dma16(cw + (a + 16 <= cend ? a : 0), lds_addr(codes) + (uint32_t)o);
+        }
+    }
+    if constexpr (SHARED) {
+        if (lane < 4) lds_dma16<true>(p.lut + 4 * lane, lds_addr(tabs));
+    } else {
+        // row q's table set (nb 64 bytes) starts at q nb 64 bytes if q < lut_rows_own,
+        // else at 0; rows past the tensor copy row r0's
+        const uint32_t rs = (uint32_t)nb * 64;
+        const uint8_t *lb = (const uint8_t *)p.lut;
+        const int64_t tb = (int64_t)LUTR_ROWS * rs;
+        if (r0 + LUTR_ROWS <= p.lut_rows_own && r0 + LUTR_ROWS <= p.N) {
+            for (int64_t o = 0; o < tb; o += 1024) lds_dma16(lb + r0 * rs + o + lane * 16, lds_addr(tabs) + (uint32_t)o);
+        } else {
+            for (int64_t o = 0; o < tb; o += 1024) {
+                const uint32_t a = (uint32_t)o + lane * 16;
+                int64_t q = r0 + a / rs;
+                q = q < p.N ? q : r0;
+                const int64_t src = (q < p.lut_rows_own ? q * rs : 0) + a % rs;
+                lds_dma16(lb + src, lds_addr(tabs) + (uint32_t)o);
+            }
+        }
+    }
+    if (p.st && s_load_i32(&p.st->halted)) {
+        wait_vmcnt<0>();
+        return;
+    }
+    wait_vmcnt<0>();
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_wave_barrier();
+    // ---- the chain: acc = acc + tbl[code] * x[e], mul then add, blocks in order ----
+    float acc = 0.0f;
+    const uint8_t *crow = codes + (size_t)r * nb * 16;
+    const float *trow = SHARED ? tabs : (const float *)((const uint8_t *)tabs + r * trs);
+    for (int j = 0; j < nb; ++j) {
+        const vu4 cw = *(const vu4 *)(crow + (size_t)j * 16);
+        const float *t = SHARED ? trow : trow + (size_t)j * 16;
+        const float *xj = xs + (size_t)j * 32 + c;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            // element e = 4 u + c; even e is the high nibble of byte e / 2
+            const uint32_t word = (u >> 1) == 0 ? cw.x : (u >> 1) == 1 ? cw.y : (u >> 1) == 2 ? cw.z : cw.w;
+            // byte e / 2 = 2 u + c / 2 of the block: bits 8 ((2u + c/2) & 3) of word u / 2
+            const uint32_t idx = __builtin_amdgcn_ubfe(word, 8 * ((2 * u + (c >> 1)) & 3) + ((c & 1) ? 0 : 4), 4);
+            const float prod = t[idx] * xj[4 * u];
+            acc = acc + prod;
+        }
+    }
+    const float s1 = shfl(acc, base + 1), s2 = shfl(acc, base + 2), s3 = shfl(acc, base + 3);
+    float total = flush_small(((acc + s1) + s2) + s3);  // s0 + s1 + s2 + s3, left to right
+    const int64_t row = r0 + r;
+    if (c == 0 && row < p.N) {
+        if (row < p.bias_len) total = total + p.bias[row];
+        p.y[row] = total;
+    }
+}
+
 template <int MODE, int WAVES, int STAGES, int ROWS, bool TOL = false>
 void *q4l_kernel(int G) {
     switch (G) {
@@ -2844,10 +2939,12 @@ static bool chain_ok(const GemvParams &p, int64_t npairs) {
 // against 5.10, and 1024 x 2336, 19 groups, 5.40 against 5.22; 896 x 4864 8.0 against
 // 6.0 a call).
 static bool baton_ok(const GemvParams &p) {
-    const int64_t G = (p.nb + 3) / 4, cu = device_cu_count();
-    return p.fmt == FMT_Q4_0 && (p.mode == MODE_STORE || p.mode == MODE_RESIDUAL) && !p.gnorm && !p.x_out && !p.norm_w &&
-           (G > BT_LONG || (G > BT_SHORT && 8 * p.N >= 33 * cu)) && p.N <= 8 * cu && p.K <= (1 << 20) &&
-           (size_t)baton_stride(p.K) * 32 + 1024 <= max_lds_per_block();
+    const int64_t G = (p.nb + 3) / 4;
+    if (p.fmt != FMT_Q4_0 || (p.mode != MODE_STORE && p.mode != MODE_RESIDUAL) || p.gnorm || p.x_out || p.norm_w || G <= BT_SHORT ||
+        p.K > (1 << 20))
+        return false;
+    const int64_t cu = device_cu_count();
+    return (G > BT_LONG || 8 * p.N >= 33 * cu) && p.N <= 8 * cu && (size_t)baton_stride(p.K) * 32 + 1024 <= max_lds_per_block();
 }
 
 bool gemv_chain_serves(const GemvParams &p) {
@@ -3046,16 +3143,46 @@ int launch_gemv(const GemvParams &p, hipStream_t s) {
         p.rows_valid == p.N && p.st_in < 0 && (p.lut_block_stride == 0 || p.lut_block_stride == 16) &&
         ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.lut & 15) == 0 && ((uintptr_t)p.w & 15) == 0) {
         const bool shared = p.lut_block_stride == 0;
-        // two waves of four rows (4864 x 896: 6.6 us against 7.0 with four, whose
-        // 304 workgroups load the compute units unevenly); one where the LDS
-        // holds no more (rows past 5888 with a table per block)
-        const int waves = lut4_lds_bytes(2, p.nb, shared) + 1024 <= max_lds_per_block() ? 2 : 1;
-        const size_t llds = lut4_lds_bytes(waves, p.nb, shared);
-        if (llds + 1024 <= max_lds_per_block()) {
+        const size_t lmax = max_lds_per_block();
+        // batons: two waves of four rows (4864 x 896: 6.2 us against 7.0 with four, whose
+        // 304 workgroups load the compute units unevenly); one where the LDS holds no more
+        // (rows past 6400 with a table per block)
+        const int waves = lut4_lds_bytes(2, p.nb, shared) + 1024 <= lmax ? 2 : 1;
+        const size_t llds = lut4_lds_bytes(waves, p.nb, shared), rlds = lut4_rows_lds_bytes(p.K, p.nb, shared);
+        const bool rows_fit = rlds + 1024 <= lmax;
+        // Rows that the chip takes in a round: the workgroups whose LDS (in pieces of 1280
+        // bytes) a compute unit holds, and of batons five (beside more of them a row costs
+        // what it costs in whole lanes).  A round of batons takes about 0.6 of one of whole
+        // lanes, of twice the rows at equal LDS; with the shared table, or short rows, LDS
+        // holds so many whole lanes that batons only win within their first.  Where whole
+        // lanes don't fit, against the walk that waits for each block, three rounds.
+        // Batons / whole lanes / walk, us, a table per block: 4864 x 896 6.2 / 7.5 / 10,
+        // 16384 x 896 12.4 / 9.5 / 14, 24576 x 896 16.1 / 20.1 / 17, 8192 x 3584 52.4 / 44.5 /
+        // 43.8, 5000 x 3328 37.1 / 46.0 / 40.1, 151936 x 128 15.7 / 10.2 / 13.9; 6144 x 3712
+        // 42.2 / - / 44.5, 30000 x 4096 211 / - / 91; the shared table: 10240 x 896 5.7 / 6.2
+        // / 9.7, 32768 x 896 11.3 / 8.7 / 11.8.
+        auto held = [&](size_t bytes) { return (int64_t)(lmax / ((bytes + 1279) / 1280 * 1280)); };
+        const int64_t cu = device_cu_count(), once = cu * waves * LUTL_WR * std::min<int64_t>(5, held(llds));
+        bool batons = llds + 1024 <= lmax;
+        if (!rows_fit) {
+            batons = batons && p.N <= 3 * once;
+        } else if (shared || p.K < 256) {
+            batons = batons && p.N <= once;
+        } else {
+            const int64_t rb = batons ? (p.N + once - 1) / once : INT64_MAX / 8, ronce = cu * LUTR_ROWS * held(rlds);
+            batons = 5 * rb <= 8 * ((p.N + ronce - 1) / ronce);
+        }
+        if (batons) {
             const dim3 grid((unsigned)((p.N + waves * LUTL_WR - 1) / (waves * LUTL_WR)));
             void (*lf)(GemvParams) = waves == 2 ? (shared ? gemv_lut4_lds_kernel<2, true> : gemv_lut4_lds_kernel<2, false>)
                                                 : (shared ? gemv_lut4_lds_kernel<1, true> : gemv_lut4_lds_kernel<1, false>);
             hipLaunchKernelGGL(lf, grid, dim3(waves * WAVE), llds, s, p);
+            GAJE_HIP_CHECK(hipGetLastError());
+            return GAJE_OK;
+        }
+        if (rows_fit) {
+            hipLaunchKernelGGL(shared ? gemv_lut4_rows_kernel<true> : gemv_lut4_rows_kernel<false>,
+                               dim3((unsigned)((p.N + LUTR_ROWS - 1) / LUTR_ROWS)), dim3(WAVE), rlds, s, p);
             GAJE_HIP_CHECK(hipGetLastError());
             return GAJE_OK;
         }

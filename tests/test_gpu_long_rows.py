@@ -66,8 +66,13 @@ def test_long_rows_in_a_decode_step(hip, O, tmp_models, kwta):
 
 
 # odd numbers of blocks, partial workgroups, a table per row and block or the shared
-# one, tables of only the first rows, and rows that leave LDS for one wave a workgroup
-@pytest.mark.parametrize("n,k,own", [(9, 96, 9), (6, 32, 3), (21, 928, 21), (13, 928, -1), (7, 6016, 7), (10, 8960, 5),
+# one, tables of only the first rows, and rows that leave LDS for one wave a workgroup; then
+# both sides of the lines to a lane per chain (more rows than a round takes, short rows,
+# a second round) and to the walk (three rounds)
+@pytest.mark.parametrize("n,k,own", [(10240, 640, 10240), (10243, 640, 10243), (10243, 640, 5000), (24580, 672, 24580),
+                                     (10250, 96, 10250), (10240, 96, 7), (10240, 896, -1), (10253, 928, -1),
+                                     (6144, 3712, 6144), (6145, 3712, 6145), (3073, 8960, 3073),
+                                     (9, 96, 9), (6, 32, 3), (21, 928, 21), (13, 928, -1), (7, 6016, 7), (10, 8960, 5),
                                      (5, 8992, -1)])
 def test_lut4_rows_match_the_oracle(hip, O, n, k, own):
     codes, lut = hip.synth.lut4_tensor(41, f"long.{n}.{k}", n, k)

@@ -2624,7 +2624,8 @@ __global__ __launch_bounds__(THREADS) void gemv_q4_chain_kernel(GemvParams p, in
 // operand reads, 2.4 instructions per step when one lane walks a chain alone and
 // 2.4 / L here.  (Reading values that other waves dequantised into LDS costs about
 // 11 cycles a step against 5.7 here, and its LDS footprint ran 1536 x 8960 in two
-// rounds of workgroups: 22.5 us against 11.4 with L = 8.)
+// rounds of workgroups: 22.5 us, 11.4 as batons with L = 8, and 10.1 with L = 4, as it
+// runs; the chain kernel 21.2.)
 constexpr int BT_SHORT = 12, BT_LONG = 18;  // packed groups past which it serves (baton_ok)
 // Floats of a chain's activations: phases of 32 steps, 4 floats apart in the
 // banks, neighbouring chains 16 apart.

@@ -18,10 +18,10 @@ TINY = dict(n_embd=128, n_head=4, n_head_kv=2, n_blocks=2, ffn=256, vocab_size=1
             rope_base=1e4, arch_family=1, qkv_bias=1, tied_embeddings=0)
 HD64 = dict(n_embd=256, n_head=4, n_head_kv=2, n_blocks=2, ffn=512, vocab_size=1000, eps=1e-6,
             rope_base=1e4, arch_family=1, qkv_bias=1, tied_embeddings=0)
-# gate/up rows >= 16384: the two-rows-per-lane batched matvec
+# gate/up of 16384 rows: past the few-tile form from 8 sequences on
 WIDE = dict(n_embd=128, n_head=4, n_head_kv=2, n_blocks=1, ffn=8192, vocab_size=1000, eps=1e-6,
             rope_base=1e4, arch_family=1, qkv_bias=1, tied_embeddings=0)
-# the same rows with K = 1024: the two-rows-per-lane matvec over two activation chunks
+# the same rows with K = 1024: several stages of the ring
 WIDE_K = dict(n_embd=1024, n_head=8, n_head_kv=2, n_blocks=1, ffn=8192, vocab_size=1000, eps=1e-6,
               rope_base=1e4, arch_family=1, qkv_bias=1, tied_embeddings=0)
 HD128 = dict(n_embd=256, n_head=2, n_head_kv=1, n_blocks=1, ffn=256, vocab_size=512, eps=1e-6,
@@ -141,7 +141,7 @@ def test_batch_long_context_hd128(hip, O, tmp_models, lengths):
 @pytest.mark.parametrize("n_seq", [4, 11, 16])
 def test_batch_benchmark_shape(hip, O, tmp_models, n_seq):
     """The Qwen2.5-1.5B block shapes (hd 128, GQA 6:1, ffn 8960, QKV bias), two blocks; at 16 and
-    11 sequences the 17920-row gate_up runs the two-rows-per-lane matvec over three chunks."""
+    11 sequences the 17920-row gate_up runs 16-row tiles, at 4 the few-tile form."""
     p = _write(hip, tmp_models / "batch_c3_2blk.flat", preset="qwen2.5-1.5b", seed=0, n_blocks=2,
                vocab_size=4096)
     prompts = _prompts(n_seq, [12], 4096, 31)

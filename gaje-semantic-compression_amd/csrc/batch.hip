@@ -488,10 +488,14 @@ int launch_gemv_batch(const BatchGemvParams &p, hipStream_t s) {
     if (p.fmt == FMT_F32) {
         if (!p.f32_tiled || p.K % 8) return set_error(GAJE_ERR_UNSUPPORTED, "batched matvec: f32 rows must be tiled");
         if (p.mode != MODE_STORE) return set_error(GAJE_ERR_UNSUPPORTED, "batched matvec: f32 rows store only");
-        // 16 vectors in LDS (K to 2540 or so): the matrix cores, at any count faster
-        if ((size_t)16 * p.K * 4 + 1024 <= max_lds_per_block()) {
-            const int64_t nblk = (p.N + F32M_ROWS - 1) / F32M_ROWS;
-            hipLaunchKernelGGL(gemv_batch_f32_mfma_kernel, dim3((unsigned)std::min<int64_t>(nblk, device_cu_count())),
+        // 16 vectors in LDS (K to 2540 or so): the matrix cores.  For up to four vectors, whose
+        // VALU form is bound by the weights too and spreads over the compute units evenly,
+        // not where the last round of blocks is mostly empty (2 vectors, 40000 x 1536 55.7 us
+        // against 50.4, 49152 x 576 24.5 against 22.1; 32768 x 1536 34.9 against 46.0, 65536 x
+        // 1536 64.9 against 67.1).
+        const int64_t nblk = (p.N + F32M_ROWS - 1) / F32M_ROWS, cu = device_cu_count(), rounds = (nblk + cu - 1) / cu;
+        if ((size_t)16 * p.K * 4 + 1024 <= max_lds_per_block() && (nv > 4 || rounds == 1 || 10 * nblk >= 9 * rounds * cu)) {
+            hipLaunchKernelGGL(gemv_batch_f32_mfma_kernel, dim3((unsigned)std::min<int64_t>(nblk, cu)),
                                dim3(F32M_NT), (size_t)16 * (p.K + 4) * 4, s, p, nv, nblk);
             GAJE_HIP_CHECK(hipGetLastError());
             return GAJE_OK;
@@ -499,9 +503,9 @@ int launch_gemv_batch(const BatchGemvParams &p, hipStream_t s) {
         if (nv == 4) return launch_f32<4>(p, s);
         if (nv == 8) return launch_f32<8>(p, s);
         if ((size_t)4 * p.K * 4 + 1024 <= max_lds_per_block()) {
-            const int64_t nblk = (p.N + F32B_ROWS - 1) / F32B_ROWS;
-            const int64_t grid = (nblk + 7) / 8 * 32;  // 4 vector groups per block
-            hipLaunchKernelGGL(gemv_batch_f32_rb_kernel, dim3((unsigned)grid), dim3(F32B_NT), (size_t)4 * p.K * 4, s, p, nblk);
+            const int64_t blocks = (p.N + F32B_ROWS - 1) / F32B_ROWS;
+            const int64_t grid = (blocks + 7) / 8 * 32;  // 4 vector groups per block
+            hipLaunchKernelGGL(gemv_batch_f32_rb_kernel, dim3((unsigned)grid), dim3(F32B_NT), (size_t)4 * p.K * 4, s, p, blocks);
             GAJE_HIP_CHECK(hipGetLastError());
             return GAJE_OK;
         }

@@ -213,12 +213,14 @@ def test_batch_nan_guard_halts_one_sequence(hip, O, tmp_models):
 
 
 @pytest.mark.parametrize("heads,vocab,n_seq", [(3, 293, 16), (5, 33, 9), (3, 32900, 16), (1, 33000, 2), (2, 1025, 5),
-                                                 (39, 293, 16), (40, 293, 3), (40, 161, 7), (40, 1500, 16), (40, 33, 9)])
+                                                 (39, 293, 16), (40, 293, 3), (40, 161, 7), (40, 1500, 16), (40, 33, 9),
+                                                 (1, 65500, 3), (1, 65537, 4)])
 def test_batch_lm_head_edges(hip, O, tmp_models, heads, vocab, n_seq):
     """The batched f32 head: vocabularies about its 16, 32 and 128-row tiles and past one 128-row block
     per compute unit, widths that end a read-ahead group early, 2 to 16 vectors; the widest
     whose 16 vectors fit LDS and the first past it, where 4, 8 and 16 lanes have kernels of
-    their own (512-row blocks for 16)."""
+    their own (512-row blocks for 16); up to four lanes with the last round of blocks
+    full or not."""
     cfg = dict(HD64, n_embd=64 * heads, n_head=heads, n_head_kv=1, n_blocks=1, ffn=64, vocab_size=vocab)
     p = _write(hip, tmp_models / f"batch_head_{heads}_{vocab}.flat", seed=25, **cfg)
     prompts = _prompts(n_seq, [2], vocab, 26)

@@ -1948,7 +1948,7 @@ extern "C" int gaje_hip_batch_feed(gaje_hip_batch *b, const uint32_t *ids, int64
     GAJE_HIP_CHECK(hipMemcpyAsync(b->ids, ids, need * 4, hipMemcpyHostToDevice, s));
     // The last step gives the logits; the steps before it run as rows, from two on (one is
     // a step without its head, but waits for the guards: 4 sequences of SmolLM2-135M
-    // widths, two tokens each, 943 us as two steps and 971 that way)
+    // widths, two tokens each, 927 us as two steps and 977 that way)
     const int64_t room = n > 2 && rows_supported(m) ? rows_room(b, m, b->rb, b->nseq * (n - 1)) : 0;
     if (room >= b->nseq) {
         GAJE_TRY(batch_feed_rows(b, ids, n, 0, n - 1, room));
